@@ -8,6 +8,8 @@ rounding (rtol 8e-3, atol 1e-2).  The fused add + RMSNorm must equal add then
 RMSNorm bit for bit.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -123,3 +125,39 @@ def test_add_reference_cases():
     assert add(gpu.allocate((0, 3), np.float32), gpu.allocate((0, 3), np.float32)).shape == (0, 3)
     with pytest.raises(AssertionError):
         add(gpu.allocate((4,), np.float32), gpu.allocate((5,), np.float32))
+
+
+def _at_offset(host, dtype, elems):
+    """The array on the GPU, starting ``elems`` elements into its block (0: 16-byte aligned)."""
+    flat = host.reshape(-1)
+    base = H.upload(np.concatenate([np.zeros(elems, flat.dtype), flat]), dtype)
+    t = gpu.DeviceTensor(ctypes.c_void_p(base.data_ptr() + elems * flat.itemsize), host.shape, base.dtype, flat.nbytes,
+                         defer_free=False)
+    t.base = base
+    return t
+
+
+# 16-byte accesses serve aligned operands (rows of whole 16-byte chunks, one to
+# eight chunks a thread); other rows and pointers go one element at a time.
+# Tolerances: one rounding of the output (2^-8 / 2^-11 of the value) over the
+# fp32 sums' own error (1e-5).
+@pytest.mark.parametrize("dtype,rel", [("float32", 0.0), ("float16", 2.0 ** -11), ("bfloat16", 2.0 ** -8)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_vector_and_scalar_routes(dtype, rel, offset):
+    rng = np.random.default_rng(17)
+    v = 4 if dtype == "float32" else 8
+    for n in (1, v - 1, v, 256 * v - v, 256 * v, 256 * v + v, 512 * v, 1024 * v + v, 2048 * v, 2048 * v + v):
+        print(f"[case] layers {dtype} offset {offset} n {n}", flush=True)
+        a, b = (on.to_storage(rng.standard_normal((3, n), dtype=np.float32), dtype) for _ in range(2))
+        w = on.to_storage(rng.standard_normal(n, dtype=np.float32), dtype)
+        af, bf, wf = (on.from_storage(t, dtype) for t in (a, b, w))
+        ad, bd, wd, hd, yd = (_at_offset(t, dtype, offset) for t in (a, b, w, a, a))
+        s = on.to_storage(af + bf, dtype)
+        np.testing.assert_array_equal(H.download(add(ad, bd, hd)), s)
+        add_rms_norm(ad, bd, hd, wd, yd)
+        np.testing.assert_array_equal(H.download(hd), s)
+        ref = ol.rms_norm_ref(on.from_storage(s, dtype), wf)
+        np.testing.assert_allclose(on.from_storage(H.download(yd), dtype), ref, rtol=1e-5 + rel, atol=1e-6)
+        swiglu(ad, bd, yd)
+        np.testing.assert_allclose(on.from_storage(H.download(yd), dtype), ol.swiglu_ref(af, bf), rtol=1e-5 + rel,
+                                   atol=1e-6)
