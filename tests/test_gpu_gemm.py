@@ -153,8 +153,7 @@ def test_gemm_prompt_shapes_mfma(dtype, M, K, N):
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 @pytest.mark.parametrize("M,K,Ns", [(1900, 136, (16456,)), (2048, 264, (16384,)), (2000, 72, (8192, 8200))])
 def test_gemm_prompt_huge_tiles(dtype, M, K, Ns):
-    """16-bit products with at least two 256 x 256 tiles per CU (520, 512 and
-    520 such tiles here) take the eight-wave 256 x 256 tile kernel: ragged M
+    """Large 16-bit products (520, 512 and 520 tiles of 256 x 256 here): ragged M
     and N, K tails inside a 32-k stage, and the grouped form."""
     print(f"[case] gemm huge {dtype} {M}x{K} -> {Ns}", flush=True)
     rng = np.random.default_rng(M + K + sum(Ns))
@@ -409,3 +408,40 @@ def test_gemm_zero_k_strided_output_keeps_padding():
     c, c2h = c_dev.to_numpy(), c2.to_numpy()
     assert not c[:, :N].any() and (c[:, N:] == 7.0).all()
     assert not c2h[:, :8].any() and (c2h[:, 8:] == 7.0).all()
+
+
+# The 16-bit prompt kernel's tiles (64 x 128 to 256 x 256), each reached by
+# capping the CUs the plan counts rounds for: ragged last rows and columns, odd
+# and even counts of 32-k stages, k tails of 8, 16 and 24, one stage, groups; NaN
+# past k in A's padding, past n in B's. Tolerance as above: the output's rounding.
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,K,Ns,cus", [
+    (300, 136, (584,), 1), (300, 136, (584,), 3), (300, 136, (584,), 4), (300, 136, (584,), 6), (300, 136, (584,), 8),
+    (300, 136, (584,), 16), (300, 136, (584, 200), 5), (193, 1000, (400,), 1), (193, 1000, (400,), 2),
+    (130, 264, (328,), 4),
+    (449, 72, (776,), 3), (449, 72, (776,), 256), (257, 24, (264,), 1), (65, 32, (8,), 256), (16, 8, (136,), 256),
+    (1025, 64, (256,), 2)])
+def test_gemm_wide_tiles(monkeypatch, dtype, M, K, Ns, cus):
+    print(f"[case] gemm wide {dtype} {M}x{K} -> {Ns} cus {cus}", flush=True)
+    H.set_override(monkeypatch, "TRITON_LLM_HIP_MAX_CUS", cus)
+    rng = np.random.default_rng(M + K + cus)
+    pad = lambda x, w: np.concatenate([x, np.full((x.shape[0], w), np.nan, np.float32)], 1)  # noqa: E731
+    a = on.to_storage(pad(rng.standard_normal((M, K), dtype=np.float32), 8), dtype)
+    bs = [on.to_storage(pad(rng.standard_normal((K, n), dtype=np.float32) / np.float32(np.sqrt(K)), 8), dtype)
+          for n in Ns]
+    lib, code, n_g = gpu.runtime(), gpu.dtype_code(H.GPU_DTYPES[dtype]), len(Ns)
+    for extra in (0, 4, 1):  # rows of C that take 16-byte stores, shorter runs, single elements
+        a_dev, b_dev = H.upload(a, dtype), [H.upload(b, dtype) for b in bs]
+        c_dev = [H.upload(on.to_storage(np.full((M, n + extra), 3.0, np.float32), dtype), dtype) for n in Ns]
+        ws = gpu.allocate((max(1, lib.tl_gemm_grouped_workspace_bytes(M, K, n_g, (ctypes.c_int * n_g)(*Ns), code)),),
+                          np.uint8)
+        st = lib.tl_gemm_grouped(a_dev.ptr, M, K, K + 8, n_g, (ctypes.c_void_p * n_g)(*[b.data_ptr() for b in b_dev]),
+                                 (ctypes.c_void_p * n_g)(*[c.data_ptr() for c in c_dev]), (ctypes.c_int * n_g)(*Ns),
+                                 (ctypes.c_int64 * n_g)(*[n + 8 for n in Ns]),
+                                 (ctypes.c_int64 * n_g)(*[n + extra for n in Ns]), ws.ptr, ws.nbytes, code, None)
+        assert st == 0
+        for b, c, n in zip(bs, c_dev, Ns):
+            got = on.from_storage(H.download(c), dtype)
+            exp = gemm_ref(on.from_storage(a, dtype)[:, :K], on.from_storage(b, dtype)[:, :n])
+            np.testing.assert_allclose(got[:, :n], exp, rtol=8e-3, atol=1e-2)
+            assert (got[:, n:] == 3.0).all()

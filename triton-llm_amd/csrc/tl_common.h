@@ -269,6 +269,14 @@ __device__ __forceinline__ void lds_dma16(const i32x4& rsrc, uint32_t voff, uint
                : "memory");
 }
 
+// The same with a wave-uniform byte offset soff added to voff (the range check
+// covers the sum).
+__device__ __forceinline__ void lds_dma16(const i32x4& rsrc, uint32_t voff, uint32_t lds_addr, uint32_t soff) {
+  const uint32_t la = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr);
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(la), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+
 // s_waitcnt vmcnt(N) (gfx9 encoding; expcnt and lgkmcnt left unconstrained).
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {

@@ -6,12 +6,12 @@
 //
 // Two regimes:
 //   * a prompt (m > kSkinnyMaxM rows) is a compute-bound GEMM on the matrix
-//     cores: gemm_mfma_kernel (128 x 128 tiles, LDS-DMA staging, fp32
-//     accumulation); shapes whose rows are not 16-byte aligned take the
-//     simple fp32-FMA gemm_simple_kernel.  A batch of decoded tokens (a few
-//     dozen rows) has too few tiles to fill the device: K is split into
-//     slices with fp32 partials and a reduce pass, and up to 64 rows take
-//     64-row tiles;
+//     cores with fp32 accumulation: gemm_wide_kernel (tl_gemm_wide.hip) for the
+//     16-bit types, gemm_mfma_kernel (128 x 128 tiles, LDS-DMA staging) for
+//     fp32 and for 16-bit products whose k is not a multiple of 8; shapes whose
+//     rows are not 16-byte aligned take the simple fp32-FMA gemm_simple_kernel.
+//     A batch of decoded tokens (a few dozen rows) has too few tiles to fill
+//     the device: K is split into slices with fp32 partials and a reduce pass;
 //   * a decoded token (m <= kSkinnyMaxM rows) reads every weight once for a
 //     handful of multiply-adds per element: an HBM-bound skinny product,
 //     where rocBLAS measured 0.4-0.7 TB/s.  skinny_partial_kernel cuts B
@@ -19,19 +19,18 @@
 //     weight bytes are in flight to stream at HBM speed; each tile's
 //     partial sums go to the workspace and skinny_reduce_kernel adds the
 //     K-slices and rounds to the output type.
-#include "tl_common.h"
+#include "tl_gemm.h"
+#include "tl_gemm_wide.h"
+
+using namespace tlg;
 
 namespace {
 
 constexpr int kSkinnyMaxM = 8;     // rows of A handled by the skinny path
 constexpr int kMaxSmallSplit = 32; // K-slices at most for few-row MFMA products
-// 64-row tiles for at most 64 rows: half the padding MFMA work of 128-row
-// tiles (Llama-3.2-3B layer at 9-64 rows: fp32 286-300 -> 169-189 us, bf16
-// 84.5 -> 73.7 us at 9 rows); 16-bit keeps 64 k per stage in two stages
-// (32 k in four measured 3-5% slower).
+// 64-row tiles for at most 64 fp32 rows: half the padding MFMA work of 128-row
+// tiles (Llama-3.2-3B layer at 9-64 rows: 286-300 -> 169-189 us).
 constexpr int kNarrowMaxM = 64;
-constexpr int kNarrowBkb16 = 128;
-constexpr int kNarrowNst16 = 2;
 // fp32 MFMA kernels, k per LDS stage: 16, except 32 for the 64-row tiles a
 // prompt takes by the occupancy model below (72 KiB in three stages, still
 // two workgroups per CU; SmolLM2-360M's fp32 prompt layer 387 -> 380 us).
@@ -60,30 +59,6 @@ struct SkinnyPlan {
   int tk;       // rows per K-slice
   int ks;       // K-slices
 };
-
-// Products that share A (q/k/v, gate/up): C_g = A . B_g, B_g (k x n_g), for
-// g < count, run as one tile space in one launch.  tile0[g] is group g's
-// first tile in that space (tile0[count] = all tiles); col0[g] its first
-// column in the concatenated width (the split-K partials).
-constexpr int kMaxGroups = 4;
-struct GemmGroups {
-  int count;
-  const void* b[kMaxGroups];
-  void* c[kMaxGroups];
-  int n[kMaxGroups];
-  int64_t ldb[kMaxGroups], ldc[kMaxGroups];
-  int tile0[kMaxGroups + 1];
-  int col0[kMaxGroups + 1];
-};
-
-// The group whose tiles (or columns, with col0) include t.
-__device__ __forceinline__ int find_group(const int (&first)[kMaxGroups + 1], int count, int t) {
-  int g = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxGroups; ++i)
-    if (i < count && t >= first[i]) g = i;
-  return g;
-}
 
 SkinnyPlan skinny_plan(const GemmGroups& G, int k, int esize) {
   SkinnyPlan s;
@@ -311,59 +286,23 @@ int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* 
 constexpr int kGmTile = 128;
 constexpr int kGmThreads = 256;
 
-struct GemmParams {
-  const void* a;
-  int m, k;
-  int64_t lda;
-  GemmGroups G;   // tile0 counts 128 x 128 tiles of C
-  int tiles_m, per_xcd;
-  int vec_store;  // bit g: C_g's rows and base allow 4-column vector stores
-  // Split K (ksplit > 1): item (slice s, tile t) covers stages
-  // [s kt_per, (s + 1) kt_per) and stores its fp32 partial tile at
-  // ws + ws_off[g] + (s m + row) n_g + col; split_reduce_kernel sums them.
-  int ksplit, kt_per;
-  float* ws;
-  int64_t ws_off[kMaxGroups];
-};
-
-// Work item of workgroup L: each XCD (workgroups are dealt to the 8 XCDs in
-// turn) takes a contiguous run of items, row tiles fastest, so the
-// workgroups an XCD runs at once share their B column tiles and A row tiles
-// in its L2; items are slice-major (all tiles of K-slice 0, then slice 1).
-__device__ __forceinline__ bool gemm_tile(const GemmParams& p, int& grp, int& tm, int& tn, int& ks) {
-  const int L = blockIdx.x;
-  const int it = (L % 8) * p.per_xcd + L / 8;
-  const int tiles = p.G.tile0[p.G.count];
-  if (it >= tiles * p.ksplit) return false;
-  ks = it / tiles;
-  const int t = it - ks * tiles;
-  grp = find_group(p.G.tile0, p.G.count, t);
-  const int local = t - p.G.tile0[grp];
-  tm = local % p.tiles_m;
-  tn = local / p.tiles_m;
-  return true;
-}
-
 // BKB: bytes of k per A row per stage (64 or 128); NST: stages in LDS; MBW:
 // 32-row blocks per wave along m (1: 64 x 128 tiles for few rows, 2: 128 x
-// 128 tiles, 4: 256 x 128 tiles, where each B fragment a wave reads feeds
-// four MFMAs instead of two); NWV: waves (4, or 8 for 16-bit 256 x 256 tiles:
-// two along m by four along n, B staged as 512-byte rows, one workgroup per
-// CU, half the operand bytes staged per MFMA of two 256 x 128 workgroups).
-template <typename T, int BKB, int NST, int MBW, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV, NWV == 8 ? 1 : 2) void gemm_mfma_kernel(GemmParams p) {
+// 128 tiles).
+template <typename T, int BKB, int NST, int MBW>
+__global__ __launch_bounds__(kGmThreads, 2) void gemm_mfma_kernel(GemmParams p) {
+  constexpr int NWV = 4;
   constexpr bool F32 = T::size == 4;
   constexpr int TM = 64 * MBW;                // rows of C per tile
   constexpr int BK = BKB / T::size;           // k per stage
   constexpr int ACH = BKB / 16;               // 16-byte chunks per A row (4 or 8)
-  constexpr int TN = 32 * NWV;               // columns of C per tile (128 or 256)
+  constexpr int TN = kGmTile;               // columns of C per tile
   constexpr int BROW = TN * T::size;          // bytes per B row in LDS
   constexpr int NQ = F32 ? BK / 8 : BK / 16;  // fp32 k-groups / 16-bit k-steps per stage
   constexpr int kGmStages = NST;
   constexpr int kGmStageA = TM * BKB;         // bytes of one A stage
   constexpr int kGmStageB = BK * BROW;        // bytes of one B stage
   static_assert(kGmStageA % (1024 * NWV) == 0 && kGmStageB % (1024 * NWV) == 0, "every wave loads whole 1 KiB regions");
-  static_assert(NWV == 4 || !F32, "eight waves: 16-bit only");
   using Bits = typename T::bits;
   __shared__ __attribute__((aligned(1024))) char smem[kGmStages * (kGmStageA + kGmStageB)];
 
@@ -401,16 +340,12 @@ __global__ __launch_bounds__(64 * NWV, NWV == 8 ? 1 : 2) void gemm_mfma_kernel(G
   constexpr int A_RPR = 1024 / BKB;
   const int a_row0 = A_RPR * wave + lane / ACH;
   const uint32_t a_off = (uint32_t)(m_tile + a_row0) * lda2 + (uint32_t)(((lane % ACH) ^ a_swz(a_row0)) * 16);
-  static_assert(NWV == 4 || BKB == 64, "eight waves: 64-byte A rows (the swizzle bits survive a 128-row step)");
   // B, 16-bit: regions of 4 rows of 256 bytes, lane i -> row 4 R + i / 16,
   // slot i % 16 (swizzle 4 (row % 4) = 4 (i / 16)).  fp32: regions of 2 rows
   // of 512 bytes, lane i -> row 2 R + i / 32, slot i % 32 (swizzle
   // 8 ((row >> 2) & 1) = 8 ((R >> 1) & 1), and R = wave + 4 j keeps that bit).
   uint32_t b_off;
-  if constexpr (!F32 && NWV == 8)  // 512-byte rows: regions of 2 rows, lane i -> row 2 R + i / 32
-    b_off = (uint32_t)(2 * wave + lane / 32) * ldb2 + (uint32_t)(n_tile * 2) +
-            (uint32_t)(((lane % 32) ^ (4 * ((2 * wave + lane / 32) & 3))) * 16);
-  else if constexpr (!F32)
+  if constexpr (!F32)
     b_off = (uint32_t)(4 * wave + lane / 16) * ldb2 + (uint32_t)(n_tile * 2) +
             (uint32_t)(((lane % 16) ^ (4 * (lane / 16))) * 16);
   else
@@ -679,7 +614,6 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(GemmParams p) {
 
 // How a prompt-sized product runs on the MFMA kernel: tile height and K split.
 struct PromptPlan {
-  bool huge;      // 16-bit 256 x 256 tiles (eight waves)
   bool narrow;    // 64 x 128 tiles (few rows: half the padding of 128-row tiles)
   bool f32_deep;  // fp32 64-row tiles with 32-k stages (prompts)
   int tiles_m, tiles;
@@ -687,15 +621,6 @@ struct PromptPlan {
   size_t ws_bytes;  // fp32 partials when split
 };
 
-// 16-bit: 256 x 256 tiles (eight waves, one workgroup per CU; each B
-// fragment feeds four MFMAs) where they still give every CU two: at a
-// 2048-row Llama-3.2-3B prompt gate/up 206-209 -> 191 us, the layer
-// 456-462 -> 442 us.  Fewer, larger tiles leave CUs idle on the narrower
-// products (q/k/v, o and down keep 128 x 128).  (A 256 x 128 tile, taken
-// at four or more per CU, measured gate/up 226 -> 219 us; every shape with
-// four such tiles per CU has at least two 256 x 256 ones, so it was never
-// reached once those existed, and it was removed.)
-//
 // K split (fp32): a CU's time is set by the items it runs, and a whole tile
 // is the unit, so 384 tiles on 256 CUs cost two tiles' time where 1.5 would
 // do.  Splitting K in S slices makes the unit 1 / S of a tile at the price of
@@ -710,18 +635,13 @@ PromptPlan prompt_plan(int m, int k, const GemmGroups& G, int esize) {
   const int cus = tl_device_cus();
   int64_t ncols = 0;
   for (int g = 0; g < G.count; ++g) ncols += G.n[g];
-  int huge_tiles = 0;
-  for (int g = 0; g < G.count; ++g)
-    huge_tiles += ((m + 2 * kGmTile - 1) / (2 * kGmTile)) * ((G.n[g] + 2 * kGmTile - 1) / (2 * kGmTile));
-  P.huge = esize == 2 && huge_tiles >= 2 * cus;
-  P.narrow = !P.huge && m <= kNarrowMaxM;
-  const int tm = P.huge ? 2 * kGmTile : (P.narrow ? kGmTile / 2 : kGmTile);
+  P.narrow = esize == 4 && m <= kNarrowMaxM;
+  const int tm = P.narrow ? kGmTile / 2 : kGmTile;
   P.tiles_m = (m + tm - 1) / tm;
   P.tiles = 0;
-  const int tn = P.huge ? 2 * kGmTile : kGmTile;
-  for (int g = 0; g < G.count; ++g) P.tiles += P.tiles_m * ((G.n[g] + tn - 1) / tn);
+  for (int g = 0; g < G.count; ++g) P.tiles += P.tiles_m * ((G.n[g] + kGmTile - 1) / kGmTile);
   // k per LDS stage of the kernel used
-  const int bk = esize == 2 ? (P.huge ? 32 : (P.narrow ? kNarrowBkb16 / 2 : 64)) : kF32Bk;
+  const int bk = esize == 2 ? 64 : kF32Bk;
   int n_kt = (k + bk - 1) / bk;
   // modelled seconds: the product at a sustained rate, scaled by the busiest
   // CU's share of items; the reduce as HBM traffic plus a launch
@@ -806,6 +726,38 @@ PromptPlan prompt_plan(int m, int k, const GemmGroups& G, int esize) {
   return P;
 }
 
+// Whether a 16-bit product whose rows are 16-byte aligned runs on
+// gemm_wide_kernel: k in whole 16-byte chunks (its last stage drops the chunks
+// past k, and only whole ones), and 32-bit offsets for a row tile of A and for
+// the stages its prefetch counts past the end of each B.
+bool wide_ok(const GemmGroups& G, int m, int k, int64_t lda) {
+  bool ok = k % 8 == 0 && lda * 2 * 256 < ((int64_t)1 << 31);
+  for (int g = 0; g < G.count; ++g) ok = ok && ((int64_t)k + 512) * G.ldb[g] * 2 < ((int64_t)1 << 32);
+  return ok;
+}
+
+// Fills the K split of p, whose tile0 is set: slices, partials' places, items per XCD.
+void set_split(GemmParams& p, int m, int ksplit, int kt_per, void* workspace) {
+  p.ksplit = ksplit;
+  p.kt_per = kt_per;
+  p.ws = (float*)workspace;
+  int64_t off = 0;
+  for (int g = 0; g < p.G.count; ++g) {
+    p.ws_off[g] = off;
+    off += (int64_t)ksplit * m * p.G.n[g];
+  }
+  p.per_xcd = (p.G.tile0[p.G.count] * ksplit + 7) / 8;
+}
+
+template <typename T>
+int launch_split_reduce(const GemmParams& p, int m, hipStream_t st) {
+  int64_t runs = 0;
+  for (int g = 0; g < p.G.count; ++g) runs = (int64_t)m * (p.G.n[g] / 4) > runs ? (int64_t)m * (p.G.n[g] / 4) : runs;
+  const unsigned rb = (unsigned)((runs + 255) / 256 < 4096 ? (runs + 255) / 256 : 4096);
+  hipLaunchKernelGGL((split_reduce_kernel<T>), dim3(rb, p.G.count), dim3(256), 0, st, p);
+  return tl_launch_status();
+}
+
 template <typename T>
 int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, void* workspace,
                 size_t workspace_bytes, hipStream_t st) {
@@ -828,40 +780,41 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
               ((int64_t)k + 64 + 1) * G.ldb[g] * esize < ((int64_t)1 << 32);
     widest = G.n[g] > widest ? G.n[g] : widest;
   }
+  if constexpr (T::size == 2) {
+    if (aligned && wide_ok(G, m, k, lda)) {
+      // as many K-slices as the workspace query's plan has, where it was given
+      const PromptPlan P = prompt_plan(m, k, G, 2);
+      const bool room = workspace && workspace_bytes >= P.ws_bytes && ((uintptr_t)workspace % 16) == 0;
+      const WidePlan W = gemm_wide_plan(m, k, G, room ? P.ksplit : 1);
+      p.tiles_m = (m + W.tm - 1) / W.tm;
+      for (int g = 0; g < G.count; ++g) {
+        p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + W.tn - 1) / W.tn);
+        // whole runs: 8 columns from the kernel, 4 from the reduce
+        const int run = W.ksplit > 1 ? 4 : 8;
+        if (G.ldc[g] % run == 0 && ((uintptr_t)G.c[g] % (run * esize)) == 0) p.vec_store |= 1 << g;
+      }
+      set_split(p, m, W.ksplit, W.kt_per, workspace);
+      const int e = launch_gemm_wide<T>(p, W, st);
+      return e || p.ksplit == 1 ? e : launch_split_reduce<T>(p, m, st);
+    }
+  }
   if (aligned) {
     const PromptPlan P = prompt_plan(m, k, G, (int)esize);
     p.tiles_m = P.tiles_m;
     p.G.tile0[0] = 0;
     p.vec_store = 0;
     for (int g = 0; g < G.count; ++g) {
-      const int tn = P.huge ? 2 * kGmTile : kGmTile;
-      p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + tn - 1) / tn);
+      p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + kGmTile - 1) / kGmTile);
       if (G.ldc[g] % 4 == 0 && ((uintptr_t)G.c[g] % (4 * esize)) == 0) p.vec_store |= 1 << g;
     }
     // the split needs its partials' workspace; without it the product runs whole
     const bool split = P.ksplit > 1 && workspace && workspace_bytes >= P.ws_bytes && ((uintptr_t)workspace % 16) == 0;
-    p.ksplit = split ? P.ksplit : 1;
-    p.kt_per = split ? P.kt_per : (k + 15) / 16 + 1;  // whole: one slice covers every stage
-    p.ws = (float*)workspace;
-    int64_t off = 0;
-    for (int g = 0; g < G.count; ++g) {
-      p.ws_off[g] = off;
-      off += (int64_t)p.ksplit * m * G.n[g];
-    }
-    p.per_xcd = (p.G.tile0[G.count] * p.ksplit + 7) / 8;
-    // Measured at the models' prompt shapes (2048 rows): 16-bit runs best
-    // with 64 k per stage in two stages (729 against 645 TFLOP/s with 32 k
-    // in three, 691 with 32 k in four, 507 with 64 k in three); fp32 is
-    // within 1% across those and keeps 16 k in three stages, except the
-    // 64-row tiles a prompt takes by the occupancy model (kF32BkDeep).
+    set_split(p, m, split ? P.ksplit : 1, split ? P.kt_per : (k + 15) / 16 + 1, workspace);  // whole: one slice covers every stage
+    // fp32 is within 1% across stage shapes and keeps 16 k in three stages,
+    // except the 64-row tiles a prompt takes by the occupancy model (kF32BkDeep).
     const dim3 grid((unsigned)(8 * p.per_xcd));
     if constexpr (T::size == 2) {
-      if (P.huge)
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 3, 4, 8>), grid, dim3(512), 0, st, p);
-      else if (P.narrow)
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, kNarrowBkb16, kNarrowNst16, 1>), grid, dim3(kGmThreads), 0, st, p);
-      else
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 2, 2>), grid, dim3(kGmThreads), 0, st, p);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 2, 2>), grid, dim3(kGmThreads), 0, st, p);
     } else {
       if (P.narrow && P.f32_deep)
         hipLaunchKernelGGL((gemm_mfma_kernel<T, 4 * kF32BkDeep, 3, 1>), grid, dim3(kGmThreads), 0, st, p);
@@ -870,13 +823,8 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
       else
         hipLaunchKernelGGL((gemm_mfma_kernel<T, 4 * kF32Bk, 3, 2>), grid, dim3(kGmThreads), 0, st, p);
     }
-    int e = tl_launch_status();
-    if (e || p.ksplit == 1) return e;
-    int64_t runs = 0;
-    for (int g = 0; g < G.count; ++g) runs = (int64_t)m * (G.n[g] / 4) > runs ? (int64_t)m * (G.n[g] / 4) : runs;
-    const unsigned rb = (unsigned)((runs + 255) / 256 < 4096 ? (runs + 255) / 256 : 4096);
-    hipLaunchKernelGGL((split_reduce_kernel<T>), dim3(rb, G.count), dim3(256), 0, st, p);
-    return tl_launch_status();
+    const int e = tl_launch_status();
+    return e || p.ksplit == 1 ? e : launch_split_reduce<T>(p, m, st);
   }
   dim3 grid((unsigned)((widest + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)G.count);
   hipLaunchKernelGGL((gemm_simple_kernel<T>), grid, dim3(256), 0, st, p);
