@@ -445,3 +445,96 @@ def test_gemm_wide_tiles(monkeypatch, dtype, M, K, Ns, cus):
             exp = gemm_ref(on.from_storage(a, dtype)[:, :K], on.from_storage(b, dtype)[:, :n])
             np.testing.assert_allclose(got[:, :n], exp, rtol=8e-3, atol=1e-2)
             assert (got[:, n:] == 3.0).all()
+
+
+# fp32 products split into bf16 parts: tile edges, k tails, both tile heights, K
+# slices, rows of C that take scalar stores. Tolerance: six fp32 roundings a
+# 32-k stage, each 2^-24 of the sum's magnitude bound |a| . |b|.
+@pytest.mark.parametrize("M,K,Ns,cus", [(9, 4, (4,), 256), (65, 36, (132, 8), 256), (128, 32, (128,), 1),
+                                        (129, 100, (260,), 2), (200, 1000, (196,), 4), (300, 2560, (264,), 256),
+                                        (1100, 64, (516,), 8)])
+def test_gemm_fp32_parts_tiles(monkeypatch, M, K, Ns, cus):
+    print(f"[case] gemm fp32 parts {M}x{K} -> {Ns} cus {cus}", flush=True)
+    H.set_override(monkeypatch, "TRITON_LLM_HIP_MAX_CUS", cus)
+    rng = np.random.default_rng(M + K)
+    a = rng.standard_normal((M, K), dtype=np.float32)
+    bs = [rng.standard_normal((K, n), dtype=np.float32) for n in Ns]
+    outs = gemm_grouped(gpu.to_device(a), [gpu.to_device(b) for b in bs])
+    lib = gpu.runtime()
+    c1 = gpu.to_device(np.full((M, Ns[0] + 1), 3.0, np.float32))
+    a_d, b_d = gpu.to_device(a), gpu.to_device(bs[0])
+    assert lib.tl_gemm(a_d.ptr, b_d.ptr, c1.ptr, M, Ns[0], K, K, Ns[0], Ns[0] + 1, None, 0, 0, None) == 0
+    got1 = H.download(c1)
+    assert (got1[:, Ns[0]:] == 3.0).all()
+    for b, got in list(zip(bs, map(H.download, outs))) + [(bs[0], got1[:, :Ns[0]])]:
+        exact = a.astype(np.float64) @ b.astype(np.float64)
+        bound = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+        assert (np.abs(got - exact) <= 6 * (K / 32 + 1) * 2.0 ** -24 * bound + 1e-30).all()
+
+
+def test_gemm_fp32_parts_whole_range():
+    """Values whose parts do not cover them -- NaN, infinities, magnitudes near
+    the ends of fp32 -- give what fp32 multiply-adds give, in their rows and
+    columns and nowhere else; zeros and mixed magnitudes stay exact enough."""
+    M, K, N = 150, 96, 200
+    rng = np.random.default_rng(3)
+    for what in ("nan", "inf", "inf0", "huge", "tiny-row", "tiny-column", "zero-row", "mixed"):
+        a = rng.standard_normal((M, K), dtype=np.float32)
+        b = rng.standard_normal((K, N), dtype=np.float32)
+        if what == "nan":
+            a[3, 5], b[7, 131] = np.nan, np.nan
+        elif what == "inf":
+            a[140, 95], b[0, 0] = np.inf, -np.inf
+            b[95, :4] = 1.5  # exact in one part: infinity times the other parts' zeros must not appear
+        elif what == "inf0":
+            a[2, 2] = np.inf
+            b[2, 9] = 0.0
+        elif what == "huge":
+            a[17, :] = np.float32(3e38) * np.sign(a[17])
+            b *= np.float32(1e-3)
+        elif what == "tiny-row":
+            a[10] *= np.float32(1e-35)
+        elif what == "tiny-column":
+            b[:, 199] *= np.float32(1e-35)
+        elif what == "zero-row":
+            a[5], b[:, 6] = 0.0, 0.0
+        else:
+            a[:, ::3] *= np.float32(1e-12)
+            b[1::2] *= np.float32(1e10)
+        print(f"[case] gemm fp32 whole range {what}", flush=True)
+        got = H.download(gemm(gpu.to_device(a), gpu.to_device(b)))
+        with np.errstate(all="ignore"):
+            ref = (a[:, :, None] * b[None]).astype(np.float32).sum(1, dtype=np.float64)
+            bound = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+        # an fp32 chain may overflow where the sum stays finite; elsewhere the patterns are the same
+        sure = np.abs(ref) < 3e38
+        np.testing.assert_array_equal(np.isnan(got)[~np.isfinite(ref)], np.isnan(ref)[~np.isfinite(ref)])
+        inf = np.isinf(ref) & ~np.isnan(got)
+        np.testing.assert_array_equal(got[inf], ref[inf].astype(np.float32))
+        ok = np.isfinite(ref) & sure & (bound < 1e38)
+        assert (np.abs(got[ok] - ref[ok]) <= (K + 4) * 2.0 ** -24 * bound[ok] + 1e-45).all(), what
+
+
+@pytest.mark.parametrize("dtype,K,lda", [("bfloat16", 130, 136), ("float16", 1001, 1008), ("float32", 131, 136),
+                                         ("float32", 998, 1000)])
+@pytest.mark.parametrize("M", [40, 150])
+def test_gemm_partial_k_chunk(dtype, K, lda, M):
+    """Aligned rows whose k ends inside a 16-byte chunk, NaN behind it (the
+    kernel for such k, whole and with K slices)."""
+    N = 136
+    print(f"[case] gemm partial k chunk {dtype} {M}x{K}", flush=True)
+    rng = np.random.default_rng(K + M)
+    a = np.full((M, lda), np.nan, np.float32)
+    a[:, :K] = rng.standard_normal((M, K), dtype=np.float32)
+    b = rng.standard_normal((K, N), dtype=np.float32) / np.float32(np.sqrt(K))
+    a_s, b_s = on.to_storage(a, dtype), on.to_storage(b, dtype)
+    lib, code = gpu.runtime(), gpu.dtype_code(H.GPU_DTYPES[dtype])
+    a_d, b_d, c_d = H.upload(a_s, dtype), H.upload(b_s, dtype), gpu.allocate((M, N), H.GPU_DTYPES[dtype])
+    exp = gemm_ref(on.from_storage(a_s, dtype)[:, :K], on.from_storage(b_s, dtype))
+    need = lib.tl_gemm_workspace_bytes(M, N, K, code)
+    ws = gpu.allocate((max(1, need),), np.uint8)
+    for ptr, size in ((None, 0), (ws.ptr, ws.nbytes)):
+        assert lib.tl_gemm(a_d.ptr, b_d.ptr, c_d.ptr, M, N, K, lda, N, N, ptr, size, code, None) == 0
+        got = on.from_storage(H.download(c_d), dtype)
+        np.testing.assert_allclose(got, exp, rtol=1e-4 if dtype == "float32" else 8e-3,
+                                   atol=1e-4 if dtype == "float32" else 1e-2)

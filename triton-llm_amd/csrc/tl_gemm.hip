@@ -7,9 +7,10 @@
 // Two regimes:
 //   * a prompt (m > kSkinnyMaxM rows) is a compute-bound GEMM on the matrix
 //     cores with fp32 accumulation: gemm_wide_kernel (tl_gemm_wide.hip) for the
-//     16-bit types, gemm_mfma_kernel (128 x 128 tiles, LDS-DMA staging) for
-//     fp32 and for 16-bit products whose k is not a multiple of 8; shapes whose
-//     rows are not 16-byte aligned take the simple fp32-FMA gemm_simple_kernel.
+//     16-bit types, gemm_f32_kernel (tl_gemm_f32.hip) for fp32; gemm_mfma_kernel
+//     (128 x 128 tiles, LDS-DMA staging) where k is not a whole number of
+//     16-byte chunks, the simple fp32-FMA gemm_simple_kernel where rows are not
+//     16-byte aligned.
 //     A batch of decoded tokens (a few dozen rows) has too few tiles to fill
 //     the device: K is split into slices with fp32 partials and a reduce pass;
 //   * a decoded token (m <= kSkinnyMaxM rows) reads every weight once for a
@@ -20,6 +21,7 @@
 //     partial sums go to the workspace and skinny_reduce_kernel adds the
 //     K-slices and rounds to the output type.
 #include "tl_gemm.h"
+#include "tl_gemm_f32.h"
 #include "tl_gemm_wide.h"
 
 using namespace tlg;
@@ -28,17 +30,10 @@ namespace {
 
 constexpr int kSkinnyMaxM = 8;     // rows of A handled by the skinny path
 constexpr int kMaxSmallSplit = 32; // K-slices at most for few-row MFMA products
-// 64-row tiles for at most 64 fp32 rows: half the padding MFMA work of 128-row
-// tiles (Llama-3.2-3B layer at 9-64 rows: 286-300 -> 169-189 us).
+// Rows up to which split_cap counts fp32 tiles of 64 rows.
 constexpr int kNarrowMaxM = 64;
-// fp32 MFMA kernels, k per LDS stage: 16, except 32 for the 64-row tiles a
-// prompt takes by the occupancy model below (72 KiB in three stages, still
-// two workgroups per CU; SmolLM2-360M's fp32 prompt layer 387 -> 380 us).
-// Few rows keep 16 (a Llama-3.2-3B layer at 64 rows: 183 against 194 us
-// with 32), and so do 128-row tiles (32 would need 96 KiB: one workgroup
-// per CU).
+// gemm_mfma_kernel, fp32: k per LDS stage.
 constexpr int kF32Bk = 16;
-constexpr int kF32BkDeep = 32;
 constexpr int kSkThreads = 256;    // 4 waves
 constexpr int kSkUnroll = 16;      // row loads in flight per lane
 constexpr int kSkMaxTk = 1024;     // rows per K-slice at most (A's slice is staged in LDS)
@@ -251,12 +246,12 @@ int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* 
 }
 
 // ---------------------------------------------------------------------------
-// Prompt-sized products on the matrix cores (m > kSkinnyMaxM).
+// Products on the matrix cores whose rows are 16-byte aligned but whose k is not
+// a whole number of 16-byte chunks (m > kSkinnyMaxM).
 //
 // Workgroup tile 128 x 128 of C, 4 waves in 2 x 2, each wave 64 x 64 (2 x 2
 // blocks of 32 x 32).  K is walked in LDS stages (16-bit: 64 k in two
-// stages; fp32: 16 k in three, 32 k for the 64-row prompt plans), every
-// tile moved global -> LDS by LDS-DMA
+// stages; fp32: 16 k in three), every tile moved global -> LDS by LDS-DMA
 // (buffer_load ... lds: no register round trip), every wave loading a
 // quarter.  Each wave computes the transposed block C^T = B^T . A^T with
 // the MFMA, so a lane ends up owning one row of C and 4 consecutive columns
@@ -286,12 +281,10 @@ int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* 
 constexpr int kGmTile = 128;
 constexpr int kGmThreads = 256;
 
-// BKB: bytes of k per A row per stage (64 or 128); NST: stages in LDS; MBW:
-// 32-row blocks per wave along m (1: 64 x 128 tiles for few rows, 2: 128 x
-// 128 tiles).
-template <typename T, int BKB, int NST, int MBW>
+// BKB: bytes of k per A row per stage (64 or 128); NST: stages in LDS.
+template <typename T, int BKB, int NST>
 __global__ __launch_bounds__(kGmThreads, 2) void gemm_mfma_kernel(GemmParams p) {
-  constexpr int NWV = 4;
+  constexpr int NWV = 4, MBW = 2;  // waves; 32-row blocks of a wave
   constexpr bool F32 = T::size == 4;
   constexpr int TM = 64 * MBW;                // rows of C per tile
   constexpr int BK = BKB / T::size;           // k per stage
@@ -612,150 +605,87 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(GemmParams p) {
     }
 }
 
-// How a prompt-sized product runs on the MFMA kernel: tile height and K split.
-struct PromptPlan {
-  bool narrow;    // 64 x 128 tiles (few rows: half the padding of 128-row tiles)
-  bool f32_deep;  // fp32 64-row tiles with 32-k stages (prompts)
-  int tiles_m, tiles;
-  int ksplit, kt_per;
-  size_t ws_bytes;  // fp32 partials when split
+// The most K-slices a product of more than kSkinnyMaxM rows may run in, and the
+// bytes of their fp32 partials: what tl_gemm_workspace_bytes answers.  The
+// kernels' own plans (gemm_wide_plan, gemm_f32_plan) choose within it.
+struct SplitCap {
+  int ksplit;
+  size_t ws_bytes;
 };
 
-// K split (fp32): a CU's time is set by the items it runs, and a whole tile
-// is the unit, so 384 tiles on 256 CUs cost two tiles' time where 1.5 would
-// do.  Splitting K in S slices makes the unit 1 / S of a tile at the price of
-// a reduce pass over S fp32 partials; S (1..4, at least 4 stages per slice)
-// is the one with the least modelled time, and a split must win by 3%.
-// Measured at a 2048-row Llama-3.2-3B prompt, fp32: q/k/v 583 -> 520, o
-// 403 -> 317, down 1061 -> 805 us (S = 2).  16-bit products are not split:
-// at their speed the partials' traffic cost more than the balance gained
-// (bf16 down 118 -> 127 us with S = 2).
-PromptPlan prompt_plan(int m, int k, const GemmGroups& G, int esize) {
-  PromptPlan P{};
+// Few rows (a batch of decoded tokens): the product streams B, and a few dozen
+// tiles of C, each walking all of K, leave most CUs idle, so K may be cut until
+// about one item per CU runs for 16-bit products and two for fp32 ones, while
+// the fp32 partials stay under half of B's bytes (which rules out large m) and
+// every slice keeps two stages.  fp32 prompts beyond that: a CU's time is set by
+// the whole items it runs (384 tiles on 256 CUs cost two tiles' time where 1.5
+// would do), so up to four slices where the busiest CU's share, plus the reduce
+// pass, comes out 3% lower, counted in 128-row tiles or 64-row ones.  16-bit
+// prompts beyond it are not split: at their speed the partials' traffic costs
+// more than the balance gains.
+SplitCap split_cap(int m, int k, const GemmGroups& G, int esize) {
   const int cus = tl_device_cus();
+  const bool narrow = esize == 4 && m <= kNarrowMaxM;
   int64_t ncols = 0;
   for (int g = 0; g < G.count; ++g) ncols += G.n[g];
-  P.narrow = esize == 4 && m <= kNarrowMaxM;
-  const int tm = P.narrow ? kGmTile / 2 : kGmTile;
-  P.tiles_m = (m + tm - 1) / tm;
-  P.tiles = 0;
-  for (int g = 0; g < G.count; ++g) P.tiles += P.tiles_m * ((G.n[g] + kGmTile - 1) / kGmTile);
-  // k per LDS stage of the kernel used
+  auto cap = [&](int S) { return SplitCap{S, S > 1 ? (size_t)S * m * ncols * sizeof(float) : 0}; };
+  auto tiles_of = [&](int tm) {
+    int64_t tiles = 0;
+    for (int g = 0; g < G.count; ++g) tiles += (int64_t)((m + tm - 1) / tm) * ((G.n[g] + kGmTile - 1) / kGmTile);
+    return tiles;
+  };
+  const int64_t tiles = tiles_of(narrow ? kGmTile / 2 : kGmTile);
   const int bk = esize == 2 ? 64 : kF32Bk;
-  int n_kt = (k + bk - 1) / bk;
-  // modelled seconds: the product at a sustained rate, scaled by the busiest
-  // CU's share of items; the reduce as HBM traffic plus a launch
-  const double rate = esize == 2 ? 9.0e14 : 1.3e14;
-  const double t1 = 2.0 * m * (double)k * (double)ncols / rate;
-  auto busiest = [&](int S) { return (double)((P.tiles * (int64_t)S + cus - 1) / cus) / S; };
-  auto reduce_t = [&](int S) { return ((double)S * 4 + esize) * m * (double)ncols / 5.0e12 + 3e-6; };
-  double best = t1;
-  P.ksplit = 1;
-  // Few rows (a batch of decoded tokens): the product streams B, and a few
-  // dozen tiles of C, each walking all of K, leave most CUs idle (a
-  // workgroup streams only tens of GB/s).  Split K until about one item per
-  // CU runs for 16-bit products and two for fp32 ones (measured, Llama-3.2-3B
-  // layer at 9-64 rows: bf16 74-91 us with two per CU against 67-81 us with
-  // one; fp32 168-184 us against 198-208), while the fp32 partials stay
-  // under half of B's bytes (which rules out large m) and every slice keeps
-  // two stages.
-  if (P.tiles < 2 * cus) {
+  const int n_kt = (k + bk - 1) / bk;
+  if (tiles < 2 * cus) {
     const int64_t by_traffic = (int64_t)k * esize / (2 * 4 * (int64_t)m);
-    const int per_cu = esize == 2 ? 1 : 2;
-    int64_t S = (per_cu * cus + P.tiles - 1) / P.tiles;
+    int64_t S = ((esize == 2 ? 1 : 2) * cus + tiles - 1) / tiles;
     S = S < by_traffic ? S : by_traffic;
     S = S < n_kt / 2 ? S : n_kt / 2;
     S = S < kMaxSmallSplit ? S : kMaxSmallSplit;
-    if (S >= 2) {
-      P.ksplit = (int)S;
-      P.kt_per = (n_kt + P.ksplit - 1) / P.ksplit;
-      P.ws_bytes = (size_t)P.ksplit * m * ncols * sizeof(float);
-      return P;
-    }
+    if (S >= 2) return cap((int)S);
   }
-  for (int S = 2; S <= 4 && esize == 4; ++S) {
-    if (n_kt < 4 * S) break;
+  if (esize == 2) return cap(1);
+  const double rate = 1.3e14;  // FLOP/s
+  auto reduce_t = [&](int S) { return ((double)S * 4 + esize) * m * (double)ncols / 5.0e12 + 3e-6; };
+  const double t1 = 2.0 * m * (double)k * (double)ncols / rate;
+  auto busiest = [&](int S) { return (double)((tiles * S + cus - 1) / cus) / S; };
+  int split = 1;
+  double best = t1;
+  for (int S = 2; S <= 4 && n_kt >= 4 * S; ++S) {
     const double t = t1 * busiest(S) / busiest(1) + reduce_t(S);
     if (t < 0.97 * best) {
       best = t;
-      P.ksplit = S;
+      split = S;
     }
   }
-  if (esize == 4 && !P.narrow) {
-    // fp32 with 64-row tiles instead, when a model of the busiest CU's items
-    // says they win by 3%.  A CU runs two items at once at the sustained
-    // rate; a lone item runs at about 0.7 of it (one 128 x 128 fp32
-    // workgroup alone on a CU reaches 58% of the CU's MFMA peak, two
-    // together 82%), and a 64-row tile does its FLOPs at about 0.865 of a
-    // 128-row tile's rate (Llama-3.2-3B o at 2048 rows, K split in 2 either
-    // way: 321 against 316 us).  More items of 64 rows fill the CUs that a
-    // few 128-row tiles leave with one item or none (SmolLM2-360M at 2048
-    // rows: grouped q/k/v 78 -> 73 us, gate/up 191 -> 166 us).
-    const double r2 = rate / cus, r1 = r2 * (0.58 / 0.82);
-    auto model = [&](int ctm, int S) {
-      int64_t ctiles = 0;
-      for (int g = 0; g < G.count; ++g) ctiles += (int64_t)((m + ctm - 1) / ctm) * ((G.n[g] + kGmTile - 1) / kGmTile);
-      const int64_t per_cu = (ctiles * S + cus - 1) / cus;
-      const double w = 2.0 * ctm * kGmTile * (double)k / S / (ctm < kGmTile ? 0.865 : 1.0);
-      return (double)(per_cu - per_cu % 2) * w / r2 + (double)(per_cu % 2) * w / r1 + (S > 1 ? reduce_t(S) : 0.0);
-    };
-    const double t_cur = model(kGmTile, P.ksplit);
-    double t_best = 0.97 * t_cur;
-    int best_s = 0;
-    const int n_kt64 = (k + kF32BkDeep - 1) / kF32BkDeep;
-    for (int S = 1; S <= 4; ++S) {
-      if (S > 1 && n_kt64 < 4 * S) break;
-      const double t = model(kGmTile / 2, S);
-      if (t < t_best) {
-        t_best = t;
-        best_s = S;
-      }
-    }
-    if (best_s) {
-      P.narrow = true;
-      P.tiles_m = (m + kGmTile / 2 - 1) / (kGmTile / 2);
-      P.tiles = 0;
-      for (int g = 0; g < G.count; ++g) P.tiles += P.tiles_m * ((G.n[g] + kGmTile - 1) / kGmTile);
-      P.ksplit = best_s;
-      P.f32_deep = true;
-      n_kt = n_kt64;
+  if (narrow) return cap(split);
+  // two items a CU at the rate, a lone one at 0.71 of it, 64-row ones at 0.865
+  const double r2 = rate / cus, r1 = r2 * (0.58 / 0.82);
+  auto model = [&](int tm, int S) {
+    const int64_t per_cu = (tiles_of(tm) * S + cus - 1) / cus;
+    const double w = 2.0 * tm * kGmTile * (double)k / S / (tm < kGmTile ? 0.865 : 1.0);
+    return (double)(per_cu - per_cu % 2) * w / r2 + (double)(per_cu % 2) * w / r1 + (S > 1 ? reduce_t(S) : 0.0);
+  };
+  double t_best = 0.97 * model(kGmTile, split);
+  for (int S = 1; S <= 4 && (S == 1 || (k + 31) / 32 >= 4 * S); ++S) {
+    const double t = model(kGmTile / 2, S);
+    if (t < t_best) {
+      t_best = t;
+      split = S;
     }
   }
-  P.kt_per = (n_kt + P.ksplit - 1) / P.ksplit;
-  P.ws_bytes = P.ksplit > 1 ? (size_t)P.ksplit * m * ncols * sizeof(float) : 0;
-  return P;
+  return cap(split);
 }
 
 // Whether a 16-bit product whose rows are 16-byte aligned runs on
 // gemm_wide_kernel: k in whole 16-byte chunks (its last stage drops the chunks
 // past k, and only whole ones), and 32-bit offsets for a row tile of A and for
 // the stages its prefetch counts past the end of each B.
-bool wide_ok(const GemmGroups& G, int m, int k, int64_t lda) {
+bool wide_ok(const GemmGroups& G, int k, int64_t lda) {
   bool ok = k % 8 == 0 && lda * 2 * 256 < ((int64_t)1 << 31);
   for (int g = 0; g < G.count; ++g) ok = ok && ((int64_t)k + 512) * G.ldb[g] * 2 < ((int64_t)1 << 32);
   return ok;
-}
-
-// Fills the K split of p, whose tile0 is set: slices, partials' places, items per XCD.
-void set_split(GemmParams& p, int m, int ksplit, int kt_per, void* workspace) {
-  p.ksplit = ksplit;
-  p.kt_per = kt_per;
-  p.ws = (float*)workspace;
-  int64_t off = 0;
-  for (int g = 0; g < p.G.count; ++g) {
-    p.ws_off[g] = off;
-    off += (int64_t)ksplit * m * p.G.n[g];
-  }
-  p.per_xcd = (p.G.tile0[p.G.count] * ksplit + 7) / 8;
-}
-
-template <typename T>
-int launch_split_reduce(const GemmParams& p, int m, hipStream_t st) {
-  int64_t runs = 0;
-  for (int g = 0; g < p.G.count; ++g) runs = (int64_t)m * (p.G.n[g] / 4) > runs ? (int64_t)m * (p.G.n[g] / 4) : runs;
-  const unsigned rb = (unsigned)((runs + 255) / 256 < 4096 ? (runs + 255) / 256 : 4096);
-  hipLaunchKernelGGL((split_reduce_kernel<T>), dim3(rb, p.G.count), dim3(256), 0, st, p);
-  return tl_launch_status();
 }
 
 template <typename T>
@@ -780,51 +710,51 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
               ((int64_t)k + 64 + 1) * G.ldb[g] * esize < ((int64_t)1 << 32);
     widest = G.n[g] > widest ? G.n[g] : widest;
   }
-  if constexpr (T::size == 2) {
-    if (aligned && wide_ok(G, m, k, lda)) {
-      // as many K-slices as the workspace query's plan has, where it was given
-      const PromptPlan P = prompt_plan(m, k, G, 2);
-      const bool room = workspace && workspace_bytes >= P.ws_bytes && ((uintptr_t)workspace % 16) == 0;
-      const WidePlan W = gemm_wide_plan(m, k, G, room ? P.ksplit : 1);
-      p.tiles_m = (m + W.tm - 1) / W.tm;
+  if (aligned) {
+    // as many K-slices as the workspace query's answer holds, where it was given
+    const SplitCap cap = split_cap(m, k, G, (int)esize);
+    const int max_split = workspace && workspace_bytes >= cap.ws_bytes && ((uintptr_t)workspace % 16) == 0 ? cap.ksplit : 1;
+    // tiles of tm x tn, K in ksplit slices of kt_per stages, run columns a store
+    auto place = [&](int tm, int tn, int ksplit, int kt_per, int run) {
+      p.tiles_m = (m + tm - 1) / tm;
       for (int g = 0; g < G.count; ++g) {
-        p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + W.tn - 1) / W.tn);
-        // whole runs: 8 columns from the kernel, 4 from the reduce
-        const int run = W.ksplit > 1 ? 4 : 8;
+        p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + tn - 1) / tn);
         if (G.ldc[g] % run == 0 && ((uintptr_t)G.c[g] % (run * esize)) == 0) p.vec_store |= 1 << g;
       }
-      set_split(p, m, W.ksplit, W.kt_per, workspace);
-      const int e = launch_gemm_wide<T>(p, W, st);
-      return e || p.ksplit == 1 ? e : launch_split_reduce<T>(p, m, st);
-    }
-  }
-  if (aligned) {
-    const PromptPlan P = prompt_plan(m, k, G, (int)esize);
-    p.tiles_m = P.tiles_m;
-    p.G.tile0[0] = 0;
-    p.vec_store = 0;
-    for (int g = 0; g < G.count; ++g) {
-      p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + kGmTile - 1) / kGmTile);
-      if (G.ldc[g] % 4 == 0 && ((uintptr_t)G.c[g] % (4 * esize)) == 0) p.vec_store |= 1 << g;
-    }
-    // the split needs its partials' workspace; without it the product runs whole
-    const bool split = P.ksplit > 1 && workspace && workspace_bytes >= P.ws_bytes && ((uintptr_t)workspace % 16) == 0;
-    set_split(p, m, split ? P.ksplit : 1, split ? P.kt_per : (k + 15) / 16 + 1, workspace);  // whole: one slice covers every stage
-    // fp32 is within 1% across stage shapes and keeps 16 k in three stages,
-    // except the 64-row tiles a prompt takes by the occupancy model (kF32BkDeep).
-    const dim3 grid((unsigned)(8 * p.per_xcd));
-    if constexpr (T::size == 2) {
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 2, 2>), grid, dim3(kGmThreads), 0, st, p);
+      p.ksplit = ksplit;
+      p.kt_per = kt_per;
+      p.ws = (float*)workspace;
+      int64_t off = 0;
+      for (int g = 0; g < G.count; ++g) {
+        p.ws_off[g] = off;
+        off += (int64_t)ksplit * m * G.n[g];
+      }
+      p.per_xcd = (p.G.tile0[G.count] * ksplit + 7) / 8;
+    };
+    int e;
+    if (T::size == 4 && k % 4 == 0) {
+      const F32Plan W = gemm_f32_plan(m, k, G, max_split);
+      place(W.tm, kGmTile, W.ksplit, W.kt_per, 4);
+      e = launch_gemm_f32(p, W.tm, st);
+    } else if (T::size == 2 && wide_ok(G, k, lda)) {
+      const WidePlan W = gemm_wide_plan(m, k, G, max_split);
+      place(W.tm, W.tn, W.ksplit, W.kt_per, W.ksplit > 1 ? 4 : 8);  // the reduce stores 4 columns, the kernel 8
+      e = launch_gemm_wide(p, W, (int)T::code, st);
     } else {
-      if (P.narrow && P.f32_deep)
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 4 * kF32BkDeep, 3, 1>), grid, dim3(kGmThreads), 0, st, p);
-      else if (P.narrow)
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 4 * kF32Bk, 3, 1>), grid, dim3(kGmThreads), 0, st, p);
-      else
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 4 * kF32Bk, 3, 2>), grid, dim3(kGmThreads), 0, st, p);
+      // the stage of gemm_mfma_kernel: 64 k (16-bit), kF32Bk k (fp32)
+      const int bk = T::size == 2 ? 64 : kF32Bk, n_kt = (k + bk - 1) / bk;
+      place(kGmTile, kGmTile, max_split, (n_kt + max_split - 1) / max_split, 4);
+      const dim3 grid((unsigned)(8 * p.per_xcd));
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, T::size == 2 ? 128 : 4 * kF32Bk, T::size == 2 ? 2 : 3>), grid, dim3(kGmThreads),
+                         0, st, p);
+      e = tl_launch_status();
     }
-    const int e = tl_launch_status();
-    return e || p.ksplit == 1 ? e : launch_split_reduce<T>(p, m, st);
+    if (e || p.ksplit == 1) return e;
+    int64_t runs = 0;
+    for (int g = 0; g < G.count; ++g) runs = (int64_t)m * (G.n[g] / 4) > runs ? (int64_t)m * (G.n[g] / 4) : runs;
+    const unsigned rb = (unsigned)((runs + 255) / 256 < 4096 ? (runs + 255) / 256 : 4096);
+    hipLaunchKernelGGL((split_reduce_kernel<T>), dim3(rb, G.count), dim3(256), 0, st, p);
+    return tl_launch_status();
   }
   dim3 grid((unsigned)((widest + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)G.count);
   hipLaunchKernelGGL((gemm_simple_kernel<T>), grid, dim3(256), 0, st, p);
@@ -923,7 +853,7 @@ size_t groups_workspace_bytes(int m, int k, const GemmGroups& G, int dtype) {
   // (if its plan splits; a product that falls back to the simple kernel
   // uses none of it)
   if (m <= kSkinnyMaxM) return skinny_workspace_bytes(m, live, k, esize);
-  return prompt_plan(m, k, live, esize).ws_bytes;
+  return split_cap(m, k, live, esize).ws_bytes;
 }
 
 }  // namespace

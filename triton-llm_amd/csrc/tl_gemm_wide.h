@@ -19,7 +19,6 @@ WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int max_split);
 
 // p's tiles, split and items are w's; p.vec_store marks the groups whose rows
 // take 16-byte stores (the reduce's own runs when K is split).
-template <typename T>
-int launch_gemm_wide(const GemmParams& p, const WidePlan& w, hipStream_t st);
+int launch_gemm_wide(const GemmParams& p, const WidePlan& w, int dtype, hipStream_t st);
 
 }  // namespace tlg

@@ -330,24 +330,31 @@ WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int max_split) {
   return best;
 }
 
+namespace {
 template <typename T>
-int launch_gemm_wide(const GemmParams& p, const WidePlan& w, hipStream_t st) {
+void launch(const GemmParams& p, const WidePlan& w, hipStream_t st) {
   const dim3 grid((unsigned)(8 * p.per_xcd)), block(256);
   if (w.tm == 256)
     hipLaunchKernelGGL((gemm_wide_kernel<T, 8, 8, 5>), grid, block, 0, st, p);
   else if (w.tm == 192)
     hipLaunchKernelGGL((gemm_wide_kernel<T, 6, 8, 5>), grid, block, 0, st, p);
+  else if (w.tm == 64)
+    hipLaunchKernelGGL((gemm_wide_kernel<T, 2, 4, 12>), grid, block, 0, st, p);
   else if (w.tn == 256)
     hipLaunchKernelGGL((gemm_wide_kernel<T, 4, 8, 6>), grid, block, 0, st, p);
   else if (w.tn == 192)
     hipLaunchKernelGGL((gemm_wide_kernel<T, 4, 6, 8>), grid, block, 0, st, p);
-  else if (w.tm == 64)
-    hipLaunchKernelGGL((gemm_wide_kernel<T, 2, 4, 12>), grid, block, 0, st, p);
   else
     hipLaunchKernelGGL((gemm_wide_kernel<T, 4, 4, 8>), grid, block, 0, st, p);
+}
+}  // namespace
+
+int launch_gemm_wide(const GemmParams& p, const WidePlan& w, int dtype, hipStream_t st) {
+  if (dtype == TL_DTYPE_BF16)
+    launch<BF16>(p, w, st);
+  else
+    launch<F16>(p, w, st);
   return tl_launch_status();
 }
-template int launch_gemm_wide<BF16>(const GemmParams&, const WidePlan&, hipStream_t);
-template int launch_gemm_wide<F16>(const GemmParams&, const WidePlan&, hipStream_t);
 
 }  // namespace tlg
