@@ -10,6 +10,7 @@ point raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 from ._build import LIB_PATH
@@ -147,8 +148,10 @@ def noalloc_scratch_bytes() -> int:
     return int(ctypes.c_size_t.in_dll(load(), "tl_decode_noalloc_scratch_bytes").value)
 
 
+@functools.lru_cache(maxsize=1024)
 def strides(*vals: int) -> ctypes.Array:
-    """Pack element strides into the int64[] the C ABI takes."""
+    """Pack element strides into the int64[] the C ABI takes (which only reads
+    them: calls of one shape share an array)."""
     arr = (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
     return arr
 

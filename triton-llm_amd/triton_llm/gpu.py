@@ -30,6 +30,7 @@ ziliangpeng/triton-llm: ``DeviceTensor`` :184-227, ``allocate`` :230,
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 import threading
 
@@ -49,12 +50,15 @@ bfloat16 = np.dtype(np.uint16, metadata={"triton_llm.dtype": "bfloat16"})
 _SUPPORTED_COMPUTE = {"float32": _lib.DTYPE_F32, "float16": _lib.DTYPE_F16, "bfloat16": _lib.DTYPE_BF16}
 
 
+_NAME_BY_CHAR = {"f": "float32", "e": "float16"}  # np.dtype.name takes a microsecond to put together
+
+
 def dtype_name(dtype) -> str:
     """Canonical dtype name; ``'bfloat16'`` for the tagged uint16 dtype."""
     dt = np.dtype(dtype)
     if dt.metadata and dt.metadata.get("triton_llm.dtype") == "bfloat16":
         return "bfloat16"
-    return dt.name
+    return _NAME_BY_CHAR.get(dt.char) or dt.name
 
 
 def dtype_code(dtype) -> int:
@@ -224,7 +228,7 @@ class DeviceTensor:
 
     @property
     def size(self):
-        return int(np.prod(self.shape)) if self.shape else 1
+        return math.prod(self.shape) if self.shape else 1
 
 
 # Keep-alive lists of the active graph captures and launcher recordings
@@ -246,7 +250,7 @@ def allocate(shape, dtype=np.float32):
     rounded size if one is free, else ``hipMalloc``."""
     _initialize()
     shape = tuple(int(s) for s in shape)
-    nbytes = int(np.prod(shape) * np.dtype(dtype).itemsize)
+    nbytes = math.prod(shape) * np.dtype(dtype).itemsize
     if nbytes == 0:
         return DeviceTensor(ctypes.c_void_p(), shape, dtype, 0)
     size = _block_size(nbytes)
@@ -302,8 +306,8 @@ def synchronize():
 
 def view(tensor: DeviceTensor, new_shape: tuple) -> DeviceTensor:
     """Zero-copy reshape; the view does not own the memory (reference gpu.py:266)."""
-    n_elems = int(np.prod(tensor.shape))
-    n_new = int(np.prod(new_shape))
+    n_elems = math.prod(tensor.shape)
+    n_new = math.prod(new_shape)
     if n_elems != n_new:
         raise ValueError(
             f"Cannot view {tensor.shape} ({n_elems} elements) as "

@@ -77,6 +77,9 @@ def record(thunk) -> Launcher:
 
 def same_dtype(*tensors) -> int:
     """Dtype code shared by all tensors; ValueError if they differ."""
+    first = tensors[0].dtype
+    if all(t.dtype is first for t in tensors):  # one dtype object, as tensors of a call mostly have
+        return gpu.dtype_code(first)
     names = {gpu.dtype_name(t.dtype) for t in tensors}
     if len(names) != 1:
         raise ValueError(f"inputs must share one dtype, got {sorted(names)}")

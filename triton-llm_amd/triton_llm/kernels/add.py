@@ -4,6 +4,8 @@ float32, float16 and bfloat16, fp32 arithmetic."""
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from triton_llm import gpu
@@ -16,7 +18,7 @@ def add(x_dev: "gpu.DeviceTensor", y_dev: "gpu.DeviceTensor",
     assert x_dev.shape == y_dev.shape, f"Shape mismatch: {x_dev.shape} vs {y_dev.shape}"
     if out_dev is not None:
         assert out_dev.shape == x_dev.shape, f"out_dev shape mismatch: expected {x_dev.shape}, got {out_dev.shape}"
-    N = int(np.prod(x_dev.shape))
+    N = math.prod(x_dev.shape)
     if out_dev is None:
         out_dev = gpu.allocate(x_dev.shape, x_dev.dtype)
     if N == 0:

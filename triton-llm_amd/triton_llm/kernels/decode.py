@@ -24,6 +24,8 @@ it is not modified (the caller advances it, as the model advances
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from triton_llm import gpu
@@ -78,7 +80,7 @@ def rope_kv_append(q_dev, k_new, v_new, k_cache, v_cache, cache_lens,
     else:
         raise ValueError(f"k_new must be 3-D or 4-D, got {k_new.shape}")
     kv_shape = (batch, n_new, n_kv, d_k)
-    if int(np.prod(k_new.shape)) != int(np.prod(kv_shape)) or k_new.shape[0] != batch or k_new.shape[-1] != d_k:
+    if math.prod(k_new.shape) != math.prod(kv_shape) or k_new.shape[0] != batch or k_new.shape[-1] != d_k:
         raise ValueError(f"k_new shape {k_new.shape} does not match cache {k_cache.shape}")
     if v_new.shape != k_new.shape:
         raise ValueError(f"v_new shape {v_new.shape} != k_new shape {k_new.shape}")
@@ -86,8 +88,8 @@ def rope_kv_append(q_dev, k_new, v_new, k_cache, v_cache, cache_lens,
     if q_dev is not None:
         if q_dev.shape[0] != batch or q_dev.shape[-1] != d_k:
             raise ValueError(f"q shape {q_dev.shape} does not match cache {k_cache.shape}")
-        n_head = int(np.prod(q_dev.shape)) // (batch * n_new * d_k)
-        if n_head * batch * n_new * d_k != int(np.prod(q_dev.shape)) or n_head % n_kv:
+        n_head = math.prod(q_dev.shape) // (batch * n_new * d_k)
+        if n_head * batch * n_new * d_k != math.prod(q_dev.shape) or n_head % n_kv:
             raise ValueError(f"q shape {q_dev.shape} is not (batch, n_new, n_head, d_k)")
     _check_lens(cache_lens, batch)
     tensors = [k_new, v_new, k_cache, v_cache] + ([q_dev] if q_dev is not None else [])
@@ -139,7 +141,7 @@ def attention_decode(q_dev, k_cache, v_cache, cache_lens, n_head: int, n_kv_head
         raise ValueError(f"cache has {n_kv} KV heads, n_kv_head={n_kv_head}")
     if n_head <= 0 or n_head % n_kv_head:
         raise ValueError(f"n_head ({n_head}) must be a positive multiple of n_kv_head ({n_kv_head})")
-    if int(np.prod(q_dev.shape)) != batch * n_head * d_k:
+    if math.prod(q_dev.shape) != batch * n_head * d_k:
         raise ValueError(f"q shape {q_dev.shape} is not (batch={batch}, n_head={n_head}, d_k={d_k})")
     if d_k not in (64, 128):
         raise ValueError(f"decode supports d_k in (64, 128), got {d_k}")
@@ -149,7 +151,7 @@ def attention_decode(q_dev, k_cache, v_cache, cache_lens, n_head: int, n_kv_head
         sm_scale = default_scale(d_k)
     if out is None:
         out = gpu.allocate((batch, n_head, d_k), q_dev.dtype)
-    elif int(np.prod(out.shape)) != batch * n_head * d_k or gpu.dtype_name(out.dtype) != gpu.dtype_name(q_dev.dtype):
+    elif math.prod(out.shape) != batch * n_head * d_k or gpu.dtype_name(out.dtype) != gpu.dtype_name(q_dev.dtype):
         raise ValueError(f"out must hold (batch, n_head, d_k) of the input dtype, got {out.shape}")
     ws_bytes, split = decode_workspace_bytes(batch, n_head, n_kv_head, max_ctx, d_k, split)
     ws = scratch(ws_bytes, workspace, key="decode")
@@ -181,10 +183,10 @@ def decode_step(q_dev, k_new, v_new, k_cache, v_cache, cache_lens, n_head: int, 
         raise ValueError(f"cache has {n_kv} KV heads, n_kv_head={n_kv_head}")
     if n_head <= 0 or n_head % n_kv_head:
         raise ValueError(f"n_head ({n_head}) must be a positive multiple of n_kv_head ({n_kv_head})")
-    if int(np.prod(q_dev.shape)) != batch * n_head * d_k or q_dev.shape[0] != batch or q_dev.shape[-1] != d_k:
+    if math.prod(q_dev.shape) != batch * n_head * d_k or q_dev.shape[0] != batch or q_dev.shape[-1] != d_k:
         raise ValueError(f"q shape {q_dev.shape} is not (batch={batch}, n_head={n_head}, d_k={d_k})")
     for name, t in (("k_new", k_new), ("v_new", v_new)):
-        if int(np.prod(t.shape)) != batch * n_kv * d_k or t.shape[0] != batch or t.shape[-1] != d_k:
+        if math.prod(t.shape) != batch * n_kv * d_k or t.shape[0] != batch or t.shape[-1] != d_k:
             raise ValueError(f"{name} shape {t.shape} is not (batch={batch}, n_kv_head={n_kv}, d_k={d_k})")
     if d_k not in (64, 128):
         raise ValueError(f"decode supports d_k in (64, 128), got {d_k}")
@@ -201,7 +203,7 @@ def decode_step(q_dev, k_new, v_new, k_cache, v_cache, cache_lens, n_head: int, 
         sm_scale = default_scale(d_k)
     if out is None:
         out = gpu.allocate((batch, n_head, d_k), q_dev.dtype)
-    elif int(np.prod(out.shape)) != batch * n_head * d_k or gpu.dtype_name(out.dtype) != gpu.dtype_name(q_dev.dtype):
+    elif math.prod(out.shape) != batch * n_head * d_k or gpu.dtype_name(out.dtype) != gpu.dtype_name(q_dev.dtype):
         raise ValueError(f"out must hold (batch, n_head, d_k) of the input dtype, got {out.shape}")
     ws_bytes, split = decode_workspace_bytes(batch, n_head, n_kv_head, max_ctx, d_k, split)
     ws = scratch(ws_bytes, workspace, key="decode")

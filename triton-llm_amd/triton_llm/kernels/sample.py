@@ -26,6 +26,7 @@ Ties with the k-th largest logit are all kept by the top_k filter
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 
@@ -73,7 +74,7 @@ def _flat_rows(logits_dev) -> tuple[int, int]:
     if len(logits_dev.shape) < 1 or logits_dev.shape[-1] <= 0:
         raise ValueError(f"logits must be (..., vocab) with vocab > 0, got {logits_dev.shape}")
     vocab = int(logits_dev.shape[-1])
-    return int(np.prod(logits_dev.shape[:-1], dtype=np.int64)), vocab
+    return math.prod(logits_dev.shape[:-1]), vocab
 
 
 def _launch(ptr: int, rows: int, vocab: int, row_stride: int, itemsize_dtype, temperature: float, top_k: int,

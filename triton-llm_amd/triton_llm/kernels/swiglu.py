@@ -6,6 +6,8 @@ output.  float32, float16 and bfloat16, fp32 arithmetic."""
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from triton_llm import gpu
@@ -17,7 +19,7 @@ def swiglu(gate_dev: "gpu.DeviceTensor", up_dev: "gpu.DeviceTensor",
     """GPU-resident SwiGLU activation. No sync, no host copies."""
     if gate_dev.shape != up_dev.shape:
         raise ValueError(f"gate_dev shape {gate_dev.shape} does not match up_dev shape {up_dev.shape}")
-    N = int(np.prod(gate_dev.shape))
+    N = math.prod(gate_dev.shape)
     if out_dev is not None:
         assert out_dev.shape == gate_dev.shape, f"out_dev shape mismatch: expected {gate_dev.shape}, got {out_dev.shape}"
     if out_dev is None:
