@@ -293,3 +293,36 @@ def test_sample_row_equals_batched_entry():
             gpu.synchronize()
             assert int(tok.to_numpy()[0]) == int(want[r])
         assert lib.tl_sample_row(row.ptr, V, T, k, 0.5, tok.ptr, ws.ptr, nws - 1, 0, None) != 0
+
+
+# top_k by 64-entry groups: the smallest and largest top_k of the route for a
+# vocabulary, one past it, group and segment remainders, rows not 16-byte
+# aligned, ties with the bound (more than the finish holds in LDS among them),
+# -inf entries, a NaN or +inf row.  The token has to be one the oracle's tie rule
+# keeps, and the one its inverse CDF picks (fp64, the same kept entries).
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("V", [128, 1000, 2048, 2113, 16384, 128256])
+def test_top_k_by_groups(dtype, V):
+    rng = np.random.default_rng(V)
+    groups = (V + 63) // 64
+    for top_k in sorted({1, max(1, groups // 2), groups // 2 + 1, min(V, 50)}):
+        print(f"[case] sample groups V={V} top_k={top_k} {dtype}", flush=True)
+        x = rng.standard_normal((8, V), dtype=np.float32) * 2
+        x[1] = 1.0                         # every entry ties
+        x[2] = np.round(x[2])              # many ties
+        x[3, rng.permutation(V)[: V - max(1, top_k // 2)]] = -np.inf  # fewer finite entries than top_k
+        x[4, V // 2], x[5, V - 1] = np.nan, np.inf
+        bits = on.to_storage(x, dtype)
+        xs = on.from_storage(bits, dtype)
+        u = rng.random(8)
+        got = H.download(sample_rows(H.upload(bits, dtype), 0.7, top_k, uniforms=u))
+        assert got[4] == -1 and got[5] == -1
+        for r in (0, 1, 2, 3, 6, 7):
+            row = xs[r].astype(np.float32)
+            kth = np.sort(row)[::-1][top_k - 1]
+            z = (row / np.float32(0.7)).astype(np.float32)
+            p = np.where(row >= kth, np.exp((z - z.max()).astype(np.float32)).astype(np.float64), 0.0)
+            c = np.cumsum(p)
+            exp = int(np.argmax(c > u[r] * c[-1]))
+            near = abs(c[got[r]] - u[r] * c[-1]) < 1e-5 * c[-1] or abs((c[got[r]] - p[got[r]]) - u[r] * c[-1]) < 1e-5 * c[-1]
+            assert p[got[r]] > 0 and (got[r] == exp or near), (r, got[r], exp)

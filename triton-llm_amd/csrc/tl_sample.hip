@@ -21,7 +21,9 @@
 //   * every segment records its maximum and first index;
 //   * without top_k it also records its mass at its own maximum,
 //     sum exp(x / T - m_seg / T) (fp64);
-//   * with top_k it keeps its own top_k (every entry >= its k-th largest, by
+//   * with top_k up to half the row's 64-entry groups it records each group's
+//     maximum (below);
+//   * with a larger top_k it keeps its own top_k (every entry >= its k-th largest, by
 //     a radix select on an order-preserving 32-bit key, 8 bits per step,
 //     counted with LDS atomics) as candidates, written in index order.  The row's k-th
 //     largest is >= each segment's k-th largest, so the candidates hold every
@@ -32,7 +34,11 @@
 //   * without top_k: segment masses rescaled to the row maximum locate the
 //     segment holding target = u * total, which is rescanned with the exact
 //     p = exp(x / T - max / T);
-//   * with top_k: the k-th largest candidate (radix select; candidates staged
+//   * with top_k by groups: the top_k-th largest group maximum is at most the
+//     row's k-th largest entry (top_k groups hold one that large), so only the
+//     groups that reach it are read again, and their entries that reach it, about
+//     top_k of them, are the candidates, in index order;
+//   * with top_k otherwise: the k-th largest candidate (radix select; candidates staged
 //     in LDS when they fit), then the inverse CDF over the kept candidates.
 // Every scan gives thread t the interval [lo_t, hi_t) of cumulative mass with
 // hi_t the same double as lo_{t+1}, so exactly one thread holds target.
@@ -55,6 +61,8 @@ constexpr int kMaxSeg = 128;                // segments per row (2 per lane of o
 constexpr int kMaxVocab = kMaxSeg * kSeg;   // 262144
 constexpr int kLdsCand = 6144;              // candidates the finishing workgroup stages in LDS
 constexpr int kMaxRows = 65535;             // grid.y
+constexpr int kGrp = 64;                    // entries of a group: 8 threads of a segment, one load of a wave
+constexpr int kMaxGrp = kMaxVocab / kGrp;   // groups per row
 
 struct Ws {
   double* mass;    // [rows][G] segment mass at the segment maximum
@@ -63,10 +71,15 @@ struct Ws {
   int* count;      // [rows][G] candidates kept by the segment
   float* cx;       // [rows][vocab] candidate logits, segment g's list at g * kSeg
   int* ci;         // [rows][vocab] their indices
+  // by groups, cx holds [rows][n_groups] group maxima instead
 };
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 int n_segments(int vocab) { return (vocab + kSeg - 1) / kSeg; }
+__host__ __device__ __forceinline__ int n_groups(int vocab) { return (vocab + kGrp - 1) / kGrp; }
+// Beyond half the groups the k-th group maximum excludes too little, and above
+// all of them nothing.
+__host__ __device__ __forceinline__ bool by_groups(int vocab, int top_k) { return 2 * top_k <= n_groups(vocab); }
 
 // Workspace layout; base == nullptr only sizes it.
 size_t ws_layout(int rows, int vocab, char* base, Ws* ws) {
@@ -141,6 +154,8 @@ struct LdsFin : LdsSeg {
   int off[kMaxSeg + 1];
   float cx[kLdsCand];
   int ci[kLdsCand];
+  unsigned short group[kMaxGrp];  // the groups that reach the bound
+  int cnt[2][kBW];
 };
 
 // (max, first index) over the workgroup; every thread gets the result.
@@ -250,6 +265,40 @@ __device__ __forceinline__ unsigned kth_key(Each&& each, unsigned need, LdsSeg& 
   return prefix;
 }
 
+// The same key by halving, one bit a step: key_at(q), q < slots (uniform), are
+// this thread's keys (0: none), top the largest of the row.  A step counts the
+// entries at or above a trial key by ballots.  No atomics: keys of one row
+// share their top bytes, and LDS atomics on one bin serialise, 5 ns an entry.
+// Stops when exactly `need` entries reach the prefix.
+// UNROLL > 0: that many slots, key_at's index known at compile time, no branches.
+template <int UNROLL = 0, class KeyAt>
+__device__ __forceinline__ unsigned kth_key_bits(KeyAt&& key_at, int slots, unsigned need, unsigned top, LdsFin& s) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned prefix = 0u;
+  int half = 0;
+  __syncthreads();  // earlier readers of s.cnt are done
+  for (int bit = 31; bit >= 0; --bit) {
+    const unsigned trial = prefix | 1u << bit;
+    if (trial > top) continue;
+    int c = 0;
+    if constexpr (UNROLL > 0) {
+#pragma unroll
+      for (int q = 0; q < UNROLL; ++q) c += __popcll(__ballot(key_at(q) >= trial));
+    } else {
+      for (int q = 0; q < slots; ++q) c += __popcll(__ballot(key_at(q) >= trial));
+    }
+    if (lane == 0) s.cnt[half][wave] = c;
+    __syncthreads();  // the other half of s.cnt is free: every thread is past its reads
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < kBW; ++w) total += s.cnt[half][w];
+    half ^= 1;
+    if (total >= (int)need) prefix = trial;
+    if (total == (int)need) break;
+  }
+  return prefix;
+}
+
 // One segment of one row: grid (segments, rows).
 template <typename T>
 __global__ __launch_bounds__(kBT) void segment_kernel(const void* logits, int64_t row_stride, int vocab,
@@ -267,8 +316,31 @@ __global__ __launch_bounds__(kBT) void segment_kernel(const void* logits, int64_
 
   // ---- this segment ----
   float x[kPer];
+  if (i0 + kPer <= vocab && ((uintptr_t)row & 15) == 0) {  // 16 bytes a load
+    constexpr int V = 16 / T::size;
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) x[j] = i0 + j < vocab ? logit<T>(row, i0 + j) : -INFINITY;
+    for (int q = 0; q < kPer / V; ++q) {
+      const u32x4 w = ((const u32x4*)row)[i0 / V + q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (T::size == 4) x[4 * q + e] = __uint_as_float(w[e]);
+        else unpack2<T>(w[e], x[2 * e], x[2 * e + 1]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) x[j] = i0 + j < vocab ? logit<T>(row, i0 + j) : -INFINITY;
+  }
+  if (filter && by_groups(vocab, top_k)) {
+    // the groups' maxima (a NaN is the largest) are all the finish needs
+    float gm = x[0];
+#pragma unroll
+    for (int j = 1; j < kPer; ++j) gm = __builtin_elementwise_maximum(gm, x[j]);
+#pragma unroll
+    for (int d = 1; d < kGrp / kPer; d <<= 1) gm = __builtin_elementwise_maximum(gm, __shfl_xor(gm, d));
+    if (tid % (kGrp / kPer) == 0 && i0 < vocab) ws.cx[(size_t)r * n_groups(vocab) + i0 / kGrp] = gm;
+    return;
+  }
   float m = -INFINITY;
   int a = INT_MAX;
 #pragma unroll
@@ -294,7 +366,7 @@ __global__ __launch_bounds__(kBT) void segment_kernel(const void* logits, int64_
     block_scan_d(v, lo, hi, tot, s);
     if (tid == 0) ws.mass[pi] = tot;
   }
-  if (filter) {
+  if (filter && !by_groups(vocab, top_k)) {
     unsigned thr = 0u;  // keep the whole segment when it has at most top_k entries
     if (top_k < nseg)
       thr = kth_key(
@@ -342,17 +414,35 @@ __global__ __launch_bounds__(kBT) void finish_kernel(const void* logits, int64_t
   const bool greedy = !(temperature > 0.f);
   const bool filter = !greedy && top_k > 0 && top_k < vocab;
 
+  const bool groups = filter && by_groups(vocab, top_k);
+  const double u = fmin(fmax(uniforms ? uniforms[r] : uniform, 0.0), 1.0);
+  // by groups, thread t: group maxima t * per .. , at most kMaxGrp / kBT of them
+  const int NG = n_groups(vocab), per = (NG + kBT - 1) / kBT;
+  float gmax[kMaxGrp / kBT];
   float M = -INFINITY;
   int A = INT_MAX;
-  if (tid < G) {
-    M = ws.smax[(size_t)r * G + tid];
-    A = ws.sarg[(size_t)r * G + tid];
+  if (groups) {
+#pragma unroll
+    for (int j = 0; j < kMaxGrp / kBT; ++j)
+      gmax[j] = j < per && tid * per + j < NG ? ws.cx[(size_t)r * NG + tid * per + j] : -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kMaxGrp / kBT; ++j) M = __builtin_elementwise_maximum(M, gmax[j]);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) M = __builtin_elementwise_maximum(M, __shfl_xor(M, d));
+    if (lane == 0) s.m[wave] = M;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kBW; ++w) M = __builtin_elementwise_maximum(M, s.m[w]);
+  } else {
+    if (tid < G) {
+      M = ws.smax[(size_t)r * G + tid];
+      A = ws.sarg[(size_t)r * G + tid];
+    }
+    block_argmax(M, A, s);
   }
-  block_argmax(M, A, s);
   if (tid == 0) out[r] = greedy ? A : -1;  // sampling: replaced below by the thread holding the draw
   if (greedy || !(M > -INFINITY && M < INFINITY)) return;
   const float Ms = M / temperature;
-  const double u = fmin(fmax(uniforms ? uniforms[r] : uniform, 0.0), 1.0);
 
   if (!filter) {
     // segment weights: mass at the segment maximum rescaled to the row's
@@ -436,19 +526,10 @@ __global__ __launch_bounds__(kBT) void finish_kernel(const void* logits, int64_t
     return;
   }
 
-  // ---- top_k: the candidates of all segments, in index order ----
-  if (wave == 0) {
-    const int g0 = 2 * lane, g1 = 2 * lane + 1;
-    const int c0 = g0 < G ? ws.count[(size_t)r * G + g0] : 0;
-    const int c1 = g1 < G ? ws.count[(size_t)r * G + g1] : 0;
-    const int incl = wave_incl_scan_i(c0 + c1, lane);
-    if (g0 < G) s.off[g0] = incl - c0 - c1;
-    if (g1 < G) s.off[g1] = incl - c1;
-    if (lane == 63) s.off[G] = incl;
-  }
-  __syncthreads();
-  const int C = s.off[G];
-  const bool staged = C <= kLdsCand;
+  // ---- top_k ----
+  int C;
+  bool staged;
+  unsigned thr;
   // position in the workspace of flat candidate f: the last segment whose
   // list starts at or before f (empty lists share their start with the next)
   auto locate = [&](int f) -> size_t {
@@ -462,40 +543,126 @@ __global__ __launch_bounds__(kBT) void finish_kernel(const void* logits, int64_t
     }
     return (size_t)r * vocab + (size_t)lo * kSeg + (size_t)(f - s.off[lo]);
   };
-  if (staged) {
-    // kStage loads per thread in flight: up to 4096 candidates in one round trip
-    constexpr int kStage = 16;
-    for (int f0 = tid; f0 < C; f0 += kStage * kBT) {
-      size_t at[kStage];
-      float vx[kStage];
-      int vi[kStage];
+  // candidates in LDS; else, by groups, every entry of the row is one
+  auto cand_x = [&](int f) -> float { return staged ? s.cx[f] : groups ? logit<T>(row, f) : ws.cx[locate(f)]; };
+  auto cand_i = [&](int f) -> int { return staged ? s.ci[f] : groups ? f : ws.ci[locate(f)]; };
+  if (groups) {
+    unsigned key[kMaxGrp / kBT];
 #pragma unroll
-      for (int q = 0; q < kStage; ++q) at[q] = f0 + q * kBT < C ? locate(f0 + q * kBT) : 0;
+    for (int j = 0; j < kMaxGrp / kBT; ++j) key[j] = j < per && tid * per + j < NG ? order_key(gmax[j]) : 0u;
+    const unsigned top = order_key(M);
+    auto key_at = [&](int j) { return key[j]; };
+    const unsigned bound = per <= 4   ? kth_key_bits<4>(key_at, 4, (unsigned)top_k, top, s)
+                           : per <= 8 ? kth_key_bits<8>(key_at, 8, (unsigned)top_k, top, s)
+                                      : kth_key_bits<kMaxGrp / kBT>(key_at, kMaxGrp / kBT, (unsigned)top_k, top, s);
+    // their list, in index order
+    int c = 0;
 #pragma unroll
-      for (int q = 0; q < kStage; ++q)
-        if (f0 + q * kBT < C) {
-          vx[q] = ws.cx[at[q]];
-          vi[q] = ws.ci[at[q]];
+    for (int j = 0; j < kMaxGrp / kBT; ++j) c += key[j] != 0u && key[j] >= bound ? 1 : 0;
+    const int incl = wave_incl_scan_i(c, lane);
+    if (lane == 63) s.i[wave] = incl;
+    __syncthreads();
+    int pos = incl - c, n_sel = 0;
+#pragma unroll
+    for (int w = 0; w < kBW; ++w) {
+      if (w < wave) pos += s.i[w];
+      n_sel += s.i[w];
+    }
+#pragma unroll
+    for (int j = 0; j < kMaxGrp / kBT; ++j)
+      if (key[j] != 0u && key[j] >= bound) s.group[pos++] = (unsigned short)(tid * per + j);
+    __syncthreads();
+    // Each wave takes a run of the list, a group a load, kFly loads in flight:
+    // first how many entries reach the bound, then (if they fit) their places.
+    constexpr int kFly = 16;
+    const int chunk = (n_sel + kBW - 1) / kBW;
+    const int b0 = min(n_sel, wave * chunk), b1 = min(n_sel, b0 + chunk);
+    int base = 0;
+    float v[kFly];
+    auto walk = [&](bool write) {
+      for (int b = b0; b < b1; b += kFly) {
+        if (!write || b1 - b0 > kFly) {  // a list of one batch is still in registers
+#pragma unroll
+          for (int q = 0; q < kFly; ++q) {
+            const int i = b + q < b1 ? (int)s.group[b + q] * kGrp + lane : vocab;
+            v[q] = i < vocab ? logit<T>(row, i) : NAN;
+          }
         }
 #pragma unroll
-      for (int q = 0; q < kStage; ++q)
-        if (f0 + q * kBT < C) {
-          s.cx[f0 + q * kBT] = vx[q];
-          s.ci[f0 + q * kBT] = vi[q];
+        for (int q = 0; q < kFly; ++q) {
+          const bool in = v[q] == v[q] && order_key(v[q]) >= bound;  // a finite row maximum: no NaN in the row
+          const unsigned long long m = __ballot(in);
+          if (write && in) {
+            const int at = base + __popcll(m & ((1ull << lane) - 1));
+            s.cx[at] = v[q];
+            s.ci[at] = (int)s.group[b + q] * kGrp + lane;
+          }
+          base += __popcll(m);
         }
+      }
+    };
+    walk(false);
+    if (lane == 0) s.a[wave] = base;
+    __syncthreads();
+    C = 0;
+    base = 0;
+#pragma unroll
+    for (int w = 0; w < kBW; ++w) {
+      if (w < wave) base += s.a[w];
+      C += s.a[w];
+    }
+    staged = C <= kLdsCand;  // thousands of ties with the bound: walk the row itself
+    if (staged) walk(true);
+    else C = vocab;
+    __syncthreads();
+    thr = kth_key_bits([&](int q) { return q * kBT + tid < C ? order_key(cand_x(q * kBT + tid)) : 0u; },
+                       (C + kBT - 1) / kBT, (unsigned)top_k, top, s);
+  } else {
+    // the candidates of all segments, in index order
+    if (wave == 0) {
+      const int g0 = 2 * lane, g1 = 2 * lane + 1;
+      const int c0 = g0 < G ? ws.count[(size_t)r * G + g0] : 0;
+      const int c1 = g1 < G ? ws.count[(size_t)r * G + g1] : 0;
+      const int incl = wave_incl_scan_i(c0 + c1, lane);
+      if (g0 < G) s.off[g0] = incl - c0 - c1;
+      if (g1 < G) s.off[g1] = incl - c1;
+      if (lane == 63) s.off[G] = incl;
     }
     __syncthreads();
+    C = s.off[G];
+    staged = C <= kLdsCand;
+    if (staged) {
+      // kStage loads per thread in flight: up to 4096 candidates in one round trip
+      constexpr int kStage = 16;
+      for (int f0 = tid; f0 < C; f0 += kStage * kBT) {
+        size_t at[kStage];
+        float vx[kStage];
+        int vi[kStage];
+  #pragma unroll
+        for (int q = 0; q < kStage; ++q) at[q] = f0 + q * kBT < C ? locate(f0 + q * kBT) : 0;
+  #pragma unroll
+        for (int q = 0; q < kStage; ++q)
+          if (f0 + q * kBT < C) {
+            vx[q] = ws.cx[at[q]];
+            vi[q] = ws.ci[at[q]];
+          }
+  #pragma unroll
+        for (int q = 0; q < kStage; ++q)
+          if (f0 + q * kBT < C) {
+            s.cx[f0 + q * kBT] = vx[q];
+            s.ci[f0 + q * kBT] = vi[q];
+          }
+      }
+      __syncthreads();
+    }
+    // the row's k-th largest key among the candidates (C >= top_k: every
+    // segment kept min(top_k, its size) or more)
+    thr = kth_key(
+        [&](auto&& fn) {
+          for (int f = tid; f < C; f += kBT) fn(order_key(cand_x(f)));
+        },
+        (unsigned)top_k, s);
   }
-  auto cand_x = [&](int f) -> float { return staged ? s.cx[f] : ws.cx[locate(f)]; };
-  auto cand_i = [&](int f) -> int { return staged ? s.ci[f] : ws.ci[locate(f)]; };
-
-  // the row's k-th largest key among the candidates (C >= top_k: every
-  // segment kept min(top_k, its size) or more)
-  const unsigned thr = kth_key(
-      [&](auto&& fn) {
-        for (int f = tid; f < C; f += kBT) fn(order_key(cand_x(f)));
-      },
-      (unsigned)top_k, s);
 
   // inverse CDF over the kept candidates, contiguous runs per thread
   const int run = (C + kBT - 1) / kBT;
