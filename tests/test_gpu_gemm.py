@@ -538,3 +538,21 @@ def test_gemm_partial_k_chunk(dtype, K, lda, M):
         got = on.from_storage(H.download(c_d), dtype)
         np.testing.assert_allclose(got, exp, rtol=1e-4 if dtype == "float32" else 8e-3,
                                    atol=1e-4 if dtype == "float32" else 1e-2)
+
+
+# One and two tokens on the whole-K kernel: its largest K and one past it, its
+# largest tile count and one past it, ragged columns, groups, few rows of K.
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("M,K,Ns", [(1, 1024, (8, 520)), (1, 1025, (520,)), (2, 1024, (264, 8)), (1, 1, (8,)),
+                                    (1, 130, (8192,)), (1, 130, (8200,)), (2, 500, (2048,)), (2, 500, (2056,)),
+                                    (1, 64, (16392,))])
+def test_gemm_one_token_whole_k(dtype, M, K, Ns):
+    print(f"[case] gemm whole-k {dtype} {M}x{K} -> {Ns}", flush=True)
+    rng = np.random.default_rng(M + K + sum(Ns))
+    a = on.to_storage(rng.standard_normal((M, K), dtype=np.float32), dtype)
+    bs = [on.to_storage(rng.standard_normal((K, n), dtype=np.float32) / np.float32(np.sqrt(K)), dtype) for n in Ns]
+    outs = gemm_grouped(H.upload(a, dtype), [H.upload(b, dtype) for b in bs])
+    for b, o in zip(bs, outs):
+        exp = gemm_ref(on.from_storage(a, dtype), on.from_storage(b, dtype))
+        np.testing.assert_allclose(on.from_storage(H.download(o), dtype), exp, rtol=1e-4 if dtype == "float32" else 8e-3,
+                                   atol=1e-4 if dtype == "float32" else 1e-2)

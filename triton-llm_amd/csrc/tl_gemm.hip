@@ -192,6 +192,93 @@ __global__ __launch_bounds__(kSkThreads) void skinny_partial_kernel(const void* 
   }
 }
 
+// One or two decoded tokens against a short K: a whole column tile (8 lanes x 16
+// bytes) per workgroup of 16 waves, the waves' row groups covering all of K with
+// every load in flight at once, so the product is one launch and one round trip
+// to memory.  Latency-bound.  With K-slices the same product took two launches
+// and two round trips: SmolLM2-360M fp32 at one token, rotated weights, o 8.8 ->
+// 5.0 us, q/k/v 7.8 -> 6.3, gate/up 9.8 -> 8.7; two tokens o 9.3 -> 6.1.  K of
+// 2560 takes three rounds and lost (9.3 -> 11.5 us), and so do four or more rows
+// of 16-bit weights (10.1 -> 11.5): their unpacking is not spread over enough
+// workgroups.  Narrower tiles read lines in parts: q/k/v 8.6 us with 16 bytes a row.
+constexpr int kWholeThreads = 1024;
+constexpr int kWholeChunks = 8;                                     // lanes across a row
+constexpr int kWholeUnroll = 8;                                     // loads in flight per lane
+constexpr int kWholeMaxK = kWholeThreads / kWholeChunks * kWholeUnroll;  // 1024: one round
+constexpr int kWholeMaxTiles = 256;                                 // one token; a quarter of it for two
+
+template <typename T, int MT>
+__global__ __launch_bounds__(kWholeThreads) void skinny_whole_kernel(const void* __restrict__ a, GemmGroups G, int m, int k,
+                                                                     int64_t lda, int per_xcd) {
+  constexpr int CW = kWholeChunks;
+  constexpr int CPC = 16 / T::size;  // columns per 16-byte chunk
+  constexpr int COLS = CW * CPC;     // columns per tile
+  constexpr int RW = 64 / CW;        // rows a wave's load covers
+  constexpr int WV = kWholeThreads / 64;
+  using Bits = typename T::bits;
+  __shared__ float s_a[MT][kWholeMaxK];
+  __shared__ float s_sum[WV][MT * COLS];
+  // adjacent tiles on one XCD: their lines meet in its L2
+  const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (t >= G.tile0[G.count]) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane % CW, r = lane / CW;
+  const int grp = find_group(G.tile0, G.count, t);
+  const int n = G.n[grp];
+  const int64_t ldb = G.ldb[grp];
+  const int col0 = (t - G.tile0[grp]) * COLS;
+  const uint32_t nbytes = (uint32_t)((int64_t)(k - 1) * ldb * T::size + (int64_t)min(COLS, n - col0) * T::size);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)((const Bits*)G.b[grp] + col0), (short)0,
+                                                                      (int)nbytes, kBufRsrcWord3);
+  const uint32_t row_bytes = (uint32_t)(ldb * T::size);
+  u32x4 w[kWholeUnroll];
+#pragma unroll
+  for (int u = 0; u < kWholeUnroll; ++u)  // rows past k: zeros, with no memory access
+    w[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+        rs, (uint32_t)(RW * (WV * u + wave) + r) * row_bytes + (uint32_t)(c * 16), 0, 0));
+  for (int idx = tid; idx < MT * k; idx += kWholeThreads) {
+    const int mi = idx / k, kk = idx - mi * k;
+    s_a[mi][kk] = mi < m ? to_f32<T>(((const Bits*)a)[(int64_t)mi * lda + kk]) : 0.f;
+  }
+  float acc[MT][CPC];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < CPC; ++j) acc[i][j] = 0.f;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kWholeUnroll; ++u) {
+    const int kk = RW * (WV * u + wave) + r;
+    float f[CPC];
+    unpack_words<T>(w[u], f);
+    if (kk < k) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const float x = s_a[i][kk];
+#pragma unroll
+        for (int j = 0; j < CPC; ++j) acc[i][j] = fmaf(x, f[j], acc[i][j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < CPC; ++j) {
+      float v = acc[i][j];
+#pragma unroll
+      for (int d = CW; d < 64; d <<= 1) v += __shfl_xor(v, d);
+      if (r == 0) s_sum[wave][i * COLS + c * CPC + j] = v;
+    }
+  __syncthreads();
+  for (int idx = tid; idx < MT * COLS; idx += kWholeThreads) {
+    const int mi = idx / COLS, col = col0 + idx % COLS;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < WV; ++q) v += s_sum[q][idx];
+    if (mi < m && col < n) ((Bits*)G.c[grp])[(int64_t)mi * G.ldc[grp] + col] = from_f32<T>(v);
+  }
+}
+
 // C_g[mi][col] = sum over K-slices of the partials, rounded to T, for every
 // column of the concatenated width.  The sum is latency-bound: up to
 // kReduceBatch slices' loads are in flight at once (one round trip for the
@@ -218,6 +305,22 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
 
 template <typename T>
 int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* ws, hipStream_t st) {
+  if (m <= 2 && k <= kWholeMaxK) {
+    constexpr int cols = kWholeChunks * (16 / T::size);
+    int64_t tiles = 0;
+    for (int g = 0; g < G.count; ++g) tiles += (G.n[g] + cols - 1) / cols;
+    if (tiles <= (m == 1 ? kWholeMaxTiles : kWholeMaxTiles / 4)) {
+      G.tile0[0] = 0;
+      for (int g = 0; g < G.count; ++g) G.tile0[g + 1] = G.tile0[g] + (G.n[g] + cols - 1) / cols;
+      const int per_xcd = (G.tile0[G.count] + 7) / 8;
+      const dim3 grid((unsigned)(8 * per_xcd)), block(kWholeThreads);
+      if (m == 1)
+        hipLaunchKernelGGL((skinny_whole_kernel<T, 1>), grid, block, 0, st, a, G, m, k, lda, per_xcd);
+      else
+        hipLaunchKernelGGL((skinny_whole_kernel<T, 2>), grid, block, 0, st, a, G, m, k, lda, per_xcd);
+      return tl_launch_status();
+    }
+  }
   const SkinnyPlan s = skinny_plan(G, k, T::size);
   int ntot = 0;
   G.tile0[0] = 0;
