@@ -121,11 +121,14 @@ def test_prefill_seq_q_ne_seq_k(d128_kernel, sq, sk, d_k):
     (2, 6, 2, 37, 300, True),      # key-split, bottom-right causal, GQA
     (1, 4, 2, 300, 129, True),     # key-split, the first rows fully masked
     (1, 3, 3, 70, 70, False),      # key-split, non-causal, ragged
-    (1, 16, 4, 600, 600, True),    # 80 blocks of 128 rows: the tiled kernel
-    (1, 16, 16, 520, 520, False),  # tiled, non-causal
+    (1, 16, 4, 600, 600, True),    # key-split, 304 workgroups: both block orders
+    (1, 16, 16, 520, 520, False),
+    (2, 9, 3, 700, 833, True),     # key-split, 396 workgroups, bottom-right causal
+    (1, 18, 6, 1025, 1025, True),  # 162 blocks of 128 rows: the tiled kernel
+    (8, 4, 4, 500, 470, False),    # 128 blocks: tiled, non-causal
 ])
 def test_prefill_fp32_paths(B, Hq, Hkv, sq, sk, causal, d_k):
-    """fp32 runs the key-split kernel when fewer than 64 blocks of 128 query
+    """fp32 runs the key-split kernel when fewer than 128 blocks of 128 query
     rows would run, the tiled kernel otherwise; both against the oracle."""
     dt = "float32"
     print(f"[case] fp32 B={B} Hq={Hq} Hkv={Hkv} sq={sq} sk={sk} D={d_k} causal={causal}", flush=True)

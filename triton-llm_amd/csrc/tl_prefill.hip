@@ -990,9 +990,13 @@ __global__ __launch_bounds__(kThreads, D == 128 ? 1 : 2) void flash_fwd_f32(Flas
 // ---------------------------------------------------------------------------
 constexpr int KS_ROWS = 32;  // query rows per workgroup
 constexpr int KS_KEYS = 32;  // keys per chunk
-#ifndef KS_SMALL_GRID
-#define KS_SMALL_GRID 64
-#endif
+// 128-row blocks below which the keys are split: at half the CUs the tiled
+// kernel's blocks, a CU each, still take as long as their longest chain.  Causal,
+// key-split against tiled: 15 heads of d_k 64 at 700 / 1023 tokens (90 / 120
+// blocks) 40.7 / 41.5 against 59.2 / 83.6 us, 9 heads at 1500 (108) 67 / 123, 24
+// heads of d_k 128 at 400 (96) 47.6 / 69.2; at 192 blocks and d_k 128 it loses
+// (175 / 157), non-causal from 144 blocks on (135 / 109 us, 24 heads at 700).
+constexpr int KS_SMALL_GRID = 128;
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p) {
   constexpr int NDB = D / 32;
@@ -1001,9 +1005,13 @@ __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p) {
   __shared__ float s_o[3][NDB][16][64];  // waves 1..3's O^T accumulators, lane-minor (no bank conflicts)
 
   const int n_rb = (p.seq_q + KS_ROWS - 1) / KS_ROWS;
-  const int rb = n_rb - 1 - (int)(blockIdx.x % n_rb);  // longest blocks first
-  const int hq = (int)(blockIdx.x / n_rb) % p.n_head;
-  const int b = (int)(blockIdx.x / n_rb) / p.n_head;
+  // Longest blocks first in the heads of the first 256 workgroups, shortest first
+  // in those of the next, and so on: the second workgroup a CU gets then evens
+  // out the first (15 heads, 1023 tokens: 60.8 -> 41.5 us).
+  const int head = (int)(blockIdx.x / n_rb), at = (int)(blockIdx.x % n_rb);
+  const int rb = (head * n_rb / 256) & 1 ? at : n_rb - 1 - at;
+  const int hq = head % p.n_head;
+  const int b = head / p.n_head;
   const int hkv = hq / p.group;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1036,27 +1044,45 @@ __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p) {
   const float* kbase = (const float*)p.k + b * p.k_sb + hkv * p.k_sh;
   const float* vbase = (const float*)p.v + b * p.v_sb + hkv * p.v_sh;
   const float c = p.scale_log2;
+  // K^T operand: lane (lq, h) holds key kb + lq, d = h D/2 + 4 cc + i;
+  // V^T operand of step r: key kb + 8 (r / 4) + 4 h + r % 4, d = 32 db + lq.
+  auto load_chunk = [&](int kb, f32x4 (&kf)[NC], float (&vf)[16][NDB]) __attribute__((always_inline)) {
+    const int key = kb + lq;
+    const float* krow = kbase + (int64_t)min(key, p.seq_k - 1) * p.k_ss + h * (D / 2);
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) {
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      kf[cc] = key < p.seq_k ? *(const f32x4*)(krow + 4 * cc) : z;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int kv = kb + 8 * (r >> 2) + 4 * h + (r & 3);
+      const float* vrow = vbase + (int64_t)min(kv, p.seq_k - 1) * p.v_ss + lq;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) vf[r][db] = kv < p.seq_k ? vrow[32 * db] : 0.f;
+    }
+  };
+  // d_k 64: the wave's next chunk is loaded while this one's MFMAs run (the
+  // registers of two chunks fit beside the accumulators; at d_k 128 they do not):
+  // 3% to 10% off, and 25% where a CU holds two workgroups.
+  constexpr bool AHEAD = D == 64;
+  f32x4 kn[NC];
+  float vn[16][NDB];
+  if (AHEAD && wave < n_ch) load_chunk(wave * KS_KEYS, kn, vn);
   for (int ch = wave; ch < n_ch; ch += 4) {
     const int kb = ch * KS_KEYS;
-    // K^T operand: lane (lq, h) holds key kb + lq, d = h D/2 + 4 cc + i;
-    // V^T operand of step r: key kb + 8 (r / 4) + 4 h + r % 4, d = 32 db + lq.
     f32x4 kf[NC];
     float vf[16][NDB];
-    {
-      const int key = kb + lq;
-      const float* krow = kbase + (int64_t)min(key, p.seq_k - 1) * p.k_ss + h * (D / 2);
+    if constexpr (AHEAD) {
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) {
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        kf[cc] = key < p.seq_k ? *(const f32x4*)(krow + 4 * cc) : z;
-      }
+      for (int cc = 0; cc < NC; ++cc) kf[cc] = kn[cc];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kv = kb + 8 * (r >> 2) + 4 * h + (r & 3);
-        const float* vrow = vbase + (int64_t)min(kv, p.seq_k - 1) * p.v_ss + lq;
+      for (int r = 0; r < 16; ++r)
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) vf[r][db] = kv < p.seq_k ? vrow[32 * db] : 0.f;
-      }
+        for (int db = 0; db < NDB; ++db) vf[r][db] = vn[r][db];
+      if (ch + 4 < n_ch) load_chunk(kb + 4 * KS_KEYS, kn, vn);
+    } else {
+      load_chunk(kb, kf, vf);
     }
     f32x16 s;
 #pragma unroll
