@@ -325,3 +325,30 @@ def test_prefill_w64_and_w32_agree_on_5a_rows(monkeypatch):
         H.set_override(monkeypatch, "TRITON_LLM_HIP_PREFILL_W64", 1 if kernel == "w64" else None)
         outs[kernel] = gpu_prefill(cfg, raw)
     compare("5a w64 vs w32", outs["w64"], outs["w32"], TOL[cfg.dtype])
+
+
+@pytest.mark.parametrize("v_ss", [0, 8, 128, 136])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_v_row_strides(v_ss, causal):
+    """d_k 128 reads V rows in place; rows that overlap (a stride below d_k,
+    0 included) are copied first.  Both against the oracle on the rows spelled out."""
+    from triton_llm.kernels import flash_attention_strided
+    Hq, Hkv, sq, sk, d_k, dt = 4, 2, 300, 333, 128, "bfloat16"
+    print(f"[case] prefill v_ss={v_ss} causal={causal}", flush=True)
+    rng = np.random.default_rng(v_ss + 1)
+    q = on.to_storage(rng.standard_normal((1, Hq, sq, d_k), dtype=np.float32), dt)
+    k = on.to_storage(rng.standard_normal((1, Hkv, sk, d_k), dtype=np.float32), dt)
+    head = (sk - 1) * v_ss + d_k
+    flat = on.to_storage(rng.standard_normal((Hkv, head), dtype=np.float32), dt)
+    v = np.stack([np.stack([flat[h, i * v_ss:i * v_ss + d_k] for i in range(sk)]) for h in range(Hkv)])[None]
+    pad = (head + 7) // 8 * 8
+    flat8 = np.zeros((Hkv, pad), flat.dtype)
+    flat8[:, :head] = flat
+    q_d, k_d, v_d = H.upload(q, dt), H.upload(k, dt), H.upload(flat8, dt)
+    o_d = gpu.allocate(q.shape, q_d.dtype)
+    qs, ks = (Hq * sq * d_k, sq * d_k, d_k), (Hkv * sk * d_k, sk * d_k, d_k)
+    flash_attention_strided(q_d, k_d, v_d, o_d, batch=1, n_head=Hq, n_kv_head=Hkv, seq_q=sq, seq_k=sk, d_k=d_k,
+                            q_strides=qs, k_strides=ks, v_strides=(Hkv * pad, pad, v_ss), o_strides=qs, causal=causal)
+    got = on.from_storage(H.download(o_d), dt)
+    exp = oa.attention_bhsd(*(on.from_storage(x, dt) for x in (q, k, v)), causal=causal, dtype="float32")
+    compare(f"v_ss {v_ss}", got, exp, TOL[dt])

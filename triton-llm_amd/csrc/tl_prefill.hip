@@ -29,8 +29,9 @@
 // registers (lane half h holds keys 8a + 4h + b, b < 4, of each 32-key
 // block) and the V^T operand is read with the matching key permutation.
 //
-// Kernels: vt_pack_kernel + flash_fwd_16 (f16 / bf16, d_k 64 / 128), flash_fwd_f32
-// (fp32, d_k 64 / 128), attn_generic_kernel (any d_k <= 256).
+// Kernels: flash_fwd_16 (f16 / bf16, d_k 64 / 128; V in place, or copied by
+// vt_pack_kernel where its rows overlap), flash_fwd_f32 and flash_fwd_f32_ks
+// (fp32, d_k 64 / 128), attn_generic_kernel (the other head sizes).
 #include "tl_prefill.h"
 
 #include <math.h>
@@ -145,7 +146,7 @@ __device__ __forceinline__ void decode_block(const FlashParams& p, int& b, int& 
 // pre-scaled and rounded back to 16 bits.  Taken for fp16 when
 // |sm_scale * log2 e| > 1, where the pre-scaled Q could exceed the fp16
 // range (bf16 has fp32's range; the reference scales q in fp32).
-template <typename T, int D, bool CAUSAL, bool SCALE_S = false>
+template <typename T, int D, bool CAUSAL, bool SCALE_S, bool VNAT>
 __global__ __launch_bounds__(K16_THREADS, 2) void flash_fwd_16(FlashParams p) {
   using M = Mfma<T>;
   using frag = typename M::frag;
@@ -153,10 +154,10 @@ __global__ __launch_bounds__(K16_THREADS, 2) void flash_fwd_16(FlashParams p) {
   constexpr int BN = K16_BN;
   constexpr int ROWB = D * 2;          // bytes per K / Q row in LDS
   constexpr int VROWB = BN * 2;        // bytes per V^T row in LDS (256)
-  // d_k 64 reads V in its natural layout (no V^T copy): its softmax VALU
-  // work, not LDS, limits a step, so the PV operand's transposing LDS reads
-  // (two ds_read_b64_tr_b16 per fragment) are affordable there.
-  constexpr bool VNAT = D == 64;
+  // VNAT reads V in its natural layout (two ds_read_b64_tr_b16 a fragment, no
+  // V^T copy).  At d_k 128 the copy's launch cost more than the plain reads it
+  // bought: Llama-3.2-3B heads at 1000 / 1999 / 4096 / 8192 tokens 26.7 / 40.2 /
+  // 104.9 / 341.3 -> 24.1 / 36.3 / 99.6 / 338.2 us a call, 4 x 1024 45.3 -> 39.0.
   constexpr int TILEB = BN * ROWB;     // bytes per K, V^T or 128-row Q tile
   constexpr int NSL = ROWB / 16;       // 16-byte slots per K row
   constexpr int RPR = 1024 / ROWB;     // K rows per 1 KiB region
@@ -197,11 +198,12 @@ __global__ __launch_bounds__(K16_THREADS, 2) void flash_fwd_16(FlashParams p) {
     return ((uint32_t)row * (uint32_t)p.sk_pad + (uint32_t)(((ln % 16) ^ lds_swz<128>(row)) * 8)) * 2u;
   };
   // Natural V rows (VNAT): like K rows, chunk c of key row r at slot
-  // c ^ vnat_swz(r), vnat_swz(r) = 2 ((r >> 1) & 1).  A transposing read
-  // covers 4 consecutive rows of a 16-lane group (4 lanes per row, 8 bytes
-  // each); rows 2 apart share banks, and the XOR moves one of them by 32
-  // bytes, so the group's 16 reads hit 32 distinct banks.
-  auto vnat_swz = [](int r) __attribute__((always_inline)) { return 2 * ((r >> 1) & 1); };
+  // c ^ vnat_swz(r).  A transposing read covers 4 consecutive rows of a
+  // 16-lane group (4 lanes per row, 8 bytes each).  d_k 64: rows 2 apart share
+  // banks, and the XOR moves one of them by 32 bytes, so the group's 16 reads
+  // hit 32 distinct banks.  d_k 128: all rows share banks, and the XOR gives
+  // the four rows a 64-byte piece each, for both groups of a 32-lane half.
+  auto vnat_swz = [](int r) __attribute__((always_inline)) { return D == 64 ? 2 * ((r >> 1) & 1) : 4 * (r & 3); };
   auto vnat_off = [&](int ln) __attribute__((always_inline)) {
     const int row = wq * RPR + ln / NSL;
     return ((uint32_t)row * (uint32_t)p.v_ss + (uint32_t)(((ln % NSL) ^ vnat_swz(row)) * 8)) * 2u;
@@ -459,7 +461,7 @@ __global__ __launch_bounds__(K16_THREADS, 2) void flash_fwd_16(FlashParams p) {
             typedef short v4s __attribute__((ext_vector_type(4)));
             typedef __attribute__((address_space(3))) v4s lds_v4s;
             __attribute__((address_space(3))) char* lds = (__attribute__((address_space(3))) char*)smem;
-            const int off = vn_lane + tt * 16 * ROWB + db * 64;
+            const int off = (D == 64 ? vn_lane + db * 64 : vn_lane ^ (db << 6)) + tt * 16 * ROWB;
             const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds + off));
             const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds + off + 8 * ROWB));
             vfr[g] = u32x4{__builtin_bit_cast(u32x2, lo).x, __builtin_bit_cast(u32x2, lo).y,
@@ -1580,6 +1582,29 @@ static uint64_t next_split_token() {
   return t ? t : 1;
 }
 
+// V rows that flash_fwd_16 can read in place: a tile's reads are bounded by its
+// row count times the row stride, with 32-bit byte offsets.
+bool v_rows_ok(const FlashParams& p, int d_k) {
+  return p.v_ss >= d_k && (128 * p.v_ss + d_k) * 2 < ((int64_t)1 << 32);
+}
+
+template <typename T, int D, bool SCALE_S>
+int launch_flash_16_as(const FlashParams& p, bool causal, bool vnat, hipStream_t st) {
+  const dim3 grid((unsigned)(p.q_machines * p.n_queues)), block(K16_THREADS);
+  if (vnat) {
+    if (causal)
+      hipLaunchKernelGGL((flash_fwd_16<T, D, true, SCALE_S, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((flash_fwd_16<T, D, false, SCALE_S, true>), grid, block, 0, st, p);
+  } else if constexpr (D != 64) {
+    if (causal)
+      hipLaunchKernelGGL((flash_fwd_16<T, D, true, SCALE_S, false>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((flash_fwd_16<T, D, false, SCALE_S, false>), grid, block, 0, st, p);
+  }
+  return tl_launch_status();
+}
+
 template <typename T, int D>
 int launch_flash_16(FlashParams& p, void* ws, size_t ws_bytes, bool causal, hipStream_t st) {
   // fp16 Q pre-scaled by |sm_scale log2 e| > 1 could overflow: scale scores instead
@@ -1590,6 +1615,10 @@ int launch_flash_16(FlashParams& p, void* ws, size_t ws_bytes, bool causal, hipS
   // kernel on config 5a.  Not when the scores must be scaled in fp32 (fp16,
   // large scale); it addresses a wave's 64 output rows with 32-bit offsets.
   const bool w64 = D == 128 && !scale_s && tl_overrides.prefill_w64 && (64 * p.o_ss + D) * 2 < ((int64_t)1 << 32);
+  // V in place, unless its rows overlap or a tile of them passes 32-bit offsets
+  // (d_k 64 takes no such V: mfma_shape_ok) -- those are copied, as for flash_fwd_w64
+  const bool vnat = D == 64 || (!w64 && v_rows_ok(p, D));
+  // the copy's room is part of the workspace either way (the split region follows it)
   const size_t vt_need = D == 64 ? 0 : vt_bytes(p.batch, p.n_kv, p.seq_k, D);
   const size_t room = ws && aligned16(ws) && ws_bytes > align256(vt_need) ? ws_bytes - align256(vt_need) : 0;
   p.split_ws = nullptr;
@@ -1598,30 +1627,20 @@ int launch_flash_16(FlashParams& p, void* ws, size_t ws_bytes, bool causal, hipS
     p.split_ws = (char*)ws + align256(vt_need);
     p.split_token = next_split_token();
   }
-  if constexpr (D != 64) {  // d_k 64 reads V in place
-    const int vt_tiles = p.sk_pad / 64 * p.n_kv * p.batch;
-    const int vt_grid = min(vt_tiles, 2 * tl_device_cus());
-    hipLaunchKernelGGL(vt_pack_kernel<D>, dim3(vt_grid), dim3(256), 0, st, (const uint16_t*)p.v, (uint16_t*)ws,
-                       p.seq_k, p.sk_pad, p.n_kv, vt_tiles, p.v_sb, p.v_sh, p.v_ss);
-    const int e = tl_launch_status();
-    if (e) return e;
-  }
-  if (w64) return launch_flash_w64(p, T::code, causal, st);
-  dim3 grid((unsigned)(p.q_machines * p.n_queues));
-  if constexpr (std::is_same<T, F16>::value) {
-    if (scale_s) {
-      if (causal)
-        hipLaunchKernelGGL((flash_fwd_16<T, D, true, true>), grid, dim3(K16_THREADS), 0, st, p);
-      else
-        hipLaunchKernelGGL((flash_fwd_16<T, D, false, true>), grid, dim3(K16_THREADS), 0, st, p);
-      return tl_launch_status();
+  if constexpr (D != 64) {
+    if (!vnat) {
+      const int vt_tiles = p.sk_pad / 64 * p.n_kv * p.batch;
+      const int vt_grid = min(vt_tiles, 2 * tl_device_cus());
+      hipLaunchKernelGGL(vt_pack_kernel<D>, dim3(vt_grid), dim3(256), 0, st, (const uint16_t*)p.v, (uint16_t*)ws,
+                         p.seq_k, p.sk_pad, p.n_kv, vt_tiles, p.v_sb, p.v_sh, p.v_ss);
+      const int e = tl_launch_status();
+      if (e) return e;
     }
   }
-  if (causal)
-    hipLaunchKernelGGL((flash_fwd_16<T, D, true>), grid, dim3(K16_THREADS), 0, st, p);
-  else
-    hipLaunchKernelGGL((flash_fwd_16<T, D, false>), grid, dim3(K16_THREADS), 0, st, p);
-  return tl_launch_status();
+  if (w64) return launch_flash_w64(p, T::code, causal, st);
+  if constexpr (std::is_same<T, F16>::value)
+    if (scale_s) return launch_flash_16_as<T, D, true>(p, causal, vnat, st);
+  return launch_flash_16_as<T, D, false>(p, causal, vnat, st);
 }
 
 template <int D>
@@ -1669,8 +1688,8 @@ bool mfma_shape_ok(const FlashParams& p, int d_k, int dtype) {
         p.o_ss < d_k || (32 * p.o_ss + d_k) * 2 >= ((int64_t)1 << 32) ||
         (128 * p.q_ss + d_k) * 2 >= ((int64_t)1 << 32) || (int64_t)d_k * sk_pad * 2 >= ((int64_t)1 << 32))
       return false;
-    // d_k 64 reads V tiles in place, bounded like K's
-    if (d_k == 64 && (p.v_ss < d_k || (128 * p.v_ss + d_k) * 2 >= ((int64_t)1 << 32))) return false;
+    // d_k 64 has no copy of V to fall back to
+    if (d_k == 64 && !v_rows_ok(p, d_k)) return false;
   }
   return aligned16(p.q) && aligned16(p.k) && aligned16(p.v) && aligned16(p.o);
 }
@@ -1681,8 +1700,8 @@ extern "C" {
 
 size_t tl_attention_fwd_workspace_bytes(int batch, int n_kv_head, int seq_k, int d_k,
                                         int dtype) {
-  // 16-bit MFMA path at d_k 128: the permuted key-major V^T copy.  d_k 64,
-  // fp32 and the generic kernel read V in place.
+  // 16-bit MFMA path at d_k 128: room for the permuted key-major V^T copy that a
+  // V of overlapping rows and flash_fwd_w64 take.  The others read V in place.
   if (dtype == TL_DTYPE_F32 || batch <= 0 || n_kv_head <= 0 || seq_k <= 0 || d_k != 128)
     return 0;
   return vt_bytes(batch, n_kv_head, seq_k, d_k);
