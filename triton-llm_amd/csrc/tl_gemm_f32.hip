@@ -51,7 +51,7 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& h, uint32_t
 // Measured against the fp32 MFMA tiles it replaced, Llama-3.2-3B at 2048 rows:
 // gate/up 1555 -> 1071 us (193 TFLOP/s), q/k/v 522 -> 367, o 318 -> 223, down 809
 // -> 565; SmolLM2-360M at 1023 rows gate/up 108 -> 77, q/k/v 44 -> 39, o 31 -> 28,
-// down 53 -> 45; 9 to 300 rows equal or up to 1.8x faster.  What bounds it with two
+// down 53 -> 45; 96 products of 9 to 520 rows 0.97 to 1.87 times as fast.  What bounds it with two
 // workgroups a CU is the issue port (about 240 VALU instructions, 96 MFMAs and 49
 // LDS ones per wave and stage); a lone one waits on its own LDS reads.
 template <int MB>

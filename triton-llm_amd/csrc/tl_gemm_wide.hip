@@ -62,9 +62,11 @@ __device__ __forceinline__ void mma_drain() { asm volatile("s_nop 15\n\ts_nop 15
 //     panel order of gemm_tile_panels (hipBLASLt: 1290).
 //   * C through LDS, whole row pieces: epilogue 16600 -> 9000 cycles of a tile's
 //     150000, against 8-byte stores from the accumulators.
-// gate/up 205 -> 163 us (1250 TFLOP/s), down 122 -> 103, q/k/v 84 -> 55; 9 to 64
-// rows equal or up to 1.35x faster, 100 to 4096 rows 1.04x to 1.75x faster than
-// the 64-, 128- and 256-row tiles of gemm_mfma_kernel that this replaced.  What
+// gate/up 205 -> 163 us (1250 TFLOP/s), down 122 -> 103, q/k/v 84 -> 55; of 98
+// products of these models' shapes against the 64-, 128- and 256-row tiles of
+// gemm_mfma_kernel that this replaced, 9 to 64 rows ran at 0.96 to 1.36 times
+// their speed, 100 to 4096 rows at 1.04 to 1.76 times but for one, gate/up at 384
+// rows (53.8 -> 55.9 us; 58.0 -> 56.5 in a run of an earlier variant).  What
 // bounds it now: at 4 and more rounds the power limit (1.67 GHz), at one or two
 // the HBM latency of the weights and each tile's first loads and stores.
 //

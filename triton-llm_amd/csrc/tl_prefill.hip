@@ -102,12 +102,11 @@ __device__ __forceinline__ void decode_block(const FlashParams& p, int& b, int& 
 // exceeds it by more than kRescaleLog2 (log2 units), which bounds P by
 // 2^kRescaleLog2.
 //
-// V is read from a key-major copy V^T [b][kv][d][Sk_pad] written once per
-// call by vt_pack_kernel, with each 16-key group stored in the order the
-// MFMA's k-index permutation wants (see vt_pack_kernel), so the 8 keys a lane
-// feeds into one PV MFMA are one contiguous 16 bytes: ds_read_b128, the same
-// fast LDS path as the K operand.  (A transposing LDS read of natural V,
-// ds_read_b64_tr_b16, measured ~3x lower LDS throughput per byte on gfx950.)
+// V is read in place: its natural rows go to LDS like K's, and two transposing
+// reads (ds_read_b64_tr_b16) give a lane the 8 keys of one PV MFMA.  Where V's
+// rows overlap (d_k 128) a key-major copy V^T [b][kv][d][Sk_pad] is written
+// first by vt_pack_kernel, each 16-key group in the order the MFMA's k-index
+// permutation wants, so that those 8 keys are one contiguous 16 bytes.
 //
 // LDS rows are unpadded; the 16-byte chunk c of row r lives in slot
 // c ^ lds_swz(r) (lds_swz<D> for K and Q rows, lds_swz<128> for the 256-byte
