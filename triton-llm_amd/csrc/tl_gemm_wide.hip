@@ -66,7 +66,9 @@ __device__ __forceinline__ void mma_drain() { asm volatile("s_nop 15\n\ts_nop 15
 // products of these models' shapes against the 64-, 128- and 256-row tiles of
 // gemm_mfma_kernel that this replaced, 9 to 64 rows ran at 0.96 to 1.36 times
 // their speed, 100 to 4096 rows at 1.04 to 1.76 times but for one, gate/up at 384
-// rows (53.8 -> 55.9 us; 58.0 -> 56.5 in a run of an earlier variant).  What
+// rows (53.8 -> 55.9 us; again, twice a side in turn: 58.8, 57.7 -> 58.6, 58.9,
+// where 448 rows take 61.3 -> 52.7: the model misses the best tile there).  64 rows
+// of 2560 -> 960 are slower, 12.1 -> 12.5 us.  What
 // bounds it now: at 4 and more rounds the power limit (1.67 GHz), at one or two
 // the HBM latency of the weights and each tile's first loads and stores.
 //
