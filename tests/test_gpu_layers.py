@@ -161,3 +161,25 @@ def test_vector_and_scalar_routes(dtype, rel, offset):
         swiglu(ad, bd, yd)
         np.testing.assert_allclose(on.from_storage(H.download(yd), dtype), ol.swiglu_ref(af, bf), rtol=1e-5 + rel,
                                    atol=1e-6)
+
+
+# The 16-bit sigmoid's quotient is the IEEE division's, as in the fp32 kernel:
+# over every 16-bit gate value the 16-bit result is that of the fp32 kernel's
+# silu times up, rounded to fp32 and then to 16 bits (or, where the compiler
+# fuses the last product with the conversion, rounded to 16 bits at once).
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_swiglu_16bit_division_is_the_fp32_one(dtype):
+    rng = np.random.default_rng(23)
+    bits = np.tile(np.arange(65536, dtype=np.uint16), 64)
+    x = bits if dtype == "bfloat16" else bits.view(np.float16)
+    u = on.to_storage(2 * rng.standard_normal(bits.size, dtype=np.float32), dtype)
+    xf, uf = on.from_storage(x, dtype), on.from_storage(u, dtype)
+    silu = H.download(swiglu(gpu.to_device(xf), gpu.to_device(np.ones_like(xf))))
+    got = on.from_storage(H.download(swiglu(H.upload(x, dtype), H.upload(u, dtype))), dtype)
+    with np.errstate(all="ignore"):
+        twice = on.from_storage(on.to_storage(silu * uf, dtype), dtype)
+        # the products of 24- and 8- or 11-bit values are exact in fp64
+        exact = silu.astype(np.float64) * uf.astype(np.float64)
+        once = exact.astype(np.float16).astype(np.float32) if dtype == "float16" else twice
+    same = (got == twice) | (got == once) | (np.isnan(got) & np.isnan(twice))
+    assert same.all(), (int((~same).sum()), xf[~same][:4], uf[~same][:4])

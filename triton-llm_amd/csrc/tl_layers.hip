@@ -187,18 +187,25 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_kernel(const void* a, co
   for (int i = threadIdx.x; i < n; i += kRowThreads) st<T>(y, row + i, (ld<T>(src, row + i) / rms) * ld<T>(w, i));
 }
 
+// n / d for d in [1, 2] and n in [0, 1], bit for bit what the IEEE division
+// gives: its reciprocal, Newton step and two residual corrections, without the
+// scaling and special cases that no such operand needs (every n below 2^-25
+// comes with d == 1 here, where each step is exact).
+__device__ __forceinline__ float div_unit(float n, float d) {
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.f), r, r);
+  float q = n * r;
+  q = fmaf(fmaf(-d, q, n), r, q);
+  return fmaf(fmaf(-d, q, n), r, q);
+}
+
 // silu(x) * u with the single-exp stable sigmoid: exp(-|x|) <= 1 never
-// overflows, and one division serves both signs.  For the 16-bit types the
-// quotient is a product with v_rcp_f32 of 1 + e, a value in [1, 2] (1 ulp of
-// fp32, against an output rounding 2^13 times larger): the IEEE division's ten
-// instructions made the 16-bit kernel VALU-bound.
+// overflows, and one division serves both signs.
 struct SwigluOp {
   template <typename T>
   static __device__ __forceinline__ float apply(float x, float u) {
     const float e = expf(-fabsf(x));
-    const float num = x >= 0.f ? 1.f : e;
-    const float sig = T::size == 4 ? num / (1.f + e) : num * __builtin_amdgcn_rcpf(1.f + e);
-    return x * sig * u;
+    return x * div_unit(x >= 0.f ? 1.f : e, 1.f + e) * u;
   }
 };
 struct AddOp {
