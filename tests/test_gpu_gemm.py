@@ -556,3 +556,26 @@ def test_gemm_one_token_whole_k(dtype, M, K, Ns):
         exp = gemm_ref(on.from_storage(a, dtype), on.from_storage(b, dtype))
         np.testing.assert_allclose(on.from_storage(H.download(o), dtype), exp, rtol=1e-4 if dtype == "float32" else 8e-3,
                                    atol=1e-4 if dtype == "float32" else 1e-2)
+
+
+# Operands that are the first rows and columns of larger ones, NaN in every other
+# element: the ring's loads past a slice's last row, and a ragged last tile's past
+# the last column, come from inside the allocation here and must read as zeros.
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("M,K,N", [(150, 136, 200), (300, 96, 584), (40, 1000, 136), (260, 1000, 264)])
+def test_gemm_views_of_larger_operands(dtype, M, K, N):
+    print(f"[case] gemm view {dtype} {M}x{K}x{N}", flush=True)
+    rng = np.random.default_rng(M + K + N)
+    a, b = np.full((M + 400, K + 8), np.nan, np.float32), np.full((K + 1200, N + 264), np.nan, np.float32)
+    a[:M, :K] = rng.standard_normal((M, K))
+    b[:K, :N] = rng.standard_normal((K, N)) / np.sqrt(K)
+    a_s, b_s = on.to_storage(a, dtype), on.to_storage(b, dtype)
+    exp = gemm_ref(on.from_storage(a_s, dtype)[:M, :K], on.from_storage(b_s, dtype)[:K, :N])
+    lib, code = gpu.runtime(), gpu.dtype_code(H.GPU_DTYPES[dtype])
+    a_d, b_d, c_d = H.upload(a_s, dtype), H.upload(b_s, dtype), gpu.allocate((M, N), H.GPU_DTYPES[dtype])
+    ws = gpu.allocate((max(1, lib.tl_gemm_workspace_bytes(M, N, K, code)),), np.uint8)
+    for ptr, size in ((None, 0), (ws.ptr, ws.nbytes)):
+        assert lib.tl_gemm(a_d.ptr, b_d.ptr, c_d.ptr, M, N, K, K + 8, N + 264, N, ptr, size, code, None) == 0
+        got = on.from_storage(H.download(c_d), dtype)
+        np.testing.assert_allclose(got, exp, rtol=1e-4 if dtype == "float32" else 8e-3,
+                                   atol=1e-4 if dtype == "float32" else 1e-2)

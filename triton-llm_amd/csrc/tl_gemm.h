@@ -45,6 +45,14 @@ struct GemmParams {
   int64_t ws_off[kMaxGroups];
 };
 
+// Bytes from a view's first element to the end of its last: what a buffer
+// resource over it may reach.  rows * ld instead would pass the end of the
+// allocation where the view is the last columns of wider rows, and a tile that is
+// only partly inside the view reads there.
+__host__ __device__ __forceinline__ uint32_t view_bytes(int64_t rows, int64_t ld, int64_t cols, int esize) {
+  return rows > 0 ? (uint32_t)(((rows - 1) * ld + cols) * esize) : 0u;
+}
+
 // Work item of workgroup L: each XCD (workgroups are dealt to the 8 XCDs in
 // turn) takes a contiguous run of items, row tiles fastest, so the
 // workgroups an XCD runs at once share their B column tiles and A row tiles

@@ -420,11 +420,12 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_mfma_kernel(GemmParams p) 
   const uint32_t lds0 = (uint32_t)(size_t)lds_base;
   const uint32_t lds_a = lds0, lds_b = lds0 + kGmStages * kGmStageA;
 
-  // Buffer resources over all of A (rows < m) and B (rows < k): rows past
-  // them read as zeros with no memory access.
+  // Buffer resources over all of A (rows < m, its last row to the end of its
+  // last 16-byte chunk: lda is whole chunks) and B (rows < k): rows past them
+  // read as zeros with no memory access.
   const uint32_t lda2 = (uint32_t)(p.lda * T::size), ldb2 = (uint32_t)(pldb * T::size);
-  const i32x4 ra = uniform_rsrc(p.a, (uint32_t)((uint64_t)p.m * lda2));
-  const i32x4 rb = uniform_rsrc(p.G.b[grp], (uint32_t)((uint64_t)p.k * ldb2));
+  const i32x4 ra = uniform_rsrc(p.a, view_bytes(p.m, p.lda, (p.k + 16 / T::size - 1) / (16 / T::size) * (16 / T::size), T::size));
+  const i32x4 rb = uniform_rsrc(p.G.b[grp], view_bytes(p.k, pldb, pn, T::size));
   auto dma = [&](const i32x4& rs, uint32_t voff, uint32_t la) __attribute__((always_inline)) {
     lds_dma16(rs, voff, la);
   };

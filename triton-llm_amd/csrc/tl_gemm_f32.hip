@@ -81,14 +81,14 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmParams p) {
 
   // Loads of a stage.  A: thread -> rows tid / 8 + 32 i, k 4 (tid % 8) .. + 3.
   // B: thread -> rows (tid / 32) + 8 i, columns 4 (tid % 32) .. + 3.  Buffer
-  // resources end at the tile's last row and the slice's last k: zeros past them.
+  // resources end at the tile's last row's and the slice's last k and n: zeros past them.
   constexpr int AI = TM / 32, BI = 4;
   const int rows = min(TM, p.m - m_tile);
   const uint32_t lda4 = (uint32_t)lda * 4, ldb4 = (uint32_t)ldb * 4;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a + (int64_t)m_tile * lda), (short)0, (int)((uint32_t)(rows - 1) * lda4 + (uint32_t)k_hi * 4), kBufRsrcWord3);
+      (void*)(a + (int64_t)m_tile * lda), (short)0, (int)view_bytes(rows, lda, k_hi, 4), kBufRsrcWord3);
   const __amdgpu_buffer_rsrc_t rb =
-      __builtin_amdgcn_make_buffer_rsrc((void*)b, (short)0, (int)((uint32_t)k_hi * ldb4), kBufRsrcWord3);
+      __builtin_amdgcn_make_buffer_rsrc((void*)b, (short)0, (int)view_bytes(k_hi, ldb, pn, 4), kBufRsrcWord3);
   const int a_row = tid >> 3, a_k = 4 * (tid & 7);
   const int b_row = tid >> 5, b_n = 4 * (tid & 31);
   u32x4 av[AI], bv[BI];

@@ -110,12 +110,12 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
   const int k_hi = min(p.k, kt_hi * BK);
   const uint32_t lda2 = (uint32_t)(p.lda * 2), ldb2 = (uint32_t)(p.G.ldb[grp] * 2);
   const int rows = min(TM, p.m - m_tile);
-  // A from this tile's first row, to its last row's k; B to the slice's last row.
+  // A from this tile's first row, to its last row's k; B to the slice's last row's n.
   // The range check covers voff + soff, and what is past it reads as zeros: rows
   // past m, k rows past the slice.  A's chunks past the slice are sent out of range
   // (a_cur below); a stage of zeros adds nothing, so the ring needs no tail.
-  const i32x4 ra = uniform_rsrc((const char*)p.a + (int64_t)m_tile * lda2, (uint32_t)(rows - 1) * lda2 + (uint32_t)p.k * 2);
-  const i32x4 rb = uniform_rsrc(p.G.b[grp], (uint32_t)k_hi * ldb2);
+  const i32x4 ra = uniform_rsrc((const char*)p.a + (int64_t)m_tile * lda2, view_bytes(rows, p.lda, p.k, 2));
+  const i32x4 rb = uniform_rsrc(p.G.b[grp], view_bytes(k_hi, p.G.ldb[grp], pn, 2));
 
   auto b_swz = [](int row) __attribute__((always_inline)) {
     return (BCH % 16 == 0 ? 4 * (row & 3) : 4 * ((row >> 1) & 1)) ^ (2 * ((row >> 3) & 1));
