@@ -579,3 +579,18 @@ def test_gemm_views_of_larger_operands(dtype, M, K, N):
         got = on.from_storage(H.download(c_d), dtype)
         np.testing.assert_allclose(got, exp, rtol=1e-4 if dtype == "float32" else 8e-3,
                                    atol=1e-4 if dtype == "float32" else 1e-2)
+
+
+def test_gemm_one_token_adds_its_waves_by_halves():
+    """The sixteen waves' sums of the whole-K kernel, rows 8 w .. 8 w + 7 each:
+    one of them is 1, the others 0.99 * 2^-24, which a chain that starts at 1
+    would drop one by one (15 * 2^-24 in all).  By halves each of the four levels
+    rounds once, and the first drops one of the small sums."""
+    K, N = 1024, 64
+    b = np.zeros((K, N), np.float32)
+    b[8:128:8] = 0.99 * 2.0 ** -24
+    b[0] = 1.0
+    a = np.ones((1, K), np.float32)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    got = H.download(gemm(gpu.to_device(a), gpu.to_device(b)))
+    assert (np.abs(got - exact) <= 5 * 2.0 ** -24).all(), got[0, 0] - exact[0, 0]

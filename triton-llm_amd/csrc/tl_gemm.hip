@@ -272,10 +272,14 @@ __global__ __launch_bounds__(kWholeThreads) void skinny_whole_kernel(const void*
   __syncthreads();
   for (int idx = tid; idx < MT * COLS; idx += kWholeThreads) {
     const int mi = idx / COLS, col = col0 + idx % COLS;
-    float v = 0.f;
+    float v[WV];
 #pragma unroll
-    for (int q = 0; q < WV; ++q) v += s_sum[q][idx];
-    if (mi < m && col < n) ((Bits*)G.c[grp])[(int64_t)mi * G.ldc[grp] + col] = from_f32<T>(v);
+    for (int q = 0; q < WV; ++q) v[q] = s_sum[q][idx];
+#pragma unroll
+    for (int d = WV / 2; d >= 1; d /= 2)  // by halves: four roundings where a chain has sixteen
+#pragma unroll
+      for (int q = 0; q < d; ++q) v[q] += v[q + d];
+    if (mi < m && col < n) ((Bits*)G.c[grp])[(int64_t)mi * G.ldc[grp] + col] = from_f32<T>(v[0]);
   }
 }
 

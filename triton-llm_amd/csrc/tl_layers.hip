@@ -112,7 +112,8 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_vec_kernel(const void* a
 #pragma unroll
   for (int j = 0; j < CH; ++j)
 #pragma unroll
-    for (int e = 0; e < V; ++e) ss += x[j][e] * x[j][e];
+    for (int e = 0; e < V; e += 4)  // fours, so that no sum is a longer chain than the scalar kernel's
+      ss += (x[j][e] * x[j][e] + x[j][e + 1] * x[j][e + 1]) + (x[j][e + 2] * x[j][e + 2] + x[j][e + 3] * x[j][e + 3]);
   const float rms = sqrtf(block_sum(ss, s_red) / (float)n + eps);
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
