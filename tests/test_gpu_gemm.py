@@ -594,3 +594,24 @@ def test_gemm_one_token_adds_its_waves_by_halves():
     exact = a.astype(np.float64) @ b.astype(np.float64)
     got = H.download(gemm(gpu.to_device(a), gpu.to_device(b)))
     assert (np.abs(got - exact) <= 5 * 2.0 ** -24).all(), got[0, 0] - exact[0, 0]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("M,N", [(1, 520), (2, 960), (2, 1024), (16, 3072), (64, 1024), (100, 1024)])
+def test_gemm_output_over_its_input(dtype, M, N):
+    """C = A in memory, where K is split: every workgroup's operands are read
+    before the reduce pass writes."""
+    print(f"[case] gemm in place {dtype} {M}x{N}", flush=True)
+    rng = np.random.default_rng(M + N)
+    a = on.to_storage(rng.standard_normal((M, N), dtype=np.float32), dtype)
+    b = on.to_storage(rng.standard_normal((N, N), dtype=np.float32) / np.float32(np.sqrt(N)), dtype)
+    lib, code = gpu.runtime(), gpu.dtype_code(H.GPU_DTYPES[dtype])
+    need = lib.tl_gemm_workspace_bytes(M, N, N, code)
+    assert need > 0
+    exp = gemm_ref(on.from_storage(a, dtype), on.from_storage(b, dtype))
+    b_d, ws = H.upload(b, dtype), gpu.allocate((need,), np.uint8)
+    for _ in range(3):
+        a_d = H.upload(a, dtype)
+        assert lib.tl_gemm(a_d.ptr, b_d.ptr, a_d.ptr, M, N, N, N, N, N, ws.ptr, need, code, None) == 0
+        np.testing.assert_allclose(on.from_storage(H.download(a_d), dtype), exp, rtol=1e-4 if dtype == "float32" else 8e-3,
+                                   atol=1e-4 if dtype == "float32" else 1e-2)

@@ -150,6 +150,11 @@ static inline int tl_launch_status() { return (int)hipGetLastError(); }
 // Resolve the stream argument of an entry point: NULL means the library stream.
 hipStream_t tl_resolve_stream(void* stream);
 
+// Whether [a, a + na) and [b, b + nb) share a byte.
+static inline bool tl_overlap(const void* a, size_t na, const void* b, size_t nb) {
+  return (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 // Fill nbytes at dst with value on stream st by a kernel (capturable in a
 // HIP graph as a kernel node).
 int tl_fill_bytes(void* dst, unsigned char value, size_t nbytes, hipStream_t st);

@@ -308,8 +308,8 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
 }
 
 template <typename T>
-int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* ws, hipStream_t st) {
-  if (m <= 2 && k <= kWholeMaxK) {
+int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* ws, bool in_place, hipStream_t st) {
+  if (m <= 2 && k <= kWholeMaxK && !in_place) {
     constexpr int cols = kWholeChunks * (16 / T::size);
     int64_t tiles = 0;
     for (int g = 0; g < G.count; ++g) tiles += (G.n[g] + cols - 1) / cols;
@@ -796,9 +796,22 @@ bool wide_ok(const GemmGroups& G, int k, int64_t lda) {
   return ok;
 }
 
+// Whether an output shares bytes with A or with a B.  Such a product comes out
+// right where K is cut: every operand is read before the reduce pass writes the
+// first output.  So it is cut where the workspace allows.
+bool writes_inputs(const void* a, const GemmGroups& G, int m, int k, int64_t lda, int esize) {
+  for (int g = 0; g < G.count; ++g) {
+    const size_t nc = ((m - 1) * G.ldc[g] + G.n[g]) * esize;
+    if (tl_overlap(G.c[g], nc, a, ((m - 1) * lda + k) * esize)) return true;
+    for (int h = 0; h < G.count; ++h)
+      if (tl_overlap(G.c[g], nc, G.b[h], ((k - 1) * G.ldb[h] + G.n[h]) * esize)) return true;
+  }
+  return false;
+}
+
 template <typename T>
 int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, void* workspace,
-                size_t workspace_bytes, hipStream_t st) {
+                size_t workspace_bytes, bool in_place, hipStream_t st) {
   GemmParams p{};
   p.a = a;
   p.m = m;
@@ -822,6 +835,7 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
     // as many K-slices as the workspace query's answer holds, where it was given
     const SplitCap cap = split_cap(m, k, G, (int)esize);
     const int max_split = workspace && workspace_bytes >= cap.ws_bytes && ((uintptr_t)workspace % 16) == 0 ? cap.ksplit : 1;
+    const int min_split = in_place && max_split > 1 ? 2 : 1;
     // tiles of tm x tn, K in ksplit slices of kt_per stages, run columns a store
     auto place = [&](int tm, int tn, int ksplit, int kt_per, int run) {
       p.tiles_m = (m + tm - 1) / tm;
@@ -841,11 +855,11 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
     };
     int e;
     if (T::size == 4 && k % 4 == 0) {
-      const F32Plan W = gemm_f32_plan(m, k, G, max_split);
+      const F32Plan W = gemm_f32_plan(m, k, G, min_split, max_split);
       place(W.tm, kGmTile, W.ksplit, W.kt_per, 4);
       e = launch_gemm_f32(p, W.tm, st);
     } else if (T::size == 2 && wide_ok(G, k, lda)) {
-      const WidePlan W = gemm_wide_plan(m, k, G, max_split);
+      const WidePlan W = gemm_wide_plan(m, k, G, min_split, max_split);
       place(W.tm, W.tn, W.ksplit, W.kt_per, W.ksplit > 1 ? 4 : 8);  // the reduce stores 4 columns, the kernel 8
       e = launch_gemm_wide(p, W, (int)T::code, st);
     } else {
@@ -927,6 +941,7 @@ int gemm_groups(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
     }
     return 0;
   }
+  const bool in_place = writes_inputs(a, live, m, k, lda, (int)esize);
   if (m <= kSkinnyMaxM) {
     bool ok = true;
     const int cpc = 16 / (int)esize;
@@ -937,16 +952,16 @@ int gemm_groups(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
       const size_t need = skinny_workspace_bytes(m, live, k, (int)esize);
       if (need && (!workspace || workspace_bytes < need)) return TL_ERR_INVALID;
       switch (dtype) {
-        case TL_DTYPE_F32: return launch_skinny<F32>(a, live, m, k, lda, workspace, st);
-        case TL_DTYPE_F16: return launch_skinny<F16>(a, live, m, k, lda, workspace, st);
-        default: return launch_skinny<BF16>(a, live, m, k, lda, workspace, st);
+        case TL_DTYPE_F32: return launch_skinny<F32>(a, live, m, k, lda, workspace, in_place, st);
+        case TL_DTYPE_F16: return launch_skinny<F16>(a, live, m, k, lda, workspace, in_place, st);
+        default: return launch_skinny<BF16>(a, live, m, k, lda, workspace, in_place, st);
       }
     }
   }
   switch (dtype) {
-    case TL_DTYPE_F32: return launch_gemm<F32>(a, live, m, k, lda, workspace, workspace_bytes, st);
-    case TL_DTYPE_F16: return launch_gemm<F16>(a, live, m, k, lda, workspace, workspace_bytes, st);
-    default: return launch_gemm<BF16>(a, live, m, k, lda, workspace, workspace_bytes, st);
+    case TL_DTYPE_F32: return launch_gemm<F32>(a, live, m, k, lda, workspace, workspace_bytes, in_place, st);
+    case TL_DTYPE_F16: return launch_gemm<F16>(a, live, m, k, lda, workspace, workspace_bytes, in_place, st);
+    default: return launch_gemm<BF16>(a, live, m, k, lda, workspace, workspace_bytes, in_place, st);
   }
 }
 

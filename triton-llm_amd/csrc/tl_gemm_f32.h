@@ -11,8 +11,8 @@ struct F32Plan {
   double us;
 };
 
-// The plan of the least modelled time with at most max_split K-slices.
-F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int max_split);
+// The plan of the least modelled time with min_split to max_split K-slices.
+F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int min_split, int max_split);
 
 // p's tiles are tm x 128 (tm 128 or 64), its stages 32 k.
 int launch_gemm_f32(const GemmParams& p, int tm, hipStream_t st);

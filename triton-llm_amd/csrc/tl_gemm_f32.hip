@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmParams p) {
 
 }  // namespace
 
-F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int max_split) {
+F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int min_split, int max_split) {
   F32Plan best{};
   const int cus = tl_device_cus();
   const int stages = (k + kBk - 1) / kBk;
@@ -294,7 +294,7 @@ F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int max_split) {
   for (const F32Tile& c : kF32Tiles) {
     int64_t tiles = 0;
     for (int g = 0; g < G.count; ++g) tiles += (int64_t)((m + c.tm - 1) / c.tm) * ((G.n[g] + 127) / 128);
-    for (int S = 1; S <= max_split && (S == 1 || stages >= 4 * S); ++S) {
+    for (int S = min_split; S <= max_split && (S == min_split || stages >= 4 * S); ++S) {
       const int64_t per_cu = (tiles * S + cus - 1) / cus;
       const int rest = (int)(per_cu % c.at_once);
       const double stage = (double)(per_cu / c.at_once) * c.stage_us[c.at_once - 1] + (rest ? c.stage_us[rest - 1] : 0.0);

@@ -13,9 +13,9 @@ struct WidePlan {
   int ksplit, kt_per;  // K-slices, and 32-k stages of one
 };
 
-// The tile and K split (at most max_split slices) of the least modelled time:
+// The tile and K split (min_split to max_split slices) of the least modelled time:
 // rounds of one tile a CU, plus the reduce pass over the fp32 partials of a split.
-WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int max_split);
+WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int min_split, int max_split);
 
 // p's tiles, split and items are w's; p.vec_store marks the groups whose rows
 // take 16-byte stores (the reduce's own runs when K is split).

@@ -310,7 +310,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
 
 }  // namespace
 
-WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int max_split) {
+WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int min_split, int max_split) {
   WidePlan best{};
   const int cus = tl_device_cus();
   const int stages = (k + 31) / 32;
@@ -320,7 +320,7 @@ WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int max_split) {
   for (WidePlan c : kWidePlans) {
     int64_t tiles = 0;
     for (int g = 0; g < G.count; ++g) tiles += (int64_t)((m + c.tm - 1) / c.tm) * ((G.n[g] + c.tn - 1) / c.tn);
-    for (int S = 1; S <= max_split && (S == 1 || stages >= 4 * S); ++S) {
+    for (int S = min_split; S <= max_split && (S == min_split || stages >= 4 * S); ++S) {
       c.ksplit = S;
       c.kt_per = (stages + S - 1) / S;
       const double reduce = S > 1 ? (8.0 * S + 2) * m * (double)ncols / 5.0e6 + 4.0 : 0.0;
