@@ -115,8 +115,9 @@ int tl_rope_inplace(void* x, const float* cos_table, const float* sin_table,
  * in fp32 instead of pre-scaling Q, whose fp16 copy could overflow.
  * Workspace: tl_attention_fwd_workspace_bytes
  * (room for a key-major copy of V on the 16-bit MFMA path at d_k 128, made
- * where V's rows overlap or on request, read in place otherwise; 0 for d_k 64
- * and fp32; NULL is accepted when 0).
+ * where V's rows overlap, where o lies over v or on request, read in place
+ * otherwise; 0 for d_k 64 and fp32; NULL is accepted when 0).  o may not
+ * overlap q or k, nor v but for that 16-bit path at d_k 128.
  * A 16-byte-aligned workspace of tl_attention_fwd_workspace_bytes_split
  * bytes (at least the above) also lets a causal 16-bit MFMA call with
  * seq_k >= seq_q and few query tiles split the key range of its costliest

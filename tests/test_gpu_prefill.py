@@ -100,7 +100,7 @@ def test_prefill_ragged_shapes(d128_kernel, dtype, d_k, causal):
 @pytest.mark.parametrize("sq,sk", [(1, 1), (1, 300), (37, 300), (130, 129), (64, 64), (5, 3), (300, 700)])
 def test_prefill_seq_q_ne_seq_k(d128_kernel, sq, sk, d_k):
     """Bottom-right causal alignment; sq > sk leaves the first rows fully masked (NaN).
-    d_k 64 reads V in place, d_k 128 through its V^T copy."""
+    V in place, and at d_k 128 through its V^T copy too (flash_fwd_w64)."""
     skip_w64_repeat(d128_kernel, d_k)
     dt = "bfloat16"
     rng = np.random.default_rng(sq * 1000 + sk + d_k)
@@ -352,3 +352,21 @@ def test_prefill_v_row_strides(v_ss, causal):
     got = on.from_storage(H.download(o_d), dt)
     exp = oa.attention_bhsd(*(on.from_storage(x, dt) for x in (q, k, v)), causal=causal, dtype="float32")
     compare(f"v_ss {v_ss}", got, exp, TOL[dt])
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_prefill_output_over_v(dtype, causal):
+    """O written into V's own memory (one KV head per query head, d_k 128): V is
+    copied before the first store.  Many tiles, so that some start after others
+    have stored."""
+    rng = np.random.default_rng(31)
+    shape = (2, 16, 2300, 128)
+    q, k, v = (on.to_storage(rng.standard_normal(shape, dtype=np.float32), dtype) for _ in range(3))
+    qd, kd = H.upload(q, dtype), H.upload(k, dtype)
+    apart = H.download(flash_attention(qd, kd, H.upload(v, dtype), causal=causal))
+    for _ in range(2):
+        vd = H.upload(v, dtype)
+        flash_attention(qd, kd, vd, causal=causal, out=vd)
+        got = on.from_storage(H.download(vd), dtype)
+        compare(f"over v {dtype}", got, on.from_storage(apart, dtype), TOL[dtype])

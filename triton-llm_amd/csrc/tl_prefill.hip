@@ -30,7 +30,7 @@
 // block) and the V^T operand is read with the matching key permutation.
 //
 // Kernels: flash_fwd_16 (f16 / bf16, d_k 64 / 128; V in place, or copied by
-// vt_pack_kernel where its rows overlap), flash_fwd_f32 and flash_fwd_f32_ks
+// vt_pack_kernel where its rows overlap or O is written over it), flash_fwd_f32 and flash_fwd_f32_ks
 // (fp32, d_k 64 / 128), attn_generic_kernel (the other head sizes).
 #include "tl_prefill.h"
 
@@ -1587,6 +1587,14 @@ bool v_rows_ok(const FlashParams& p, int d_k) {
   return p.v_ss >= d_k && (128 * p.v_ss + d_k) * 2 < ((int64_t)1 << 32);
 }
 
+// Whether O's rows touch V's, over the whole span of either: a V in place is read
+// by every workgroup until the last is done, its copy only before the first store.
+bool o_on_v(const FlashParams& p, int d_k) {
+  const size_t v = ((p.batch - 1) * p.v_sb + (p.n_kv - 1) * p.v_sh + (p.seq_k - 1) * p.v_ss + d_k) * 2;
+  const size_t o = ((p.batch - 1) * p.o_sb + (p.n_head - 1) * p.o_sh + (p.seq_q - 1) * p.o_ss + d_k) * 2;
+  return tl_overlap(p.v, v, p.o, o);
+}
+
 template <typename T, int D, bool SCALE_S>
 int launch_flash_16_as(const FlashParams& p, bool causal, bool vnat, hipStream_t st) {
   const dim3 grid((unsigned)(p.q_machines * p.n_queues)), block(K16_THREADS);
@@ -1615,8 +1623,9 @@ int launch_flash_16(FlashParams& p, void* ws, size_t ws_bytes, bool causal, hipS
   // large scale); it addresses a wave's 64 output rows with 32-bit offsets.
   const bool w64 = D == 128 && !scale_s && tl_overrides.prefill_w64 && (64 * p.o_ss + D) * 2 < ((int64_t)1 << 32);
   // V in place, unless its rows overlap or a tile of them passes 32-bit offsets
-  // (d_k 64 takes no such V: mfma_shape_ok) -- those are copied, as for flash_fwd_w64
-  const bool vnat = D == 64 || (!w64 && v_rows_ok(p, D));
+  // (d_k 64 takes no such V: mfma_shape_ok) or O is written over it -- those are
+  // copied, as for flash_fwd_w64
+  const bool vnat = D == 64 || (!w64 && v_rows_ok(p, D) && !o_on_v(p, D));
   // the copy's room is part of the workspace either way (the split region follows it)
   const size_t vt_need = D == 64 ? 0 : vt_bytes(p.batch, p.n_kv, p.seq_k, D);
   const size_t room = ws && aligned16(ws) && ws_bytes > align256(vt_need) ? ws_bytes - align256(vt_need) : 0;
@@ -1700,7 +1709,8 @@ extern "C" {
 size_t tl_attention_fwd_workspace_bytes(int batch, int n_kv_head, int seq_k, int d_k,
                                         int dtype) {
   // 16-bit MFMA path at d_k 128: room for the permuted key-major V^T copy that a
-  // V of overlapping rows and flash_fwd_w64 take.  The others read V in place.
+  // V of overlapping rows, one that O is written over and flash_fwd_w64 take (the
+  // query knows neither strides nor pointers).  The others read V in place.
   if (dtype == TL_DTYPE_F32 || batch <= 0 || n_kv_head <= 0 || seq_k <= 0 || d_k != 128)
     return 0;
   return vt_bytes(batch, n_kv_head, seq_k, d_k);
