@@ -19,6 +19,7 @@ of the reference's ``_sample`` (oracle/sample.py).
 """
 
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -326,3 +327,55 @@ def test_top_k_by_groups(dtype, V):
             exp = int(np.argmax(c > u[r] * c[-1]))
             near = abs(c[got[r]] - u[r] * c[-1]) < 1e-5 * c[-1] or abs((c[got[r]] - p[got[r]]) - u[r] * c[-1]) < 1e-5 * c[-1]
             assert p[got[r]] > 0 and (got[r] == exp or near), (r, got[r], exp)
+
+
+# Rows whose largest entries lie together, as a vocabulary ordered by frequency or
+# a constrained decoder's mask makes them: few groups with thousands of candidates
+# (more than the finish holds in LDS), and fewer finite entries than top_k.
+def _clustered(rng, what, rows, V):
+    x = (3 * rng.standard_normal((rows, V))).astype(np.float32)
+    if what == "sorted":
+        return -np.sort(-x, axis=1)
+    if what == "ties":
+        return -np.sort(-np.round(x), axis=1)
+    keep = {"10 finite": 10, "half finite": V // 2}[what]
+    y = np.full_like(x, -np.inf)
+    y[:, :keep] = x[:, :keep]
+    return y
+
+
+@pytest.mark.parametrize("what", ["sorted", "ties", "10 finite", "half finite"])
+@pytest.mark.parametrize("V,top_k", [(16384, 50), (128256, 50), (128256, 500), (128256, 1002), (262144, 2048)])
+def test_top_k_of_clustered_rows(what, V, top_k):
+    print(f"[case] sample clustered {what} V={V} top_k={top_k}", flush=True)
+    rng = np.random.default_rng(V + top_k)
+    x, u = _clustered(rng, what, 4, V), rng.random(4)
+    got = H.download(sample_rows(gpu.to_device(x), 0.7, top_k, uniforms=gpu.to_device(u)))
+    for r in range(4):
+        kth = np.sort(x[r])[::-1][top_k - 1]
+        z = (x[r] / np.float32(0.7)).astype(np.float32)
+        p = np.where(x[r] >= kth, np.exp((z - z.max()).astype(np.float32)).astype(np.float64), 0.0)
+        c = np.cumsum(p)
+        lo, t = c[got[r]] - p[got[r]], u[r] * c[-1]
+        assert p[got[r]] > 0 and lo - 1e-5 * c[-1] <= t <= c[got[r]] + 1e-5 * c[-1], (r, got[r])
+
+
+def test_masked_rows_cost_what_others_do():
+    """A row of ten finite logits was walked up to 32 times by one workgroup (55
+    times a plain row's time at this size): it may take a few times as long at most."""
+    rng = np.random.default_rng(3)
+    u, tok = gpu.to_device(rng.random(64)), gpu.allocate((64,), np.int32)
+    took = []
+    for what in (None, "10 finite"):
+        x = gpu.to_device((3 * rng.standard_normal((64, 49152))).astype(np.float32) if what is None
+                          else _clustered(rng, what, 64, 49152))
+        best = 1e9
+        for _ in range(6):
+            gpu.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                sample_rows(x, 0.8, 50, uniforms=u, out_dev=tok)
+            gpu.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        took.append(best)
+    assert took[1] < 8 * took[0], took
