@@ -21,7 +21,7 @@
 //   * every segment records its maximum and first index;
 //   * without top_k it also records its mass at its own maximum,
 //     sum exp(x / T - m_seg / T) (fp64);
-//   * with top_k up to half the row's 64-entry groups it records each group's
+//   * with top_k up to 15/16 of the row's 64-entry groups it records each group's
 //     maximum (below);
 //   * with a larger top_k it keeps its own top_k (every entry >= its k-th largest, by
 //     a radix select on an order-preserving 32-bit key, 8 bits per step,
@@ -38,11 +38,11 @@
 //     row's k-th largest entry (top_k groups hold one that large), so only the
 //     groups that reach it are read again, and their entries that reach it, about
 //     top_k of them, are the candidates, in index order.  Where they are thousands
-//     (the largest entries all in a few groups) the listed groups are walked
-//     instead.  64 rows, top_k 50 / 500, against the select in every segment: 128256
-//     normal logits 57.6 / 515.6 -> 21.4 / 59.4 us, the same sorted 82.4 / 416 ->
-//     28.2 / 181, all but ten -inf 2435 / 2433 -> 22.2 / 22.2; one row of 49152
-//     sorted, top_k 50, 22.4 -> 23.9;
+//     (the largest entries all in a few groups) the select walks the listed groups
+//     and what it keeps is staged after it.  64 rows, top_k 50 / 500, against the
+//     select in every segment: 128256 normal logits 57.6 / 518 -> 21.3 / 60 us, the
+//     same sorted 82 / 418 -> 28 / 138, all but ten -inf 2435 -> 22.4; sorted rows of
+//     49152 can lose (one row, top_k 192, 40 -> 50 us; 706, 177 -> 190);
 //   * with top_k otherwise: the k-th largest candidate (radix select; candidates staged
 //     in LDS when they fit), then the inverse CDF over the kept candidates.
 // Every scan gives thread t the interval [lo_t, hi_t) of cumulative mass with
@@ -82,9 +82,11 @@ struct Ws {
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 int n_segments(int vocab) { return (vocab + kSeg - 1) / kSeg; }
 __host__ __device__ __forceinline__ int n_groups(int vocab) { return (vocab + kGrp - 1) / kGrp; }
-// Beyond half the groups the k-th group maximum excludes too little, and above
-// all of them nothing.
-__host__ __device__ __forceinline__ bool by_groups(int vocab, int top_k) { return 2 * top_k <= n_groups(vocab); }
+// The nearer top_k comes to the number of groups, the less the k-th group maximum
+// excludes: at 15/16 of them 64 rows take 72 us against 248 with the select in
+// every segment (49152 entries), 180 against 1824 (128256), 15.1 against 16.0
+// (2048); with as many as there are groups 2048 entries lose (16.1 against 15.8).
+__host__ __device__ __forceinline__ bool by_groups(int vocab, int top_k) { return 16 * top_k <= 15 * n_groups(vocab); }
 
 // Workspace layout; base == nullptr only sizes it.
 size_t ws_layout(int rows, int vocab, char* base, Ws* ws) {
@@ -578,7 +580,7 @@ __global__ __launch_bounds__(kBT) void finish_kernel(const void* logits, int64_t
       if (key[j] != 0u && key[j] >= bound) s.group[pos++] = (unsigned short)(tid * per + j);
     __syncthreads();
     // Each wave takes a run of the list, a group a load, kFly loads in flight:
-    // first how many entries reach the bound, then (if they fit) their places.
+    // first how many entries reach thr, then (if they fit) their places.
     constexpr int kFly = 16;
     const int chunk = (n_sel + kBW - 1) / kBW;
     const int b0 = min(n_sel, wave * chunk), b1 = min(n_sel, b0 + chunk);
@@ -595,7 +597,7 @@ __global__ __launch_bounds__(kBT) void finish_kernel(const void* logits, int64_t
         }
 #pragma unroll
         for (int q = 0; q < kFly; ++q) {
-          const bool in = v[q] > -INFINITY && order_key(v[q]) >= bound;
+          const bool in = v[q] > -INFINITY && order_key(v[q]) >= thr;
           const unsigned long long m = __ballot(in);
           if (write && in) {
             const int at = base + __popcll(m & ((1ull << lane) - 1));
@@ -606,38 +608,48 @@ __global__ __launch_bounds__(kBT) void finish_kernel(const void* logits, int64_t
         }
       }
     };
-    walk(false);
-    if (lane == 0) s.a[wave] = base;
-    __syncthreads();
-    C = 0;
-    base = 0;
-#pragma unroll
-    for (int w = 0; w < kBW; ++w) {
-      if (w < wave) base += s.a[w];
-      C += s.a[w];
-    }
-    staged = C <= kLdsCand;  // else thousands of them in few groups, or ties with the bound
-    const bool select = C > top_k;
-    if (staged) walk(true);
-    else C = n_sel * kGrp;
-    __syncthreads();
     thr = bound;
-    if (select)
+    for (bool exact = false;; exact = true) {
+      base = 0;
+      walk(false);
+      __syncthreads();  // earlier readers of s.a are done
+      if (lane == 0) s.a[wave] = base;
+      __syncthreads();
+      C = 0;
+      base = 0;
+#pragma unroll
+      for (int w = 0; w < kBW; ++w) {
+        if (w < wave) base += s.a[w];
+        C += s.a[w];
+      }
+      staged = C <= kLdsCand;
+      if (staged) {
+        walk(true);
+        __syncthreads();
+        if (!exact && C > top_k)
+          thr = kth_key(
+              [&](auto&& fn) {
+                for (int f = tid; f < C; f += kBT) fn(order_key(s.cx[f]));
+              },
+              (unsigned)top_k, bound, top, s);
+        break;
+      }
+      // thousands in few groups: select among the listed entries and stage what is
+      // kept; thousands that tie with the last one kept stay where they are
+      C = n_sel * kGrp;
+      if (exact) break;
       thr = kth_key(
           [&](auto&& fn) {
-            if (staged) {
-              for (int f = tid; f < C; f += kBT) fn(order_key(s.cx[f]));
-            } else {
-              for (int f0 = tid; f0 < C; f0 += kFly * kBT) {
+            for (int f0 = tid; f0 < C; f0 += kFly * kBT) {
 #pragma unroll
-                for (int q = 0; q < kFly; ++q) v[q] = f0 + q * kBT < C ? group_x(in_groups(f0 + q * kBT)) : -INFINITY;
+              for (int q = 0; q < kFly; ++q) v[q] = f0 + q * kBT < C ? group_x(in_groups(f0 + q * kBT)) : -INFINITY;
 #pragma unroll
-                for (int q = 0; q < kFly; ++q)
-                  if (v[q] > -INFINITY) fn(order_key(v[q]));
-              }
+              for (int q = 0; q < kFly; ++q)
+                if (v[q] > -INFINITY) fn(order_key(v[q]));
             }
           },
           (unsigned)top_k, bound, top, s);
+    }
   } else {
     // the candidates of all segments, in index order
     if (wave == 0) {
