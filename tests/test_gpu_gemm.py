@@ -615,3 +615,54 @@ def test_gemm_output_over_its_input(dtype, M, N):
         assert lib.tl_gemm(a_d.ptr, b_d.ptr, a_d.ptr, M, N, N, N, N, N, ws.ptr, need, code, None) == 0
         np.testing.assert_allclose(on.from_storage(H.download(a_d), dtype), exp, rtol=1e-4 if dtype == "float32" else 8e-3,
                                    atol=1e-4 if dtype == "float32" else 1e-2)
+
+
+# fp32 products whose parts do not cover an operand, on both tile heights, whole,
+# with K in slices (the outlier in one of them) and in a group, rows of C that take
+# vector and scalar stores: the tile comes from the fp32 MFMA, its rows and
+# columns without an outlier unchanged in value.  Bound as for the parts.
+@pytest.mark.parametrize("M,K,Ns,cus", [(150, 96, (200,), 256), (200, 1000, (196,), 4), (128, 68, (128, 40), 1),
+                                        (300, 2560, (264,), 256)])
+@pytest.mark.parametrize("what", ["nan", "inf", "huge", "tiny row", "tiny column", "tiny entries"])
+def test_gemm_fp32_outliers(monkeypatch, M, K, Ns, cus, what):
+    print(f"[case] gemm fp32 outliers {what} {M}x{K} -> {Ns} cus {cus}", flush=True)
+    H.set_override(monkeypatch, "TRITON_LLM_HIP_MAX_CUS", cus)
+    rng = np.random.default_rng(M + K)
+    a = rng.standard_normal((M, K), dtype=np.float32)
+    bs = [rng.standard_normal((K, n), dtype=np.float32) for n in Ns]
+    if what == "nan":
+        a[M // 2, K - 1], bs[0][0, 3] = np.nan, np.nan
+    elif what == "inf":
+        a[3, K - 1] = np.inf
+        bs[0][K - 1, ::2] = 0.0
+    elif what == "huge":
+        a[M - 1, K // 2] = 1e30
+        bs[0][K // 2] = 1e-3
+    elif what == "tiny row":
+        a[5] *= np.float32(1e-20)
+    elif what == "tiny column":
+        bs[0][:, 7] *= np.float32(1e-20)
+    else:  # below 2^-102 beside ones, against columns that are zero where the ones are
+        a[9, : K // 2] *= np.float32(1e-33)
+        bs[0][K // 2:, : Ns[0] // 2] = 0.0
+    lib, n_g = gpu.runtime(), len(Ns)
+    a_d, b_d = gpu.to_device(a), [gpu.to_device(b) for b in bs]
+    ns = (ctypes.c_int * n_g)(*Ns)
+    ws = gpu.allocate((max(1, lib.tl_gemm_grouped_workspace_bytes(M, K, n_g, ns, 0)),), np.uint8)
+    for extra in (0, 1):
+        c_d = [gpu.to_device(np.full((M, n + extra), 3.0, np.float32)) for n in Ns]
+        st = lib.tl_gemm_grouped(a_d.ptr, M, K, K, n_g, (ctypes.c_void_p * n_g)(*[b.data_ptr() for b in b_d]),
+                                 (ctypes.c_void_p * n_g)(*[c.data_ptr() for c in c_d]), ns,
+                                 (ctypes.c_int64 * n_g)(*Ns), (ctypes.c_int64 * n_g)(*[n + extra for n in Ns]),
+                                 ws.ptr, ws.nbytes, 0, None)
+        assert st == 0
+        for b, c, n in zip(bs, c_d, Ns):
+            got = H.download(c)
+            assert (got[:, n:] == 3.0).all()
+            with np.errstate(all="ignore"):
+                exact = a.astype(np.float64) @ b.astype(np.float64)
+                bound = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+            ok = np.isfinite(exact)
+            np.testing.assert_array_equal(np.isnan(got[:, :n]), np.isnan(exact))
+            np.testing.assert_array_equal(got[:, :n][np.isinf(exact)], exact[np.isinf(exact)].astype(np.float32))
+            assert (np.abs(got[:, :n][ok] - exact[ok]) <= (K + 4) * 2.0 ** -24 * bound[ok] + 1e-44).all()

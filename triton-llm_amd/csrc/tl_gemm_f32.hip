@@ -34,9 +34,23 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& h, uint32_t
   l = pack2<BF16>(s);
 }
 
+// The wave's largest value, with no LDS: by rows of 16 lanes, then the four rows'.
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, dpp_mov<0xB1>(x));   // quad_perm [1,0,3,2]
+  x = fmaxf(x, dpp_mov<0x4E>(x));   // quad_perm [2,3,0,1]
+  x = fmaxf(x, dpp_mov<0x141>(x));  // row_half_mirror
+  x = fmaxf(x, dpp_mov<0x140>(x));  // row_mirror
+  float r[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __uint_as_float(__builtin_amdgcn_readlane((int)__float_as_uint(x), 16 * i));
+  return fmaxf(fmaxf(r[0], r[1]), fmaxf(r[2], r[3]));
+}
+
 // Workgroup tile 32 MB x 128 of C, four waves of 16 MB x 64.  Each fp32 operand is
-// the exact sum of three bf16 parts, and a product is six 16x16x32 bf16 MFMAs
-// (2.5 PFLOP/s / 6) where the fp32 MFMA's peak is 157 TFLOP/s.  A stage's fp32
+// the exact sum of three bf16 parts (Henry, Tang, Heinecke: Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations, ARITH 2019),
+// and a product is six 16x16x32 bf16 MFMAs (2.5 PFLOP/s / 6) where the fp32 MFMA's
+// peak is 157 TFLOP/s.  A stage's fp32
 // values are loaded to registers two stages ahead, split there once per workgroup
 // while the current stage's MFMAs run, and stored as three bf16 planes in one LDS
 // buffer (48 or 36 KiB: two or three workgroups a CU cover each other's
@@ -55,11 +69,11 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& h, uint32_t
 // workgroups a CU is the issue port (about 240 VALU instructions, 96 MFMAs and 49
 // LDS ones per wave and stage); a lone one waits on its own LDS reads.
 template <int MB>
-__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmParams p) {
+__global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmParams p) {
   constexpr int TM = 32 * MB, TN = 128, NB = 4;
   constexpr int SA = TM * 64, SB = kBk * 256;  // bytes of one plane of a stage
   __shared__ __attribute__((aligned(1024))) char smem[3 * (SA + SB)];
-  __shared__ float s_row[TM], s_col[8][TN];
+  __shared__ float s_row[TM], s_col[8][TN], s_max[4], s_least[4];
 
   int grp, tm, tn, ks;
   if (!gemm_tile_panels(p, grp, tm, tn, ks)) return;
@@ -185,8 +199,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmParams p) {
     }
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    // The small products first, into sums of their own; a part of a times b's two
-    // parts below it (2^-27 of the product and less) is left out.
+    // The small products first, into sums of their own; the middle part times the
+    // smallest, either way, and the smallest times itself are left out: up to 2^-24.2
+    // of the product, 2^-27 in the root mean square.
     constexpr int PA[5] = {0, 2, 1, 0, 1}, PB[5] = {2, 0, 1, 1, 0};
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -215,45 +230,124 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmParams p) {
     }
   }
 
-  // The parts stand for every fp32 value between 2^-102 and 2^127; a row of A or a
-  // column of B whose largest magnitude is not between 2^-40 and 2^60 (NaN and
-  // infinity included; all zeros are fine) sends the tile through plain fp32.
+  // From here on lane values are made again: none of them is kept through the loop.
+  int tid_e = (int)threadIdx.x;
+  asm volatile("" : "+v"(tid_e));
+  const int wave_e = __builtin_amdgcn_readfirstlane(tid_e >> 6);
+  const int lc_e = tid_e & 15, g_e = (tid_e >> 4) & 3;
+  const int m_e = 16 * MB * (wave_e & 1), n_e = 64 * (wave_e >> 1);  // the wave's corner in the tile
+  const int a_row_e = tid_e >> 3, b_row_e = tid_e >> 5, b_n_e = 4 * (tid_e & 31);
+
+  // The parts stand for every fp32 value between 2^-102 and 2^127.  Two things send
+  // the tile through the fp32 MFMA: a row of A or a column of B whose largest
+  // magnitude is not between 2^-40 and 2^60 (NaN and infinity included; all zeros are
+  // fine), and a sum below 2^-44 of its row's largest times its column's, which may
+  // be made of entries below 2^-102 alone (above it they weigh k 2^-42 at most).  The
+  // look at the sums costs 0.5 us a product, 1.4% of a SmolLM2-360M layer; one at
+  // every entry as it is split costs more.
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
     float v = a_max[i];
 #pragma unroll
     for (int o = 4; o >= 1; o >>= 1) v = __builtin_elementwise_maximum(v, __shfl_xor(v, o));
-    if ((tid & 7) == 0) s_row[a_row + 32 * i] = v;
+    if ((tid_e & 7) == 0) s_row[a_row_e + 32 * i] = v;
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) s_col[b_row][b_n + e] = b_max[e];
+  for (int e = 0; e < 4; ++e) s_col[b_row_e][b_n_e + e] = b_max[e];
+  // The tile's smallest sum against its largest row's and column's magnitudes; the
+  // sums one by one only where that falls short.
+  float least = INFINITY;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const f32x4 c = acc[mb][nb];
+      const bool inside = m_tile + m_e + 16 * mb + lc_e < p.m && n_tile + n_e + 16 * nb + 4 * g_e < pn;
+      least = fminf(least, inside ? fminf(fminf(fabsf(c[0]), fabsf(c[1])), fminf(fabsf(c[2]), fabsf(c[3]))) : INFINITY);
+    }
   __syncthreads();
-  float v = 1.f;
-  if (tid < TM) {
-    v = s_row[tid];
-  } else if (tid >= 128 && n_tile + tid - 128 < pn) {  // columns past n hold the next row's values
-    v = s_col[0][tid - 128];
+  float v = 0.f;  // waves 0 and 1: a row's largest magnitude, 2 and 3: a column's
+  if (tid_e < TM) {
+    v = s_row[tid_e];
+  } else if (tid_e >= 128) {
+    v = s_col[0][tid_e - 128];
 #pragma unroll
-    for (int i = 1; i < 8; ++i) v = __builtin_elementwise_maximum(v, s_col[i][tid - 128]);
+    for (int i = 1; i < 8; ++i) v = __builtin_elementwise_maximum(v, s_col[i][tid_e - 128]);
+    if (n_tile + tid_e - 128 >= pn) v = 0.f;  // columns past n hold the next row's values
+    s_col[0][tid_e - 128] = v;
   }
-  const bool plain = __syncthreads_or(!(v == 0.f || (v >= 0x1p-40f && v <= 0x1p60f)));
+  const bool in_range = __all(v == 0.f || (v >= 0x1p-40f && v <= 0x1p60f));
+  v = wave_max(v);
+  least = -wave_max(-least);
+  if ((tid_e & 63) == 0) {
+    s_max[wave_e] = in_range ? v : INFINITY;
+    s_least[wave_e] = least;
+  }
+  __syncthreads();
+  const float most = fmaxf(s_max[0], s_max[1]) * 0x1p-44f * fmaxf(s_max[2], s_max[3]);
+  bool plain = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3])) == INFINITY;
+  if (!plain && fminf(fminf(s_least[0], s_least[1]), fminf(s_least[2], s_least[3])) < most) {
+    float short_of = 0.f;  // by how much a sum falls short of its bound, at most
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const float row = s_row[m_e + 16 * mb + lc_e] * 0x1p-44f;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)  // 0 past n, and past m
+          short_of = fmaxf(short_of, fmaf(row, s_col[0][n_e + 16 * nb + 4 * g_e + e], -fabsf(acc[mb][nb][e])));
+    }
+    plain = __syncthreads_or(short_of > 0.f);
+  }
 
-  const int mw = m_tile + 16 * MB * wm, nw = n_tile + 64 * wn;
+  const int mw = m_tile + m_e, nw = n_tile + n_e;
   if (plain) {
+    // Once more, on 16x16x4 fp32 MFMAs: rows of A of 128 bytes, chunk c of row r at
+    // slot c ^ ((r >> 1) & 7); rows of B of 512 bytes, chunk c of row r at slot c ^
+    // 4 ((r >> 2) & 3).  Step t of a 16-k half takes k = 4 g + t, so that one 16-byte
+    // read of A serves four steps.  2048 x 3072 x 3072, with one NaN, a row times
+    // 1e-30, all of A times 1e-30: 222 us, 450, 454, 503 (an fp32 MFMA kernel alone: 318).
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int m = min(mw + 16 * mb + lc, p.m - 1), n = min(nw + 16 * nb + 4 * g, pn - 4);
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
-        for (int k = k_lo; k < k_hi; ++k) {
-          const float x = a[(int64_t)m * lda + k];
-          const f32x4 y = *(const f32x4*)(b + (int64_t)k * ldb + n);
+      for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int B0 = TM * 128;
+    static_assert(B0 + kBk * 512 <= 3 * (SA + SB), "a stage of fp32 operands fits the planes' room");
+    load(kt_lo);
+    for (int kt = kt_lo; kt < kt_hi; ++kt) {
+      lds_barrier();
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] = fmaf(x, y[e], s[e]);
-        }
-        acc[mb][nb] = s;
+      for (int i = 0; i < AI; ++i) {
+        const int row = a_row_e + 32 * i;
+        *(lds_u32x4*)(lds + row * 128 + (((tid_e & 7) ^ ((row >> 1) & 7)) << 4)) = av[i];
       }
+#pragma unroll
+      for (int i = 0; i < BI; ++i) {
+        const int row = b_row_e + 8 * i;
+        *(lds_u32x4*)(lds + B0 + row * 512 + (((b_n_e >> 2) ^ (4 * ((row >> 2) & 3))) << 4)) = bv[i];
+      }
+      load(kt + 1);
+      lds_barrier();
+#pragma unroll 1
+      for (int half = 0; half < 2; ++half) {
+        u32x4 x[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const int row = m_e + 16 * mb + lc_e;
+          x[mb] = *(lds_u32x4*)(lds + row * 128 + (((4 * half + g_e) ^ ((row >> 1) & 7)) << 4));
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const int col = n_e + 16 * nb + lc_e;
+            const float y = *(lds_f32*)(lds + B0 + (16 * half + 4 * g_e + t) * 512 + (((col >> 2) ^ (4 * g_e)) << 4) + 4 * (col & 3));
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+              acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, __uint_as_float(x[mb][t]), acc[mb][nb], 0, 0, 0);
+          }
+      }
+    }
   }
 
   // Lane (lc, g) holds row 16 mb + lc of the wave's block, columns 16 nb + 4 g + 0..3.
@@ -267,11 +361,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmParams p) {
   }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    const int m = mw + 16 * mb + lc;
+    const int m = mw + 16 * mb + lc_e;
     if (m >= p.m) continue;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      const int n = nw + 16 * nb + 4 * g;
+      const int n = nw + 16 * nb + 4 * g_e;
       if (n >= pn) continue;
       if (vec) {
         *(f32x4*)(out + (int64_t)m * ldo + n) = acc[mb][nb];
