@@ -107,13 +107,14 @@ struct PvMfma<F16> {
 
 // S^T = K . Q^T + C with Q^T (the B operand) in AGPRs and C, S^T in VGPRs:
 // first() starts a chain from the seed c (S is written to registers apart
-// from c, which stays live), acc() continues it.
+// from c, which stays live), acc() continues it.  The seed may come from a VALU
+// instruction just before: first() waits its two states itself.
 template <typename T>
 struct SMfma;
 template <>
 struct SMfma<BF16> {
   static __device__ __forceinline__ void first(f32x16& s, const u32x4& k, const u32x4& q, const f32x16& c) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(s) : "v"(k), "a"(q), "v"(c));
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(s) : "v"(k), "a"(q), "v"(c));
   }
   static __device__ __forceinline__ void acc(f32x16& s, const u32x4& k, const u32x4& q) {
     asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "a"(q));
@@ -122,7 +123,7 @@ struct SMfma<BF16> {
 template <>
 struct SMfma<F16> {
   static __device__ __forceinline__ void first(f32x16& s, const u32x4& k, const u32x4& q, const f32x16& c) {
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(s) : "v"(k), "a"(q), "v"(c));
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(s) : "v"(k), "a"(q), "v"(c));
   }
   static __device__ __forceinline__ void acc(f32x16& s, const u32x4& k, const u32x4& q) {
     asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "a"(q));
