@@ -35,3 +35,24 @@ def test_compiler_m0_use_in_a_dma_kernel_fails(use):
 def test_m0_use_in_a_kernel_without_the_dma_is_allowed():
     text = listing("k_dma", DMA) + listing("k_other", "\ts_mov_b32 m0, -1\n\tds_read_b32 v0, v1\n")
     assert _build.check_m0(text, "t.hip") == 1
+
+
+MFMA = "\t;;#ASMSTART\n\tv_mfma_f32_16x16x32_f16 a[0:3], v[4:7], v[8:11], a[0:3]\n\t;;#ASMEND\n"
+
+
+def test_spaced_asm_mfma_passes():
+    text = listing("k_mfma", "\tv_mov_b32_e32 v4, v1\n\ts_nop 1\n" + MFMA + "\ts_nop 10\n\tv_accvgpr_read_b32 v0, a1\n")
+    assert _build.check_mfma_asm(text, "t.hip") == 1
+    assert _build.check_mfma_asm(listing("k_other", "\tv_mfma_f32_16x16x32_f16 a[0:3], v[4:7], v[8:11], 0\n"), "t.hip") == 0
+
+
+@pytest.mark.parametrize("body", [
+    "\tv_mov_b32_e32 v9, v1\n\ts_nop 0\n" + MFMA,                          # operand written one state before
+    "\tv_accvgpr_write_b32 a2, v1\n" + MFMA,                               # accumulator likewise
+    MFMA + "\ts_nop 9\n\tv_accvgpr_read_b32 v0, a3\n",                     # result read one state early
+    MFMA + "\tv_accvgpr_write_b32 a0, v1\n",                               # result overwritten
+    ".LBB0_1:\n\tv_accvgpr_read_b32 v0, a3\n\ts_nop 10\n" + MFMA + "\ts_cbranch_scc0 .LBB0_1\n",  # around a loop
+])
+def test_asm_mfma_without_its_wait_states_fails(body):
+    with pytest.raises(RuntimeError, match="k_bad"):
+        _build.check_mfma_asm(listing("k_bad", body), "t.hip")

@@ -24,7 +24,8 @@ typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
 // accumulators between VGPRs and AGPRs, and to scratch, in every pass of the loop.
 // The compiler does not see these as MFMAs: whoever reads an accumulator waits
 // first (mma_drain), and operands come from LDS reads, never from a VALU
-// instruction just before.
+// instruction just before.  The build checks the assembly for both
+// (triton_llm/_build.py check_mfma_asm).
 template <typename T>
 __device__ __forceinline__ void mma16(f32x4& acc, const u32x4& a, const u32x4& b) {
   if constexpr (T::code == TL_DTYPE_BF16)
@@ -32,8 +33,9 @@ __device__ __forceinline__ void mma16(f32x4& acc, const u32x4& a, const u32x4& b
   else
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
-__device__ __forceinline__ void mma_zero(f32x4& acc, const u32x4& zero) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %1, 0" : "=a"(acc) : "v"(zero));
+__device__ __forceinline__ void mma_zero(f32x4& acc) {
+  acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  asm volatile("" : "+a"(acc));
 }
 // The accumulator's value from here on: keeps its copy to VGPRs next to its use.
 __device__ __forceinline__ const f32x4& mma_take(f32x4& acc) {
@@ -189,14 +191,13 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
   for (int s = 0; s < NST - 1; ++s)
 #pragma unroll
     for (int j = 0; j < PER; ++j) load_one(lds0 + s * STAGE, j);
-  {  // while the first stages are on their way: acc = 0 . 0 + 0
-    u32x4 zero = {0, 0, 0, 0};
-    asm volatile("s_nop 1" : "+v"(zero));  // a VALU result an MFMA reads: two wait states
+  // While the first stages are on their way.  Not by an MFMA: where the accumulators
+  // fill every AGPR the register allocator may move one aside here, and would read it
+  // before the MFMA has written it.
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+  for (int i = 0; i < MB; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) mma_zero(acc[i][j], zero);
-  }
+    for (int j = 0; j < NB; ++j) mma_zero(acc[i][j]);
   wait_vmcnt<(NST - 2) * PER>();
   lds_barrier();
 #pragma unroll

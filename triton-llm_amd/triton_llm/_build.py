@@ -107,9 +107,98 @@ def check_m0(asm_text: str, source: str) -> int:
     return sum(1 for dma, _ in funcs.values() if dma)
 
 
+# Wait states: a VALU result before an MFMA reads it; the result of an MFMA of up to
+# 8 passes, or of 16 (32 x 32 blocks), before anything but an MFMA that accumulates
+# on it reads or overwrites it.
+_VALU_TO_MFMA, _MFMA_TO_USE, _MFMA32_TO_USE = 2, 11, 19
+_VECTOR_REGS = re.compile(r"\b([va])(?:(\d+)|\[(\d+):(\d+)\])")
+_STORES = ("ds_write", "buffer_store", "global_store", "flat_store", "scratch_store", "ds_add", "buffer_atomic",
+           "global_atomic")
+
+
+def _vector_regs(operand: str) -> set:
+    out = set()
+    for kind, one, lo, hi in _VECTOR_REGS.findall(operand):
+        out.update((kind, i) for i in (range(int(lo), int(hi) + 1) if lo else (int(one),)))
+    return out
+
+
+def check_mfma_asm(asm_text: str, source: str) -> int:
+    """Reject a kernel whose inline-assembly MFMAs stand too close to an
+    instruction of the compiler's that writes one of their operands or uses their
+    result: its hazard recogniser does not know them as MFMAs and inserts no
+    wait.  Instructions are taken in order, each as one wait state, a branch
+    backwards also as followed by what stands at its target.  Returns the number
+    of kernels that hold such MFMAs."""
+    kernels: dict[str, list] = {}  # name -> [(opcode, operands, inside asm)], labels as (None, name, False)
+    name, in_asm = None, False
+    for line in asm_text.splitlines():
+        m = re.match(r"\s*\.type\s+([^,\s]+)\s*,\s*@function", line)
+        if m:
+            name, in_asm = m.group(1), False
+            kernels[name] = []
+            continue
+        if name is None:
+            continue
+        if ";;#ASMSTART" in line or ";;#ASMEND" in line:
+            in_asm = ";;#ASMSTART" in line
+            continue
+        code = line.split(";", 1)[0].strip()
+        if code.endswith(":"):
+            kernels[name].append((None, code[:-1], False))
+        elif code and not code.startswith("."):
+            op, _, rest = code.partition(" ")
+            kernels[name].append((op, [t.strip() for t in re.split(r",(?![^\[]*\])", rest)], in_asm))
+
+    bad: list[str] = []
+
+    def step(past, op, args, asm):
+        """Check one instruction against the last ones and add it to them."""
+        if op == "s_nop":
+            return past + [(op, set(), set(), int(args[0], 0) + 1)]
+        mfma = op.startswith("v_mfma") and asm
+        writes = _vector_regs(args[0]) if args and not op.startswith(_STORES) else set()
+        reads = set().union(*map(_vector_regs, args[1:])) if len(args) > 1 else set()
+        if op.startswith(_STORES):
+            reads |= _vector_regs(args[0])
+        waited = 0
+        for pop, pwrites, _, states in reversed(past):
+            from_mfma = pop.startswith("asm v_mfma")
+            need = _MFMA32_TO_USE if "_32x32" in pop else _MFMA_TO_USE
+            if mfma and waited < _VALU_TO_MFMA and pop.startswith("v_") and pwrites & reads:
+                bad.append(f"{name}: {op} {', '.join(args)} {waited} wait states after {pop}")
+            if not mfma and waited < need and from_mfma and pwrites & (reads | writes):
+                bad.append(f"{name}: {op} {', '.join(args)} {waited} wait states after an MFMA")
+            waited += states
+            if waited >= _MFMA32_TO_USE:
+                break
+        return (past + [("asm " + op if mfma else op, writes, reads, 1)])[-2 * _MFMA32_TO_USE:]
+
+    held = 0
+    for name, code in kernels.items():
+        if not any(op and op.startswith("v_mfma") and asm for op, _, asm in code):
+            continue
+        held += 1
+        at = {args: i for i, (op, args, _) in enumerate(code) if op is None}
+        past: list = []
+        for i, (op, args, asm) in enumerate(code):
+            if op is None:
+                continue
+            past = step(past, op, args, asm)
+            if op.startswith("s_cbranch") and at.get(args[0], i) < i:
+                again = past
+                for o, a, s in code[at[args[0]]:at[args[0]] + _MFMA32_TO_USE]:
+                    if o is not None:
+                        again = step(again, o, a, s)
+    if bad:
+        raise RuntimeError(f"{os.path.basename(source)}: inline-assembly MFMAs without their wait states:\n  "
+                           + "\n  ".join(bad[:6]))
+    return held
+
+
 def _compile_one(src: str, obj: str) -> None:
     # -save-temps=obj leaves the device assembly next to the object (in the
-    # build's temporary directory) for check_m0.
+    # build's temporary directory) for check_m0 and check_mfma_asm.
     cmd = [_hipcc(), *HIPCC_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-save-temps=obj", "-c", src,
            "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True, cwd=os.path.dirname(obj))
@@ -124,10 +213,14 @@ def _compile_one(src: str, obj: str) -> None:
     if not os.path.exists(asm):
         raise RuntimeError(f"device assembly {asm} missing: cannot check m0 use")
     with open(asm) as f:
-        n_dma = check_m0(f.read(), src)
+        text = f.read()
+    n_dma, n_mfma = check_m0(text, src), check_mfma_asm(text, src)
     with open(src) as f:
-        calls_dma = "lds_dma16(" in f.read()
-    if calls_dma and n_dma == 0:
+        source = f.read()
+    if '"v_mfma' in source and n_mfma == 0:
+        raise RuntimeError(f"{os.path.basename(src)} has inline-assembly MFMAs but check_mfma_asm found none: "
+                           "the guard no longer recognises them")
+    if "lds_dma16(" in source and n_dma == 0:
         raise RuntimeError(f"{os.path.basename(src)} calls lds_dma16 but check_m0 found no kernel issuing it: "
                            "the guard no longer recognises the DMA")
 
