@@ -666,3 +666,62 @@ def test_gemm_fp32_outliers(monkeypatch, M, K, Ns, cus, what):
             np.testing.assert_array_equal(np.isnan(got[:, :n]), np.isnan(exact))
             np.testing.assert_array_equal(got[:, :n][np.isinf(exact)], exact[np.isinf(exact)].astype(np.float32))
             assert (np.abs(got[:, :n][ok] - exact[ok]) <= (K + 4) * 2.0 ** -24 * bound[ok] + 1e-44).all()
+
+
+# Aligned rows whose k ends inside a 16-byte chunk, on the tiles and K slices that
+# whole chunks take: every remainder, fewer k than a chunk, NaN in A's padding and
+# behind B's last row, groups, each way C is stored.
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("M,K,Ns,cus", [(9, 1, (8,), 256), (9, 7, (136,), 256), (65, 33, (264, 8), 256),
+                                        (130, 1002, (328,), 256), (40, 3069, (256,), 256), (300, 135, (584,), 1),
+                                        (300, 134, (584,), 4), (300, 138, (584, 200), 16), (300, 1003, (200,), 256)])
+def test_gemm_ragged_k(monkeypatch, dtype, M, K, Ns, cus):
+    print(f"[case] gemm ragged k {dtype} {M}x{K} -> {Ns} cus {cus}", flush=True)
+    H.set_override(monkeypatch, "TRITON_LLM_HIP_MAX_CUS", cus)
+    rng = np.random.default_rng(M + K + cus)
+    lda = (K + 7) // 8 * 8
+    a = np.full((M, lda), np.nan, np.float32)
+    a[:, :K] = rng.standard_normal((M, K))
+    bs = [np.full((K + 2, n), np.nan, np.float32) for n in Ns]
+    for b in bs:
+        b[:K] = rng.standard_normal((K, b.shape[1])) / np.sqrt(K)
+    a, bs = on.to_storage(a, dtype), [on.to_storage(b, dtype) for b in bs]
+    lib, code, n_g = gpu.runtime(), gpu.dtype_code(H.GPU_DTYPES[dtype]), len(Ns)
+    a_d, b_d, ns = H.upload(a, dtype), [H.upload(b, dtype) for b in bs], (ctypes.c_int * n_g)(*Ns)
+    ws = gpu.allocate((max(1, lib.tl_gemm_grouped_workspace_bytes(M, K, n_g, ns, code)),), np.uint8)
+    for extra, ptr, size in ((0, ws.ptr, ws.nbytes), (4, None, 0), (1, ws.ptr, ws.nbytes)):
+        c_d = [H.upload(on.to_storage(np.full((M, n + extra), 3.0, np.float32), dtype), dtype) for n in Ns]
+        st = lib.tl_gemm_grouped(a_d.ptr, M, K, lda, n_g, (ctypes.c_void_p * n_g)(*[b.data_ptr() for b in b_d]),
+                                 (ctypes.c_void_p * n_g)(*[c.data_ptr() for c in c_d]), ns,
+                                 (ctypes.c_int64 * n_g)(*Ns), (ctypes.c_int64 * n_g)(*[n + extra for n in Ns]),
+                                 ptr, size, code, None)
+        assert st == 0
+        for b, c, n in zip(bs, c_d, Ns):
+            got = on.from_storage(H.download(c), dtype)
+            exp = gemm_ref(on.from_storage(a, dtype)[:, :K], on.from_storage(b, dtype)[:K])
+            np.testing.assert_allclose(got[:, :n], exp, rtol=1e-4 if dtype == "float32" else 8e-3,
+                                       atol=1e-4 if dtype == "float32" else 1e-2)
+            assert (got[:, n:] == 3.0).all()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("lda,ldb", [((1 << 22) + 8, 24), (80, 1 << 24)])
+def test_gemm_long_strides(dtype, lda, ldb):
+    """Row strides whose tiles and stages, counted past the operands' ends, come near
+    or past 32 bits."""
+    M, K, N = 9, 9, 24
+    if dtype == "float32":
+        ldb = min(ldb, 1 << 23)
+    print(f"[case] gemm long strides {dtype} lda {lda} ldb {ldb}", flush=True)
+    rng = np.random.default_rng(lda)
+    a, b = np.zeros((M, lda), np.float32), np.zeros((K, ldb), np.float32)
+    a[:, :K], b[:, :N] = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+    a[:, K:K + 8] = np.nan
+    a_s, b_s = on.to_storage(a, dtype), on.to_storage(b, dtype)
+    exp = gemm_ref(on.from_storage(a_s[:, :K], dtype), on.from_storage(b_s[:, :N], dtype))
+    lib, code = gpu.runtime(), gpu.dtype_code(H.GPU_DTYPES[dtype])
+    a_d, b_d, c_d = H.upload(a_s, dtype), H.upload(b_s, dtype), gpu.allocate((M, N), H.GPU_DTYPES[dtype])
+    assert lib.tl_gemm(a_d.ptr, b_d.ptr, c_d.ptr, M, N, K, lda, ldb, N, None, 0, code, None) == 0
+    got = on.from_storage(H.download(c_d), dtype)
+    np.testing.assert_allclose(got, exp, rtol=1e-4 if dtype == "float32" else 8e-3,
+                               atol=1e-4 if dtype == "float32" else 1e-2)

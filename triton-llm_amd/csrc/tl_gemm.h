@@ -34,9 +34,9 @@ struct GemmParams {
   const void* a;
   int m, k;
   int64_t lda;
-  GemmGroups G;   // tile0 counts 128 x 128 tiles of C
+  GemmGroups G;   // tile0 counts the kernel's tiles of C
   int tiles_m, per_xcd;
-  int vec_store;  // bit g: C_g's rows and base allow 4-column vector stores
+  int vec_store;  // bit g: C_g's rows and base allow vector stores (16 bytes whole, 4 columns where K is split)
   // Split K (ksplit > 1): item (slice s, tile t) covers stages
   // [s kt_per, (s + 1) kt_per) and stores its fp32 partial tile at
   // ws + ws_off[g] + (s m + row) n_g + col; split_reduce_kernel sums them.
@@ -54,28 +54,13 @@ __host__ __device__ __forceinline__ uint32_t view_bytes(int64_t rows, int64_t ld
 }
 
 // Work item of workgroup L: each XCD (workgroups are dealt to the 8 XCDs in
-// turn) takes a contiguous run of items, row tiles fastest, so the
-// workgroups an XCD runs at once share their B column tiles and A row tiles
-// in its L2; items are slice-major (all tiles of K-slice 0, then slice 1).
-__device__ __forceinline__ bool gemm_tile(const GemmParams& p, int& grp, int& tm, int& tn, int& ks) {
-  const int L = blockIdx.x;
-  const int it = (L % 8) * p.per_xcd + L / 8;
-  const int tiles = p.G.tile0[p.G.count];
-  if (it >= tiles * p.ksplit) return false;
-  ks = it / tiles;
-  const int t = it - ks * tiles;
-  grp = find_group(p.G.tile0, p.G.count, t);
-  const int local = t - p.G.tile0[grp];
-  tm = local % p.tiles_m;
-  tn = local / p.tiles_m;
-  return true;
-}
-
-// The same with panels of up to kPanelRows row tiles: a group's tiles are taken
-// panel by panel, rows fastest, so that the tiles an XCD runs at once (32) stay
-// near 8 x 4 whatever the product's height.
+// turn) takes a contiguous run of items, so the workgroups an XCD runs at once
+// share their B column tiles and A row tiles in its L2; items are slice-major (all
+// tiles of K-slice 0, then slice 1).  A group's tiles are taken in panels of up to
+// kPanelRows row tiles, rows fastest, so that the tiles an XCD runs at once (32)
+// stay near 8 x 4 whatever the product's height.
 constexpr int kPanelRows = 8;
-__device__ __forceinline__ bool gemm_tile_panels(const GemmParams& p, int& grp, int& tm, int& tn, int& ks) {
+__device__ __forceinline__ bool gemm_tile(const GemmParams& p, int& grp, int& tm, int& tn, int& ks) {
   const int L = blockIdx.x;
   const int it = (L % 8) * p.per_xcd + L / 8;
   const int tiles = p.G.tile0[p.G.count];

@@ -7,10 +7,8 @@
 // Two regimes:
 //   * a prompt (m > kSkinnyMaxM rows) is a compute-bound GEMM on the matrix
 //     cores with fp32 accumulation: gemm_wide_kernel (tl_gemm_wide.hip) for the
-//     16-bit types, gemm_f32_kernel (tl_gemm_f32.hip) for fp32; gemm_mfma_kernel
-//     (128 x 128 tiles, LDS-DMA staging) where k is not a whole number of
-//     16-byte chunks, the simple fp32-FMA gemm_simple_kernel where rows are not
-//     16-byte aligned.
+//     16-bit types, gemm_f32_kernel (tl_gemm_f32.hip) for fp32, the simple
+//     fp32-FMA gemm_simple_kernel where rows are not 16-byte aligned.
 //     A batch of decoded tokens (a few dozen rows) has too few tiles to fill
 //     the device: K is split into slices with fp32 partials and a reduce pass;
 //   * a decoded token (m <= kSkinnyMaxM rows) reads every weight once for a
@@ -32,8 +30,8 @@ constexpr int kSkinnyMaxM = 8;     // rows of A handled by the skinny path
 constexpr int kMaxSmallSplit = 32; // K-slices at most for few-row MFMA products
 // Rows up to which split_cap counts fp32 tiles of 64 rows.
 constexpr int kNarrowMaxM = 64;
-// gemm_mfma_kernel, fp32: k per LDS stage.
-constexpr int kF32Bk = 16;
+constexpr int kF32Bk = 16;   // k of a stage as split_cap counts them, fp32
+constexpr int kGmTile = 128; // and its tiles' columns
 constexpr int kSkThreads = 256;    // 4 waves
 constexpr int kSkUnroll = 16;      // row loads in flight per lane
 constexpr int kSkMaxTk = 1024;     // rows per K-slice at most (A's slice is staged in LDS)
@@ -352,283 +350,6 @@ int launch_skinny(const void* a, GemmGroups G, int m, int k, int64_t lda, void* 
   return tl_launch_status();
 }
 
-// ---------------------------------------------------------------------------
-// Products on the matrix cores whose rows are 16-byte aligned but whose k is not
-// a whole number of 16-byte chunks (m > kSkinnyMaxM).
-//
-// Workgroup tile 128 x 128 of C, 4 waves in 2 x 2, each wave 64 x 64 (2 x 2
-// blocks of 32 x 32).  K is walked in LDS stages (16-bit: 64 k in two
-// stages; fp32: 16 k in three), every tile moved global -> LDS by LDS-DMA
-// (buffer_load ... lds: no register round trip), every wave loading a
-// quarter.  Each wave computes the transposed block C^T = B^T . A^T with
-// the MFMA, so a lane ends up owning one row of C and 4 consecutive columns
-// per accumulator group: stores are 8 (16-bit) or 16 (fp32) contiguous bytes.
-//
-// Operand layouts in LDS (rows unpadded, 16-byte chunks XOR-swizzled so that
-// every operand read is conflict-free):
-//   A stage: 128 rows (m) x BKB bytes (k), chunk c of row r at slot
-//            c ^ a_swz(r).  A fragment: lane (l % 32, h = l / 32) reads
-//            one 16-byte chunk of row l % 32 of its block: 8 consecutive k
-//            (16-bit) or 4 (fp32).
-//   B stage, 16-bit: 64 rows (k) x 256 bytes (n), chunk c of row r at slot
-//            c ^ (4 (r % 4)).  The MFMA wants 8 consecutive k of one column
-//            per lane, i.e. B read down a column: two ds_read_b64_tr_b16.
-//            That instruction transposes within each 16-lane group: output
-//            lane j, element e is element j % 4 of what lane 4 e + j / 4 of
-//            the group read.  So lane 4 e + p of group g reads row
-//            8 (g / 2) + 4 t + e, columns n0 + 16 (g % 2) + 4 p .. + 3, and
-//            lane 16 g + j receives column n0 + 16 (g % 2) + j, rows
-//            8 (g / 2) + 4 t + 0..3 (t = 0, 1: the two reads).
-//   B stage, fp32: 16 rows (k) x 512 bytes (n), chunk c of row r at slot
-//            c ^ (8 ((r >> 2) & 1)); a lane reads one float of its column.
-// fp32 uses v_mfma_f32_32x32x2f32 with the k order permuted: in k-group q
-// (8 k), step s, lane half h uses k = 8 q + 4 h + s, so one 16-byte A read
-// feeds 4 steps.
-// ---------------------------------------------------------------------------
-constexpr int kGmTile = 128;
-constexpr int kGmThreads = 256;
-
-// BKB: bytes of k per A row per stage (64 or 128); NST: stages in LDS.
-template <typename T, int BKB, int NST>
-__global__ __launch_bounds__(kGmThreads, 2) void gemm_mfma_kernel(GemmParams p) {
-  constexpr int NWV = 4, MBW = 2;  // waves; 32-row blocks of a wave
-  constexpr bool F32 = T::size == 4;
-  constexpr int TM = 64 * MBW;                // rows of C per tile
-  constexpr int BK = BKB / T::size;           // k per stage
-  constexpr int ACH = BKB / 16;               // 16-byte chunks per A row (4 or 8)
-  constexpr int TN = kGmTile;               // columns of C per tile
-  constexpr int BROW = TN * T::size;          // bytes per B row in LDS
-  constexpr int NQ = F32 ? BK / 8 : BK / 16;  // fp32 k-groups / 16-bit k-steps per stage
-  constexpr int kGmStages = NST;
-  constexpr int kGmStageA = TM * BKB;         // bytes of one A stage
-  constexpr int kGmStageB = BK * BROW;        // bytes of one B stage
-  static_assert(kGmStageA % (1024 * NWV) == 0 && kGmStageB % (1024 * NWV) == 0, "every wave loads whole 1 KiB regions");
-  using Bits = typename T::bits;
-  __shared__ __attribute__((aligned(1024))) char smem[kGmStages * (kGmStageA + kGmStageB)];
-
-  // 16 lanes read one chunk of 16 consecutive A rows: the XOR spreads them
-  // over all 16 four-bank groups (64-byte rows: bits 2-3 of the row; 128-byte
-  // rows: bits 1-3).
-  auto a_swz = [](int row) __attribute__((always_inline)) {
-    return ACH == 4 ? (row >> 2) & 3 : (row >> 1) & 7;
-  };
-  int grp, tm, tn, ks;
-  if (!gemm_tile(p, grp, tm, tn, ks)) return;
-  const int pn = p.G.n[grp];
-  const int64_t pldb = p.G.ldb[grp], pldc = p.G.ldc[grp];
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int wm = wave & 1, wn = wave >> 1;  // this wave's (32 MBW) x 64 block
-  const int m_tile = tm * TM, n_tile = tn * TN;
-  __attribute__((address_space(3))) char* const lds_base = (__attribute__((address_space(3))) char*)smem;
-  const uint32_t lds0 = (uint32_t)(size_t)lds_base;
-  const uint32_t lds_a = lds0, lds_b = lds0 + kGmStages * kGmStageA;
-
-  // Buffer resources over all of A (rows < m, its last row to the end of its
-  // last 16-byte chunk: lda is whole chunks) and B (rows < k): rows past them
-  // read as zeros with no memory access.
-  const uint32_t lda2 = (uint32_t)(p.lda * T::size), ldb2 = (uint32_t)(pldb * T::size);
-  const i32x4 ra = uniform_rsrc(p.a, view_bytes(p.m, p.lda, (p.k + 16 / T::size - 1) / (16 / T::size) * (16 / T::size), T::size));
-  const i32x4 rb = uniform_rsrc(p.G.b[grp], view_bytes(p.k, pldb, pn, T::size));
-  auto dma = [&](const i32x4& rs, uint32_t voff, uint32_t la) __attribute__((always_inline)) {
-    lds_dma16(rs, voff, la);
-  };
-  // DMA lane offsets (bytes, stage k0 = 0).  A: region R (1 KiB: 1024 / BKB
-  // rows) is filled by wave R % 4; lane i -> row R * (1024 / BKB) + i / ACH,
-  // slot i % ACH.  The slot swizzle (see a_swz) depends on bits of the row
-  // that the region step 4 j does not change, so one offset serves every
-  // region of this wave.
-  constexpr int A_RPR = 1024 / BKB;
-  const int a_row0 = A_RPR * wave + lane / ACH;
-  const uint32_t a_off = (uint32_t)(m_tile + a_row0) * lda2 + (uint32_t)(((lane % ACH) ^ a_swz(a_row0)) * 16);
-  // B, 16-bit: regions of 4 rows of 256 bytes, lane i -> row 4 R + i / 16,
-  // slot i % 16 (swizzle 4 (row % 4) = 4 (i / 16)).  fp32: regions of 2 rows
-  // of 512 bytes, lane i -> row 2 R + i / 32, slot i % 32 (swizzle
-  // 8 ((row >> 2) & 1) = 8 ((R >> 1) & 1), and R = wave + 4 j keeps that bit).
-  uint32_t b_off;
-  if constexpr (!F32)
-    b_off = (uint32_t)(4 * wave + lane / 16) * ldb2 + (uint32_t)(n_tile * 2) +
-            (uint32_t)(((lane % 16) ^ (4 * (lane / 16))) * 16);
-  else
-    b_off = (uint32_t)(2 * wave + lane / 32) * ldb2 + (uint32_t)(n_tile * 4) +
-            (uint32_t)(((lane % 32) ^ (8 * ((wave >> 1) & 1))) * 16);
-  constexpr int A_REG = kGmStageA / 1024 / NWV;  // regions per wave per stage
-  constexpr int B_REG = kGmStageB / 1024 / NWV;
-  constexpr int B_RPR = 1024 / BROW;           // B rows per region
-  auto load_stage = [&](int kt, int buf) __attribute__((always_inline)) {
-    const uint32_t ka = (uint32_t)(kt * BK * T::size);  // A: column bytes of the stage
-    const uint32_t kb = (uint32_t)(kt * BK) * ldb2;     // B: row offset of the stage
-#pragma unroll
-    for (int j = 0; j < A_REG; ++j)
-      dma(ra, a_off + ka + (uint32_t)(NWV * A_RPR * j) * lda2, lds_a + buf * kGmStageA + (wave + NWV * j) * 1024);
-#pragma unroll
-    for (int j = 0; j < B_REG; ++j)
-      dma(rb, b_off + kb + (uint32_t)(NWV * B_RPR * j) * ldb2, lds_b + buf * kGmStageB + (wave + NWV * j) * 1024);
-  };
-
-  f32x16 acc[MBW][2];  // [m block][n block], C^T layout
-#pragma unroll
-  for (int i = 0; i < MBW; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // Operand read offsets inside a stage.
-  const int lq = lane & 31, h = lane >> 5;
-  // A: row 32 MBW wm + 32 mb + lq, chunk c at slot c ^ a_swz(row).
-  auto a_addr = [&](int mb, int c) __attribute__((always_inline)) {
-    const int row = 32 * MBW * wm + 32 * mb + lq;
-    return row * BKB + ((c ^ a_swz(row)) << 4);
-  };
-  const int n_kt = (p.k + BK - 1) / BK;
-  const int k_rem = p.k - (n_kt - 1) * BK;  // valid k of the last stage
-  const int kt_lo = ks * p.kt_per;          // this item's stages
-  const int kt_hi = min(n_kt, kt_lo + p.kt_per);
-
-#pragma unroll
-  for (int s = 0; s < kGmStages - 1; ++s)
-    if (kt_lo + s < kt_hi) load_stage(kt_lo + s, (kt_lo + s) % kGmStages);
-
-  for (int kt = kt_lo; kt < kt_hi; ++kt) {
-    // stage kt has landed (this wave's loads; the barrier covers the others'):
-    // the stages issued after it, up to NST - 2 of them, may stay in flight
-    constexpr int PER = A_REG + B_REG;
-    if constexpr (NST >= 4) {
-      if (kt + 2 < kt_hi) wait_vmcnt<2 * PER>();
-      else if (kt + 1 < kt_hi) wait_vmcnt<PER>();
-      else wait_vmcnt<0>();
-    } else if constexpr (NST == 3) {
-      if (kt + 1 < kt_hi) wait_vmcnt<PER>();
-      else wait_vmcnt<0>();
-    } else {
-      wait_vmcnt<0>();
-    }
-    lds_barrier();
-    if (kt + kGmStages - 1 < kt_hi) load_stage(kt + kGmStages - 1, (kt + kGmStages - 1) % kGmStages);
-    const int buf = kt % kGmStages;
-    const char* sa = smem + buf * kGmStageA;
-    const char* sb = smem + kGmStages * kGmStageA + buf * kGmStageB;
-    const bool tail = kt == n_kt - 1 && k_rem < BK;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      if constexpr (!F32) {
-        // k-step q: k = 16 q + 8 h + 0..7 of the stage.
-        bf16x8 af[MBW];
-#pragma unroll
-        for (int mb = 0; mb < MBW; ++mb) {
-          u32x4 raw = *(const u32x4*)(sa + a_addr(mb, 2 * q + h));
-          if (tail) {
-            uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (16 * q + 8 * h + e >= k_rem) w[e / 2] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-            raw = u32x4{w[0], w[1], w[2], w[3]};
-          }
-          af[mb] = __builtin_bit_cast(bf16x8, raw);
-        }
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          // lane 16 g + 4 e + p reads row 16 q + 8 (g / 2) + 4 t + e, column
-          // chunk of n = 64 wn + 32 nb + 16 (g % 2) + 4 p.
-          const int g = lane >> 4, e = (lane >> 2) & 3, pp = lane & 3;
-          const int row = 16 * q + 8 * (g >> 1) + e;
-          const int n = 64 * wn + 32 * nb + 16 * (g & 1) + 4 * pp;
-          const int addr = row * BROW + ((((n >> 3)) ^ (4 * (row & 3))) << 4) + 8 * ((n >> 2) & 1);
-          typedef short v4s __attribute__((ext_vector_type(4)));
-          typedef __attribute__((address_space(3))) v4s lds_v4s;
-          const int boff = kGmStages * kGmStageA + buf * kGmStageB + addr;
-          const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_base + boff));
-          const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_base + boff + 4 * BROW));
-          const u32x4 braw = u32x4{__builtin_bit_cast(u32x2, lo).x, __builtin_bit_cast(u32x2, lo).y,
-                                   __builtin_bit_cast(u32x2, hi).x, __builtin_bit_cast(u32x2, hi).y};
-#pragma unroll
-          for (int mb = 0; mb < MBW; ++mb)
-            acc[mb][nb] = Mfma<T>::mma(__builtin_bit_cast(typename Mfma<T>::frag, braw),
-                                       __builtin_bit_cast(typename Mfma<T>::frag, af[mb]), acc[mb][nb]);
-        }
-      } else {
-        // k-group q: k = 8 q + 4 h + s, s = 0..3.
-        f32x4 af[MBW];
-#pragma unroll
-        for (int mb = 0; mb < MBW; ++mb) {
-          f32x4 v = *(const f32x4*)(sa + a_addr(mb, 2 * q + h));
-          if (tail) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-              if (8 * q + 4 * h + s >= k_rem) v[s] = 0.f;
-          }
-          af[mb] = v;
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int row = 8 * q + 4 * h + s;
-#pragma unroll
-          for (int nb = 0; nb < 2; ++nb) {
-            const int byte = (64 * wn + 32 * nb + lq) * 4;
-            const float bv = *(const float*)(sb + row * BROW + (byte ^ (128 * ((row >> 2) & 1))));
-#pragma unroll
-            for (int mb = 0; mb < MBW; ++mb)
-              acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv, af[mb][s], acc[mb][nb], 0, 0, 0);
-          }
-        }
-      }
-    }
-  }
-  wait_vmcnt<0>();
-
-  // lane (lq, h) holds row m = m_tile + 32 MBW wm + 32 mb + lq and, for
-  // a = 0..3, columns n = n_tile + 64 wn + 32 nb + 8 a + 4 h + 0..3.
-  if (p.ksplit > 1) {
-    // fp32 partial of this K-slice; n_g is a multiple of 4 on this path, so
-    // every 4-column run is whole and 16-byte aligned
-    float* wsb = p.ws + p.ws_off[grp] + (int64_t)ks * p.m * pn;
-#pragma unroll
-    for (int mb = 0; mb < MBW; ++mb) {
-      const int m = m_tile + 32 * MBW * wm + 32 * mb + lq;
-      if (m >= p.m) continue;
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int n = n_tile + 64 * wn + 32 * nb + 8 * a + 4 * h;
-          if (n < pn)
-            *(f32x4*)(wsb + (int64_t)m * pn + n) =
-                f32x4{acc[mb][nb][4 * a], acc[mb][nb][4 * a + 1], acc[mb][nb][4 * a + 2], acc[mb][nb][4 * a + 3]};
-        }
-    }
-    return;
-  }
-  Bits* cbase = (Bits*)p.G.c[grp];
-  const bool vec = (p.vec_store >> grp) & 1;
-#pragma unroll
-  for (int mb = 0; mb < MBW; ++mb) {
-    const int m = m_tile + 32 * MBW * wm + 32 * mb + lq;
-    if (m >= p.m) continue;
-    Bits* crow = cbase + (int64_t)m * pldc;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int n = n_tile + 64 * wn + 32 * nb + 8 * a + 4 * h;
-        const float v[4] = {acc[mb][nb][4 * a], acc[mb][nb][4 * a + 1], acc[mb][nb][4 * a + 2],
-                            acc[mb][nb][4 * a + 3]};
-        if (vec && n + 3 < pn) {
-          if constexpr (F32) {
-            *(f32x4*)(crow + n) = f32x4{v[0], v[1], v[2], v[3]};
-          } else {
-            const float x0[2] = {v[0], v[1]}, x1[2] = {v[2], v[3]};
-            *(u32x2*)(crow + n) = u32x2{pack2<T>(x0), pack2<T>(x1)};
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < pn) crow[n + e] = from_f32<T>(v[e]);
-        }
-      }
-  }
-}
-
 // Split-K finish: C_g = sum over the K-slices of the fp32 partial tiles
 // (slice 0 first, so the result does not depend on timing), rounded to T.
 // One 4-column run per thread, grid-stride; blockIdx.y = group.
@@ -669,7 +390,7 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmParams p) {
   }
 }
 
-// Any shape and alignment (the MFMA kernel needs 16-byte aligned rows):
+// Any shape and alignment (the MFMA kernels need 16-byte aligned rows):
 // 64 x 64 tiles of C_g (g = blockIdx.z), 256 threads with 4 x 4 outputs
 // each, fp32 FMA over 16-deep K slices staged in LDS with bounds checks.
 // Used for small or odd shapes only.
@@ -786,16 +507,6 @@ SplitCap split_cap(int m, int k, const GemmGroups& G, int esize) {
   return cap(split);
 }
 
-// Whether a 16-bit product whose rows are 16-byte aligned runs on
-// gemm_wide_kernel: k in whole 16-byte chunks (its last stage drops the chunks
-// past k, and only whole ones), and 32-bit offsets for a row tile of A and for
-// the stages its prefetch counts past the end of each B.
-bool wide_ok(const GemmGroups& G, int k, int64_t lda) {
-  bool ok = k % 8 == 0 && lda * 2 * 256 < ((int64_t)1 << 31);
-  for (int g = 0; g < G.count; ++g) ok = ok && ((int64_t)k + 512) * G.ldb[g] * 2 < ((int64_t)1 << 32);
-  return ok;
-}
-
 // Whether an output shares bytes with A or with a B.  Such a product comes out
 // right where K is cut: every operand is read before the reduce pass writes the
 // first output.  So it is cut where the workspace allows.
@@ -820,9 +531,9 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
   p.G = G;
   const int64_t esize = T::size;
   const int64_t vec = 16 / esize;  // elements per 16-byte chunk
-  // Every operand's rows must be 16-byte aligned for the LDS-DMA staging, and
-  // all of A and each B addressable with 32-bit offsets (stage reads run up
-  // to one stage past the last row / k).
+  // Every operand's rows must be 16-byte aligned for the loads, and all of A and
+  // each B addressable with 32-bit offsets (counted up to a tile past A's last row
+  // and two stages past B's).
   bool aligned = lda % vec == 0 && ((uintptr_t)a % 16) == 0 &&
                  ((int64_t)m + 2 * kGmTile + 1) * lda * esize < ((int64_t)1 << 32);
   int widest = 0;
@@ -854,22 +565,14 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
       p.per_xcd = (p.G.tile0[G.count] * ksplit + 7) / 8;
     };
     int e;
-    if (T::size == 4 && k % 4 == 0) {
+    if (T::size == 4) {
       const F32Plan W = gemm_f32_plan(m, k, G, min_split, max_split);
-      place(W.tm, kGmTile, W.ksplit, W.kt_per, 4);
+      place(W.tm, 128, W.ksplit, W.kt_per, 4);
       e = launch_gemm_f32(p, W.tm, st);
-    } else if (T::size == 2 && wide_ok(G, k, lda)) {
+    } else {
       const WidePlan W = gemm_wide_plan(m, k, G, min_split, max_split);
       place(W.tm, W.tn, W.ksplit, W.kt_per, W.ksplit > 1 ? 4 : 8);  // the reduce stores 4 columns, the kernel 8
       e = launch_gemm_wide(p, W, (int)T::code, st);
-    } else {
-      // the stage of gemm_mfma_kernel: 64 k (16-bit), kF32Bk k (fp32)
-      const int bk = T::size == 2 ? 64 : kF32Bk, n_kt = (k + bk - 1) / bk;
-      place(kGmTile, kGmTile, max_split, (n_kt + max_split - 1) / max_split, 4);
-      const dim3 grid((unsigned)(8 * p.per_xcd));
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, T::size == 2 ? 128 : 4 * kF32Bk, T::size == 2 ? 2 : 3>), grid, dim3(kGmThreads),
-                         0, st, p);
-      e = tl_launch_status();
     }
     if (e || p.ksplit == 1) return e;
     int64_t runs = 0;

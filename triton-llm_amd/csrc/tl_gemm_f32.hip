@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   __shared__ float s_row[TM], s_col[8][TN], s_max[4], s_least[4];
 
   int grp, tm, tn, ks;
-  if (!gemm_tile_panels(p, grp, tm, tn, ks)) return;
+  if (!gemm_tile(p, grp, tm, tn, ks)) return;
   const int pn = p.G.n[grp];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -85,10 +85,11 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   const int m_tile = tm * TM, n_tile = tn * TN;
   __attribute__((address_space(3))) char* const lds = (__attribute__((address_space(3))) char*)smem;
 
-  const int n_kt = (p.k + kBk - 1) / kBk;
+  const int km = p.k & ~3;  // whole 16-byte chunks; the last k % 4 are added at the end
+  const int n_kt = (km + kBk - 1) / kBk;
   const int kt_lo = ks * p.kt_per;
   const int kt_hi = min(n_kt, kt_lo + p.kt_per);
-  const int k_lo = kt_lo * kBk, k_hi = min(p.k, kt_hi * kBk);
+  const int k_hi = min(km, kt_hi * kBk);
   const float* const a = (const float*)p.a;
   const float* const b = (const float*)p.G.b[grp];
   const int64_t lda = p.lda, ldb = p.G.ldb[grp];
@@ -107,8 +108,8 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   const int b_row = tid >> 5, b_n = 4 * (tid & 31);
   u32x4 av[AI], bv[BI];
   auto load = [&](int kt) __attribute__((always_inline)) {
-    const int k0 = kt * kBk;
-    const bool a_in = k0 + a_k < k_hi;  // k in whole 16-byte chunks
+    const int k0 = min(kt, kt_hi) * kBk;  // past the slice: zeros, and no offset that wraps
+    const bool a_in = k0 + a_k < k_hi;
 #pragma unroll
     for (int i = 0; i < AI; ++i)
       av[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
@@ -243,8 +244,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   // magnitude is not between 2^-40 and 2^60 (NaN and infinity included; all zeros are
   // fine), and a sum below 2^-44 of its row's largest times its column's, which may
   // be made of entries below 2^-102 alone (above it they weigh k 2^-42 at most).  The
-  // look at the sums costs 0.5 us a product, 1.4% of a SmolLM2-360M layer; one at
-  // every entry as it is split costs more.
+  // look at the sums costs 0.5 us a product, 1.4% of a SmolLM2-360M layer.
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
     float v = a_max[i];
@@ -350,6 +350,19 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
     }
   }
 
+  if (ks == 0)
+    for (int k = km; k < p.k; ++k)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const f32x4 y = *(const f32x4*)(b + (int64_t)k * ldb + min(nw + 16 * nb + 4 * g_e, pn - 4));
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const float x = a[(int64_t)min(mw + 16 * mb + lc_e, p.m - 1) * lda + k];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[mb][nb][e] = fmaf(x, y[e], acc[mb][nb][e]);
+        }
+      }
+
   // Lane (lc, g) holds row 16 mb + lc of the wave's block, columns 16 nb + 4 g + 0..3.
   float* out = (float*)p.G.c[grp];
   int64_t ldo = p.G.ldc[grp];
@@ -382,7 +395,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
 F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int min_split, int max_split) {
   F32Plan best{};
   const int cus = tl_device_cus();
-  const int stages = (k + kBk - 1) / kBk;
+  const int stages = (k / 4 * 4 + kBk - 1) / kBk;
   int64_t ncols = 0;
   for (int g = 0; g < G.count; ++g) ncols += G.n[g];
   for (const F32Tile& c : kF32Tiles) {

@@ -55,18 +55,18 @@ __device__ __forceinline__ void mma_drain() { asm volatile("s_nop 15\n\ts_nop 15
 //   * 16x16x32 MFMAs: with random operands the chip's power limit holds a stream
 //     of them at 2.1 PFLOP/s (2.09 GHz) and one of 32x32x16 at 1.8 (1.78 GHz).
 //   * 128 x 128 a wave: an LDS byte read feeds twice the MFMAs of the 64 x 64
-//     waves of gemm_mfma_kernel, and one wave per SIMD has the registers for it
+//     waves of an 8-wave kernel with 32x32x16 MFMAs, and one wave per SIMD has the registers for it
 //     (256 accumulators in AGPRs, two operand sets in VGPRs).
 //   * Operands a stage ahead: nothing waits on an LDS read, and the stage's
 //     1024 MFMA cycles take 1050-1250 with operands from L2, 1500 where weights
 //     come from HBM (their latency; deeper rings than LDS has would help).
 //   * Five ring stages against four: 8192^3 912 -> 1447 TFLOP/s together with the
-//     panel order of gemm_tile_panels (hipBLASLt: 1290).
+//     panel order of gemm_tile (hipBLASLt: 1290).
 //   * C through LDS, whole row pieces: epilogue 16600 -> 9000 cycles of a tile's
 //     150000, against 8-byte stores from the accumulators.
 // gate/up 205 -> 163 us (1250 TFLOP/s), down 122 -> 103, q/k/v 84 -> 55; of 98
 // products of these models' shapes against the 64-, 128- and 256-row tiles of
-// gemm_mfma_kernel that this replaced, 9 to 64 rows ran at 0.96 to 1.36 times
+// that kernel, which this replaced, 9 to 64 rows ran at 0.96 to 1.36 times
 // their speed, 100 to 4096 rows at 1.04 to 1.76 times but for one, gate/up at 384
 // rows (53.8 -> 55.9 us; again, twice a side in turn: 58.8, 57.7 -> 58.6, 58.9,
 // where 448 rows take 61.3 -> 52.7: the model misses the best tile there).  64 rows
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[NST * STAGE];
 
   int grp, tm, tn, ks;
-  if (!gemm_tile_panels(p, grp, tm, tn, ks)) return;
+  if (!gemm_tile(p, grp, tm, tn, ks)) return;
   const int pn = p.G.n[grp];
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -109,26 +109,34 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
   const int n_kt = (p.k + BK - 1) / BK;
   const int kt_lo = ks * p.kt_per;
   const int kt_hi = min(n_kt, kt_lo + p.kt_per);
-  const int k_hi = min(p.k, kt_hi * BK);
+  // Where k ends inside a 16-byte chunk the last 32-k block comes first, as stage 0:
+  // what its chunk holds past k is then cleared in LDS once (below), before the ring
+  // turns.  The blocks of the other stages are whole.
+  const bool ragged = (p.k & 7) != 0, ends_first = ragged && ks == 0;
+  const int block = ragged ? (ends_first ? n_kt - 1 : kt_lo - 1) : kt_lo;  // of the first stage
   const uint32_t lda2 = (uint32_t)(p.lda * 2), ldb2 = (uint32_t)(p.G.ldb[grp] * 2);
   const int rows = min(TM, p.m - m_tile);
-  // A from this tile's first row, to its last row's k; B to the slice's last row's n.
-  // The range check covers voff + soff, and what is past it reads as zeros: rows
-  // past m, k rows past the slice.  A's chunks past the slice are sent out of range
-  // (a_cur below); a stage of zeros adds nothing, so the ring needs no tail.
-  const i32x4 ra = uniform_rsrc((const char*)p.a + (int64_t)m_tile * lda2, view_bytes(rows, p.lda, p.k, 2));
-  const i32x4 rb = uniform_rsrc(p.G.b[grp], view_bytes(k_hi, p.G.ldb[grp], pn, 2));
+  // A from this tile's first row, to the end of its last row's last chunk; B to its
+  // last row's n.  The range check covers voff + soff, and what is past it reads as
+  // zeros: rows past m, k rows past the last.  A's chunks past the slice are sent to
+  // the resource's end (a_cur below), B's stages past it too (b_soff): no sum of
+  // offsets passes 32 bits that an address of the operands does not.  A stage of zeros
+  // adds nothing, so the ring needs no tail.
+  const uint32_t a_end = view_bytes(rows, p.lda, (p.k + 7) & ~7, 2), b_end = (uint32_t)p.k * ldb2;
+  const i32x4 ra = uniform_rsrc((const char*)p.a + (int64_t)m_tile * lda2, a_end);
+  const i32x4 rb = uniform_rsrc(p.G.b[grp], view_bytes(p.k, p.G.ldb[grp], pn, 2));
 
   auto b_swz = [](int row) __attribute__((always_inline)) {
     return (BCH % 16 == 0 ? 4 * (row & 3) : 4 * ((row >> 1) & 1)) ^ (2 * ((row >> 3) & 1));
   };
   uint32_t a_voff, b_off[B_REG], a_soff[A_REG];
-  int a_left;  // k left of this lane's chunk in the next stage to load
+  int a_left;                   // k left of this lane's chunk in the next stage to load
+  int b_left = kt_hi - kt_lo;   // stages left
   {
     const int row = 16 * wave + lane / 4;
     const int ch = (lane & 3) ^ ((row >> 2) & 3);
-    a_voff = (uint32_t)row * lda2 + (uint32_t)(ch * 16) + (uint32_t)(kt_lo * AROW);
-    a_left = k_hi - kt_lo * BK - 8 * ch;
+    a_voff = (uint32_t)row * lda2 + (uint32_t)(ch * 16) + (uint32_t)(block * AROW);
+    a_left = (ragged && !ends_first ? (kt_hi - kt_lo) * BK : min(p.k, (ends_first ? n_kt : kt_hi) * BK) - block * BK) - 8 * ch;
 #pragma unroll
     for (int j = 0; j < A_REG; ++j) a_soff[j] = (uint32_t)(64 * j) * lda2;
 #pragma unroll
@@ -138,11 +146,11 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
       b_off[j] = (uint32_t)r * ldb2 + (uint32_t)(n_tile * 2) + (uint32_t)((slot ^ b_swz(r)) * 16);
     }
   }
-  uint32_t b_soff = (uint32_t)(kt_lo * BK) * ldb2;
+  uint32_t b_soff = (uint32_t)min(block * BK, p.k) * ldb2;
   uint32_t a_cur = 0;
   // load j of the next stage in turn; j = 0 fixes the stage's A offset, the last moves on
   auto load_one = [&](uint32_t buf_base, int j) __attribute__((always_inline)) {
-    if (j == 0) a_cur = a_left > 0 ? a_voff : 0x80000000u;
+    if (j == 0) a_cur = a_left > 0 ? a_voff : a_end;
     if (j < A_REG)
       lds_dma16(ra, a_cur, buf_base + (wave + 4 * j) * 1024, a_soff[j]);
     else
@@ -150,7 +158,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
     if (j == PER - 1) {
       a_voff += AROW;
       a_left -= BK;
-      b_soff += (uint32_t)BK * ldb2;
+      b_soff = --b_left > 0 ? b_soff + (uint32_t)BK * ldb2 : b_end;
     }
   };
 
@@ -188,9 +196,15 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
   };
 
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
+  for (int s = 0; s < NST - 1; ++s) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) load_one(lds0 + s * STAGE, j);
+    if (s == 0 && ends_first) {  // on to block 0, kt_hi - 1 blocks
+      a_voff -= (uint32_t)(n_kt * AROW);
+      a_left += (kt_hi - 1) * BK - (p.k - n_kt * BK);
+      b_soff = b_left > 0 ? 0 : b_end;
+    }
+  }
   // While the first stages are on their way.  Not by an MFMA: where the accumulators
   // fill every AGPR the register allocator may move one aside here, and would read it
   // before the MFMA has written it.
@@ -200,6 +214,18 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(GemmParams p) {
     for (int j = 0; j < NB; ++j) mma_zero(acc[i][j]);
   wait_vmcnt<(NST - 2) * PER>();
   lds_barrier();
+  if (ends_first) {
+    const int row = threadIdx.x, left = p.k & 7;
+    if (row < TM) {
+      lds_u32x4* const at = (lds_u32x4*)(lds + row * AROW + (((p.k % BK / 8) ^ ((row >> 2) & 3)) << 4));
+      u32x4 w = *at;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e >= left) w[e / 2] &= e & 1 ? 0x0000ffffu : 0xffff0000u;
+      *at = w;
+    }
+    lds_barrier();
+  }
 #pragma unroll
   for (int i = 0; i < NRD; ++i) read_one(0, 0, i);
 
