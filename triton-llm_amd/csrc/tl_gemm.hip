@@ -27,11 +27,7 @@ using namespace tlg;
 namespace {
 
 constexpr int kSkinnyMaxM = 8;     // rows of A handled by the skinny path
-constexpr int kMaxSmallSplit = 32; // K-slices at most for few-row MFMA products
-// Rows up to which split_cap counts fp32 tiles of 64 rows.
-constexpr int kNarrowMaxM = 64;
-constexpr int kF32Bk = 16;   // k of a stage as split_cap counts them, fp32
-constexpr int kGmTile = 128; // and its tiles' columns
+constexpr int kMaxSplit = 32;      // K-slices at most of a matrix-core product
 constexpr int kSkThreads = 256;    // 4 waves
 constexpr int kSkUnroll = 16;      // row loads in flight per lane
 constexpr int kSkMaxTk = 1024;     // rows per K-slice at most (A's slice is staged in LDS)
@@ -434,77 +430,42 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(GemmParams p) {
     }
 }
 
-// The most K-slices a product of more than kSkinnyMaxM rows may run in, and the
-// bytes of their fp32 partials: what tl_gemm_workspace_bytes answers.  The
-// kernels' own plans (gemm_wide_plan, gemm_f32_plan) choose within it.
-struct SplitCap {
-  int ksplit;
-  size_t ws_bytes;
+// The plan of a product of more than kSkinnyMaxM rows on the matrix cores, with
+// min_split to max_split K-slices.
+struct PromptPlan {
+  WidePlan wide;  // 16-bit
+  int tm, tn, ksplit, kt_per;
 };
 
-// Few rows (a batch of decoded tokens): the product streams B, and a few dozen
-// tiles of C, each walking all of K, leave most CUs idle, so K may be cut until
-// about one item per CU runs for 16-bit products and two for fp32 ones, while
-// the fp32 partials stay under half of B's bytes (which rules out large m) and
-// every slice keeps two stages.  fp32 prompts beyond that: a CU's time is set by
-// the whole items it runs (384 tiles on 256 CUs cost two tiles' time where 1.5
-// would do), so up to four slices where the busiest CU's share, plus the reduce
-// pass, comes out 3% lower, counted in 128-row tiles or 64-row ones.  16-bit
-// prompts beyond it are not split: at their speed the partials' traffic costs
-// more than the balance gains.
-SplitCap split_cap(int m, int k, const GemmGroups& G, int esize) {
-  const int cus = tl_device_cus();
-  const bool narrow = esize == 4 && m <= kNarrowMaxM;
-  int64_t ncols = 0;
-  for (int g = 0; g < G.count; ++g) ncols += G.n[g];
-  auto cap = [&](int S) { return SplitCap{S, S > 1 ? (size_t)S * m * ncols * sizeof(float) : 0}; };
-  auto tiles_of = [&](int tm) {
-    int64_t tiles = 0;
-    for (int g = 0; g < G.count; ++g) tiles += (int64_t)((m + tm - 1) / tm) * ((G.n[g] + kGmTile - 1) / kGmTile);
-    return tiles;
-  };
-  const int64_t tiles = tiles_of(narrow ? kGmTile / 2 : kGmTile);
-  const int bk = esize == 2 ? 64 : kF32Bk;
-  const int n_kt = (k + bk - 1) / bk;
-  if (tiles < 2 * cus) {
-    const int64_t by_traffic = (int64_t)k * esize / (2 * 4 * (int64_t)m);
-    int64_t S = ((esize == 2 ? 1 : 2) * cus + tiles - 1) / tiles;
-    S = S < by_traffic ? S : by_traffic;
-    S = S < n_kt / 2 ? S : n_kt / 2;
-    S = S < kMaxSmallSplit ? S : kMaxSmallSplit;
-    if (S >= 2) return cap((int)S);
+PromptPlan prompt_plan(int m, int k, const GemmGroups& G, int esize, int min_split, int max_split) {
+  PromptPlan P{};
+  if (esize == 4) {
+    const F32Plan f = gemm_f32_plan(m, k, G, min_split, max_split);
+    P.tm = f.tm, P.tn = 128, P.ksplit = f.ksplit, P.kt_per = f.kt_per;
+  } else {
+    P.wide = gemm_wide_plan(m, k, G, min_split, max_split);
+    P.tm = P.wide.tm, P.tn = P.wide.tn, P.ksplit = P.wide.ksplit, P.kt_per = P.wide.kt_per;
   }
-  if (esize == 2) return cap(1);
-  const double rate = 1.3e14;  // FLOP/s
-  auto reduce_t = [&](int S) { return ((double)S * 4 + esize) * m * (double)ncols / 5.0e12 + 3e-6; };
-  const double t1 = 2.0 * m * (double)k * (double)ncols / rate;
-  auto busiest = [&](int S) { return (double)((tiles * S + cus - 1) / cus) / S; };
-  int split = 1;
-  double best = t1;
-  for (int S = 2; S <= 4 && n_kt >= 4 * S; ++S) {
-    const double t = t1 * busiest(S) / busiest(1) + reduce_t(S);
-    if (t < 0.97 * best) {
-      best = t;
-      split = S;
-    }
-  }
-  if (narrow) return cap(split);
-  // two items a CU at the rate, a lone one at 0.71 of it, 64-row ones at 0.865
-  const double r2 = rate / cus, r1 = r2 * (0.58 / 0.82);
-  auto model = [&](int tm, int S) {
-    const int64_t per_cu = (tiles_of(tm) * S + cus - 1) / cus;
-    const double w = 2.0 * tm * kGmTile * (double)k / S / (tm < kGmTile ? 0.865 : 1.0);
-    return (double)(per_cu - per_cu % 2) * w / r2 + (double)(per_cu % 2) * w / r1 + (S > 1 ? reduce_t(S) : 0.0);
-  };
-  double t_best = 0.97 * model(kGmTile, split);
-  for (int S = 1; S <= 4 && (S == 1 || (k + 31) / 32 >= 4 * S); ++S) {
-    const double t = model(kGmTile / 2, S);
-    if (t < t_best) {
-      t_best = t;
-      split = S;
-    }
-  }
-  return cap(split);
+  return P;
+}
+
+// K-slices whose fp32 partials are about half as large as B in 16 bits, as large as
+// B in fp32: B is what a product of few rows streams.
+int few_rows_split(int m, int k, int esize) {
+  return esize == 2 ? (int)(((int64_t)k + 4 * (int64_t)m - 1) / (4 * (int64_t)m)) : k / m;
+}
+
+// The most K-slices a plan may choose: those, 32 at most; of an fp32 product, whose
+// matrix-core time outweighs the partials' traffic at any height, four.
+int max_split(int m, int k, int esize) {
+  const int few = few_rows_split(m, k, esize), least = esize == 4 ? 4 : 1;
+  return few > kMaxSplit ? kMaxSplit : few > least ? few : least;
+}
+
+size_t split_bytes(int m, const GemmGroups& G, int ksplit) {
+  size_t ncols = 0;
+  for (int g = 0; g < G.count; ++g) ncols += (size_t)G.n[g];
+  return ksplit > 1 ? (size_t)ksplit * m * ncols * sizeof(float) : 0;
 }
 
 // Whether an output shares bytes with A or with a B.  Such a product comes out
@@ -535,7 +496,7 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
   // each B addressable with 32-bit offsets (counted up to a tile past A's last row
   // and two stages past B's).
   bool aligned = lda % vec == 0 && ((uintptr_t)a % 16) == 0 &&
-                 ((int64_t)m + 2 * kGmTile + 1) * lda * esize < ((int64_t)1 << 32);
+                 ((int64_t)m + 257) * lda * esize < ((int64_t)1 << 32);
   int widest = 0;
   for (int g = 0; g < G.count; ++g) {
     aligned = aligned && G.ldb[g] % vec == 0 && G.n[g] % vec == 0 && ((uintptr_t)G.b[g] % 16) == 0 &&
@@ -543,37 +504,26 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
     widest = G.n[g] > widest ? G.n[g] : widest;
   }
   if (aligned) {
-    // as many K-slices as the workspace query's answer holds, where it was given
-    const SplitCap cap = split_cap(m, k, G, (int)esize);
-    const int max_split = workspace && workspace_bytes >= cap.ws_bytes && ((uintptr_t)workspace % 16) == 0 ? cap.ksplit : 1;
-    const int min_split = in_place && max_split > 1 ? 2 : 1;
-    // tiles of tm x tn, K in ksplit slices of kt_per stages, run columns a store
-    auto place = [&](int tm, int tn, int ksplit, int kt_per, int run) {
-      p.tiles_m = (m + tm - 1) / tm;
-      for (int g = 0; g < G.count; ++g) {
-        p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + tn - 1) / tn);
-        if (G.ldc[g] % run == 0 && ((uintptr_t)G.c[g] % (run * esize)) == 0) p.vec_store |= 1 << g;
-      }
-      p.ksplit = ksplit;
-      p.kt_per = kt_per;
-      p.ws = (float*)workspace;
-      int64_t off = 0;
-      for (int g = 0; g < G.count; ++g) {
-        p.ws_off[g] = off;
-        off += (int64_t)ksplit * m * G.n[g];
-      }
-      p.per_xcd = (p.G.tile0[G.count] * ksplit + 7) / 8;
-    };
-    int e;
-    if (T::size == 4) {
-      const F32Plan W = gemm_f32_plan(m, k, G, min_split, max_split);
-      place(W.tm, 128, W.ksplit, W.kt_per, 4);
-      e = launch_gemm_f32(p, W.tm, st);
-    } else {
-      const WidePlan W = gemm_wide_plan(m, k, G, min_split, max_split);
-      place(W.tm, W.tn, W.ksplit, W.kt_per, W.ksplit > 1 ? 4 : 8);  // the reduce stores 4 columns, the kernel 8
-      e = launch_gemm_wide(p, W, (int)T::code, st);
+    const int most = max_split(m, k, (int)esize);
+    PromptPlan P = prompt_plan(m, k, G, (int)esize, in_place && most > 1 ? 2 : 1, most);
+    if (P.ksplit > 1 &&
+        (!workspace || workspace_bytes < split_bytes(m, G, P.ksplit) || ((uintptr_t)workspace % 16) != 0))
+      P = prompt_plan(m, k, G, (int)esize, 1, 1);
+    // columns of one store: 16 bytes from the kernels, 4 from the reduce
+    const int run = P.ksplit > 1 || esize == 4 ? 4 : 8;
+    p.tiles_m = (m + P.tm - 1) / P.tm;
+    int64_t off = 0;
+    for (int g = 0; g < G.count; ++g) {
+      p.G.tile0[g + 1] = p.G.tile0[g] + p.tiles_m * ((G.n[g] + P.tn - 1) / P.tn);
+      if (G.ldc[g] % run == 0 && ((uintptr_t)G.c[g] % (run * esize)) == 0) p.vec_store |= 1 << g;
+      p.ws_off[g] = off;
+      off += (int64_t)P.ksplit * m * G.n[g];
     }
+    p.ksplit = P.ksplit;
+    p.kt_per = P.kt_per;
+    p.ws = (float*)workspace;
+    p.per_xcd = (p.G.tile0[G.count] * P.ksplit + 7) / 8;
+    const int e = T::size == 4 ? launch_gemm_f32(p, P.tm, st) : launch_gemm_wide(p, P.wide, (int)T::code, st);
     if (e || p.ksplit == 1) return e;
     int64_t runs = 0;
     for (int g = 0; g < G.count; ++g) runs = (int64_t)m * (G.n[g] / 4) > runs ? (int64_t)m * (G.n[g] / 4) : runs;
@@ -675,11 +625,12 @@ size_t groups_workspace_bytes(int m, int k, const GemmGroups& G, int dtype) {
     if (G.n[g] > 0) live.n[live.count++] = G.n[g];
   if (live.count == 0) return 0;
   const int esize = dtype == TL_DTYPE_F32 ? 4 : 2;
-  // few rows: the K-slice partials; more: the MFMA kernel's split-K partials
-  // (if its plan splits; a product that falls back to the simple kernel
-  // uses none of it)
+  // few rows: the K-slice partials; more: those of the plan's slices, and of two
+  // where they are cheap, for a C that overlaps A or B (a product that falls back to
+  // the simple kernel uses none of it)
   if (m <= kSkinnyMaxM) return skinny_workspace_bytes(m, live, k, esize);
-  return split_cap(m, k, live, esize).ws_bytes;
+  const int chosen = prompt_plan(m, k, live, esize, 1, max_split(m, k, esize)).ksplit;
+  return split_bytes(m, live, chosen > 1 ? chosen : few_rows_split(m, k, esize) > 1 ? 2 : 1);
 }
 
 }  // namespace

@@ -18,10 +18,13 @@ struct F32Tile {
   double stage_us[3];  // a 32-k stage of one, two, three of them on a CU
 };
 // Both heights, as measured at 30 to 256 stages; a split's partials are written,
-// read and summed at about 5 TB/s, with one more launch.  Chosen so, the kernel is
-// at least as fast as the best fp32 MFMA plan was at 96 products of 9 to 2048 rows
-// (0.97 to 1.01 at the seven smallest, 1.04 to 1.87 at the others).
-const F32Tile kF32Tiles[] = {{128, 2, {1.6, 2.75, 0}}, {64, 3, {1.2, 1.8, 2.55}}};
+// read and summed at about 5 TB/s, with one more launch and a part per slice.  Of 74
+// products of 9 to 4096 rows at the Llama-3.2-3B and SmolLM2 widths, weights rotated
+// through 1 GB, 61 run at 1.0 to 2.3 times the speed of the best fp32 MFMA plan; 13, of
+// 9 to 500 rows at K 576 to 2560, at 0.88 to 0.97 (32 x 576 x (576, 192, 192) 10.1 ->
+// 11.5 us, the widest): two or three stages a slice, whose loads, splits and range
+// check follow one another.
+const F32Tile kF32Tiles[] = {{128, 2, {1.6, 2.75, 0}}, {64, 3, {1.3, 1.8, 2.55}}};
 
 // x0, x1 as three pairs of bf16 whose sums are x0 and x1 exactly (8 significant
 // bits each, rounded to nearest, so every remainder is exact).
@@ -50,8 +53,7 @@ __device__ __forceinline__ float wave_max(float x) {
 // the exact sum of three bf16 parts (Henry, Tang, Heinecke: Leveraging the bfloat16
 // Artificial Intelligence Datatype For Higher-Precision Computations, ARITH 2019),
 // and a product is six 16x16x32 bf16 MFMAs (2.5 PFLOP/s / 6) where the fp32 MFMA's
-// peak is 157 TFLOP/s.  A stage's fp32
-// values are loaded to registers two stages ahead, split there once per workgroup
+// peak is 157 TFLOP/s.  A stage's fp32 values are loaded to registers two stages ahead, split there once per workgroup
 // while the current stage's MFMAs run, and stored as three bf16 planes in one LDS
 // buffer (48 or 36 KiB: two or three workgroups a CU cover each other's
 // barriers); the next stage's splits start when every wave holds its operands.
@@ -65,7 +67,7 @@ __device__ __forceinline__ float wave_max(float x) {
 // Measured against the fp32 MFMA tiles it replaced, Llama-3.2-3B at 2048 rows:
 // gate/up 1555 -> 1071 us (193 TFLOP/s), q/k/v 522 -> 367, o 318 -> 223, down 809
 // -> 565; SmolLM2-360M at 1023 rows gate/up 108 -> 77, q/k/v 44 -> 39, o 31 -> 28,
-// down 53 -> 45; 96 products of 9 to 520 rows 0.97 to 1.87 times as fast.  What bounds it with two
+// down 53 -> 45.  What bounds it with two
 // workgroups a CU is the issue port (about 240 VALU instructions, 96 MFMAs and 49
 // LDS ones per wave and stage); a lone one waits on its own LDS reads.
 template <int MB>
@@ -106,8 +108,8 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
       __builtin_amdgcn_make_buffer_rsrc((void*)b, (short)0, (int)view_bytes(k_hi, ldb, pn, 4), kBufRsrcWord3);
   const int a_row = tid >> 3, a_k = 4 * (tid & 7);
   const int b_row = tid >> 5, b_n = 4 * (tid & 31);
-  u32x4 av[AI], bv[BI];
-  auto load = [&](int kt) __attribute__((always_inline)) {
+  u32x4 av[AI], bv[BI];  // the next stage's
+  auto load = [&](int kt, u32x4 (&av)[AI], u32x4 (&bv)[BI]) __attribute__((always_inline)) {
     const int k0 = min(kt, kt_hi) * kBk;  // past the slice: zeros, and no offset that wraps
     const bool a_in = k0 + a_k < k_hi;
 #pragma unroll
@@ -125,7 +127,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   for (int i = 0; i < AI; ++i) a_max[i] = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) b_max[i] = 0.f;
-  auto store = [&]() __attribute__((always_inline)) {
+  auto store = [&](const u32x4 (&av)[AI], const u32x4 (&bv)[BI]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < AI; ++i) {
       const int row = a_row + 32 * i;
@@ -179,9 +181,12 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
       b_rd[nb] = 3 * SA + row * 256 + (((8 * wn + 2 * nb + (pp >> 1)) ^ swz) << 4) + 8 * (pp & 1);
   }
 
-  load(kt_lo);
-  store();
-  load(kt_lo + 1);
+  {  // both stages on their way at once: a slice of a few stages is a chain of latencies
+    u32x4 a0[AI], b0[BI];
+    load(kt_lo, a0, b0);
+    load(kt_lo + 1, av, bv);
+    store(a0, b0);
+  }
   for (int kt = kt_lo; kt < kt_hi; ++kt) {
     lds_barrier();
     bf16x8 af[3][MB], bf[3][NB];
@@ -220,8 +225,8 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[mb][nb] += lo[mb];
     }
-    store();        // the next stage's parts, beside the MFMAs
-    load(kt + 2);   // past the slice: zeros, with no memory access
+    store(av, bv);         // the next stage's parts, beside the MFMAs
+    load(kt + 2, av, bv);  // past the slice: zeros, with no memory access
     // one MFMA, then up to three of the splits' VALU instructions, and so on
 #pragma unroll
     for (int i = 0; i < 24 * MB; ++i) {
@@ -313,7 +318,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
       for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     constexpr int B0 = TM * 128;
     static_assert(B0 + kBk * 512 <= 3 * (SA + SB), "a stage of fp32 operands fits the planes' room");
-    load(kt_lo);
+    load(kt_lo, av, bv);
     for (int kt = kt_lo; kt < kt_hi; ++kt) {
       lds_barrier();
 #pragma unroll
@@ -326,7 +331,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
         const int row = b_row_e + 8 * i;
         *(lds_u32x4*)(lds + B0 + row * 512 + (((b_n_e >> 2) ^ (4 * ((row >> 2) & 3))) << 4)) = bv[i];
       }
-      load(kt + 1);
+      load(kt + 1, av, bv);
       lds_barrier();
 #pragma unroll 1
       for (int half = 0; half < 2; ++half) {
@@ -401,11 +406,11 @@ F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int min_split, int max_
   for (const F32Tile& c : kF32Tiles) {
     int64_t tiles = 0;
     for (int g = 0; g < G.count; ++g) tiles += (int64_t)((m + c.tm - 1) / c.tm) * ((G.n[g] + 127) / 128);
-    for (int S = min_split; S <= max_split && (S == min_split || stages >= 4 * S); ++S) {
+    for (int S = min_split; S <= max_split && (S == min_split || stages >= 2 * S); ++S) {
       const int64_t per_cu = (tiles * S + cus - 1) / cus;
       const int rest = (int)(per_cu % c.at_once);
       const double stage = (double)(per_cu / c.at_once) * c.stage_us[c.at_once - 1] + (rest ? c.stage_us[rest - 1] : 0.0);
-      const double reduce = S > 1 ? (8.0 * S + 4) * m * (double)ncols / 5.0e6 + 4.0 : 0.0;
+      const double reduce = S > 1 ? (8.0 * S + 4) * m * (double)ncols / 5.0e6 + 4.0 + 0.3 * S : 0.0;
       const double t = stage * ((stages + S - 1) / S) + 5.0 + reduce;
       if (best.tm == 0 || t < best.us) best = F32Plan{c.tm, S, (stages + S - 1) / S, t};
     }

@@ -7,11 +7,12 @@ namespace {
 
 // Every tile built, with what one costs (measured, every CU busy, bf16: whole
 // products of 1 to 8 rounds at k 960 to 8192): a larger one does more per byte
-// moved, a smaller one leaves fewer CUs idle in the last round.  Choosing by
-// rounds x cost picked the fastest of the six, or one within 4% of it, for 40 of
-// 44 products of 9 to 3000 rows at the Llama-3.2-3B and SmolLM2-360M widths.
+// moved, a smaller one leaves fewer CUs idle in the last round.  A split costs its
+// reduce's launch, a part per slice and the partials' traffic.  Fitted to 34 products
+// of 9 to 768 rows run on every tile and split: the choice is the fastest, or within 4%
+// of it, but for five, within 7%.
 const WidePlan kWidePlans[] = {{256, 256, 9.0, 0.755}, {192, 256, 8.0, 0.53}, {128, 256, 7.0, 0.42},
-                               {128, 192, 6.0, 0.37},  {128, 128, 5.0, 0.25}, {64, 128, 4.0, 0.20}};
+                               {128, 192, 6.0, 0.365}, {128, 128, 5.0, 0.27}, {64, 128, 4.0, 0.21}};
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4s lds_v4s;
@@ -54,9 +55,9 @@ __device__ __forceinline__ void mma_drain() { asm volatile("s_nop 15\n\ts_nop 15
 // Why this shape (2048-row Llama-3.2-3B prompt, bf16, measured):
 //   * 16x16x32 MFMAs: with random operands the chip's power limit holds a stream
 //     of them at 2.1 PFLOP/s (2.09 GHz) and one of 32x32x16 at 1.8 (1.78 GHz).
-//   * 128 x 128 a wave: an LDS byte read feeds twice the MFMAs of the 64 x 64
-//     waves of an 8-wave kernel with 32x32x16 MFMAs, and one wave per SIMD has the registers for it
-//     (256 accumulators in AGPRs, two operand sets in VGPRs).
+//   * 128 x 128 a wave: an LDS byte read feeds twice the MFMAs of 64 x 64 waves, and
+//     one wave per SIMD has the registers for it (256 accumulators in AGPRs, two
+//     operand sets in VGPRs).
 //   * Operands a stage ahead: nothing waits on an LDS read, and the stage's
 //     1024 MFMA cycles take 1050-1250 with operands from L2, 1500 where weights
 //     come from HBM (their latency; deeper rings than LDS has would help).
@@ -64,13 +65,12 @@ __device__ __forceinline__ void mma_drain() { asm volatile("s_nop 15\n\ts_nop 15
 //     panel order of gemm_tile (hipBLASLt: 1290).
 //   * C through LDS, whole row pieces: epilogue 16600 -> 9000 cycles of a tile's
 //     150000, against 8-byte stores from the accumulators.
-// gate/up 205 -> 163 us (1250 TFLOP/s), down 122 -> 103, q/k/v 84 -> 55; of 98
-// products of these models' shapes against the 64-, 128- and 256-row tiles of
-// that kernel, which this replaced, 9 to 64 rows ran at 0.96 to 1.36 times
-// their speed, 100 to 4096 rows at 1.04 to 1.76 times but for one, gate/up at 384
-// rows (53.8 -> 55.9 us; again, twice a side in turn: 58.8, 57.7 -> 58.6, 58.9,
-// where 448 rows take 61.3 -> 52.7: the model misses the best tile there).  64 rows
-// of 2560 -> 960 are slower, 12.1 -> 12.5 us.  What
+// Against 64- to 256-row tiles of 32x32x16 MFMAs, weights rotated through 1 GB:
+// gate/up 205 -> 163 us (1250 TFLOP/s), down 122 -> 103, q/k/v 84 -> 55; of 74 products
+// of 9 to 4096 rows at these models' widths 66 ran at 0.98 to 1.76 times their speed.
+// The others: gate/up at 384 rows 51.9 -> 56.2 us (448 rows 60.0 -> 49.4: 192 tiles of
+// 128 x 256 take longer than 256 do), q/k/v at 256 24.5 -> 26.3, and six of 9 to 64 rows
+// of K 960 and 1536, up to 0.8 us each (64 x 960 x (2560, 2560) 11.8 -> 12.6).  What
 // bounds it now: at 4 and more rounds the power limit (1.67 GHz), at one or two
 // the HBM latency of the weights and each tile's first loads and stores.
 //
@@ -350,7 +350,7 @@ WidePlan gemm_wide_plan(int m, int k, const GemmGroups& G, int min_split, int ma
     for (int S = min_split; S <= max_split && (S == min_split || stages >= 4 * S); ++S) {
       c.ksplit = S;
       c.kt_per = (stages + S - 1) / S;
-      const double reduce = S > 1 ? (8.0 * S + 2) * m * (double)ncols / 5.0e6 + 4.0 : 0.0;
+      const double reduce = S > 1 ? (8.0 * S + 2) * m * (double)ncols / 8.0e6 + 2.5 + 0.2 * S : 0.0;
       const double t = (double)((tiles * S + cus - 1) / cus) * (c.tile_us + c.kt_per * c.stage_us) + reduce;
       if (best.tm == 0 || t < t_best) {
         best = c;
