@@ -276,8 +276,9 @@ int tl_rope_kv_append(void* q, const void* k_new, const void* v_new,
  * the workspace.  The query gives 0 when no workspace is used.
  * Given less than the query asks for, the MFMA kernel runs whole-K instead
  * of failing; the skinny kernel needs its workspace.
- * C may overlap A or B only where K is split (the query's answer is not 0 and
- * the workspace holds it): every operand is then read before C is written.
+ * C may overlap A or B only where K is split (rows 16-byte aligned, the query's
+ * answer not 0 and a 16-byte-aligned workspace that holds it): every operand is
+ * then read before C is written.
  * ------------------------------------------------------------------------- */
 size_t tl_gemm_workspace_bytes(int m, int n, int k, int dtype);
 int tl_gemm(const void* a, const void* b, void* c, int m, int n, int k, int64_t lda,

@@ -19,8 +19,7 @@
 //     partial sums go to the workspace and skinny_reduce_kernel adds the
 //     K-slices and rounds to the output type.
 #include "tl_gemm.h"
-#include "tl_gemm_f32.h"
-#include "tl_gemm_wide.h"
+#include "tl_gemm_plan.h"
 
 using namespace tlg;
 
@@ -430,25 +429,6 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(GemmParams p) {
     }
 }
 
-// The plan of a product of more than kSkinnyMaxM rows on the matrix cores, with
-// min_split to max_split K-slices.
-struct PromptPlan {
-  WidePlan wide;  // 16-bit
-  int tm, tn, ksplit, kt_per;
-};
-
-PromptPlan prompt_plan(int m, int k, const GemmGroups& G, int esize, int min_split, int max_split) {
-  PromptPlan P{};
-  if (esize == 4) {
-    const F32Plan f = gemm_f32_plan(m, k, G, min_split, max_split);
-    P.tm = f.tm, P.tn = 128, P.ksplit = f.ksplit, P.kt_per = f.kt_per;
-  } else {
-    P.wide = gemm_wide_plan(m, k, G, min_split, max_split);
-    P.tm = P.wide.tm, P.tn = P.wide.tn, P.ksplit = P.wide.ksplit, P.kt_per = P.wide.kt_per;
-  }
-  return P;
-}
-
 // K-slices whose fp32 partials are about half as large as B in 16 bits, as large as
 // B in fp32: B is what a product of few rows streams.
 int few_rows_split(int m, int k, int esize) {
@@ -462,11 +442,38 @@ int max_split(int m, int k, int esize) {
   return few > kMaxSplit ? kMaxSplit : few > least ? few : least;
 }
 
-size_t split_bytes(int m, const GemmGroups& G, int ksplit) {
+PromptPlan prompt_plan(int m, int k, const GemmGroups& G, int esize, int min_split, int max_split) {
+  PromptPlan P{};
+  if (esize == 4) {
+    const F32Plan f = gemm_f32_plan(m, k, G, min_split, max_split);
+    P.tm = f.tm, P.tn = 128, P.ksplit = f.ksplit, P.kt_per = f.kt_per;
+  } else {
+    P.wide = gemm_wide_plan(m, k, G, min_split, max_split);
+    P.tm = P.wide.tm, P.tn = P.wide.tn, P.ksplit = P.wide.ksplit, P.kt_per = P.wide.kt_per;
+  }
+  return P;
+}
+
+}  // namespace
+
+namespace tlg {
+
+PromptPlan gemm_prompt_plan(int m, int k, const GemmGroups& G, int esize, bool in_place, bool workspace) {
+  const int most = workspace ? max_split(m, k, esize) : 1;
+  const PromptPlan P = prompt_plan(m, k, G, esize, 1, most);
+  // exactly two: the workspace query's room where it counts on one
+  return in_place && P.ksplit == 1 && most > 1 ? prompt_plan(m, k, G, esize, 2, 2) : P;
+}
+
+size_t gemm_split_bytes(int m, const GemmGroups& G, int ksplit) {
   size_t ncols = 0;
   for (int g = 0; g < G.count; ++g) ncols += (size_t)G.n[g];
   return ksplit > 1 ? (size_t)ksplit * m * ncols * sizeof(float) : 0;
 }
+
+}  // namespace tlg
+
+namespace {
 
 // Whether an output shares bytes with A or with a B.  Such a product comes out
 // right where K is cut: every operand is read before the reduce pass writes the
@@ -504,11 +511,10 @@ int launch_gemm(const void* a, const GemmGroups& G, int m, int k, int64_t lda, v
     widest = G.n[g] > widest ? G.n[g] : widest;
   }
   if (aligned) {
-    const int most = max_split(m, k, (int)esize);
-    PromptPlan P = prompt_plan(m, k, G, (int)esize, in_place && most > 1 ? 2 : 1, most);
+    PromptPlan P = gemm_prompt_plan(m, k, G, (int)esize, in_place);
     if (P.ksplit > 1 &&
-        (!workspace || workspace_bytes < split_bytes(m, G, P.ksplit) || ((uintptr_t)workspace % 16) != 0))
-      P = prompt_plan(m, k, G, (int)esize, 1, 1);
+        (!workspace || workspace_bytes < gemm_split_bytes(m, G, P.ksplit) || ((uintptr_t)workspace % 16) != 0))
+      P = gemm_prompt_plan(m, k, G, (int)esize, in_place, false);
     // columns of one store: 16 bytes from the kernels, 4 from the reduce
     const int run = P.ksplit > 1 || esize == 4 ? 4 : 8;
     p.tiles_m = (m + P.tm - 1) / P.tm;
@@ -629,8 +635,8 @@ size_t groups_workspace_bytes(int m, int k, const GemmGroups& G, int dtype) {
   // where they are cheap, for a C that overlaps A or B (a product that falls back to
   // the simple kernel uses none of it)
   if (m <= kSkinnyMaxM) return skinny_workspace_bytes(m, live, k, esize);
-  const int chosen = prompt_plan(m, k, live, esize, 1, max_split(m, k, esize)).ksplit;
-  return split_bytes(m, live, chosen > 1 ? chosen : few_rows_split(m, k, esize) > 1 ? 2 : 1);
+  const int chosen = gemm_prompt_plan(m, k, live, esize, false).ksplit;
+  return gemm_split_bytes(m, live, chosen > 1 ? chosen : few_rows_split(m, k, esize) > 1 ? 2 : 1);
 }
 
 }  // namespace
