@@ -1,13 +1,17 @@
 """The plans of the matrix-core products (csrc/tl_gemm_plan.h), on the CPU: what
-the workspace query answers holds the plan that launches.  A small host program calls
-the built library's plan functions; they need no device (256 CUs, or the cap)."""
+the workspace query answers holds the plan that launches, and the GPU tests'
+shapes reach every tile, whole and with K split.  A small host program calls the
+built library's plan functions; they need no device (256 CUs, or the cap)."""
 
 import os
+import re
 import shutil
 import subprocess
 
 import numpy as np
 import pytest
+
+from tests import test_gpu_gemm as tg
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "triton-llm_amd", "csrc")
@@ -56,6 +60,11 @@ def plans(tmp_path_factory):
     return run
 
 
+def _shapes(test):  # (M, K, Ns, cus) of the test's parameters; no cap where it sets none
+    (mark,) = [m for m in test.pytestmark if m.name == "parametrize" and m.args[0].startswith("M,K,Ns")]
+    return [tuple(p) + (0,) * (4 - len(p)) for p in mark.args[1]]
+
+
 @pytest.mark.parametrize("esize", [2, 4])
 def test_query_holds_the_plan(plans, esize):
     rng = np.random.default_rng(esize)
@@ -68,3 +77,19 @@ def test_query_holds_the_plan(plans, esize):
             assert query == b, case
         if query > 0:  # then a C that overlaps A or B is cut, within that room
             assert s_in > 1 and b_in <= query, case
+
+
+def test_gpu_shapes_reach_every_wide_tile(plans):
+    cases = [(m, k, ns, 2, cus) for m, k, ns, cus in _shapes(tg.test_gemm_wide_tiles)]
+    got = {(tm, tn, s > 1) for tm, tn, s, *_ in plans(cases)}
+    with open(os.path.join(CSRC, "tl_gemm_wide.hip")) as f:  # the tiles of its table
+        table = re.search(r"kWidePlans\[\] = \{(.*?)\};", f.read(), re.S).group(1)
+    tiles = {(int(tm), int(tn)) for tm, tn in re.findall(r"\{(\d+), (\d+),", table)}
+    assert len(tiles) == 6 and got == {(*t, split) for t in tiles for split in (False, True)}
+
+
+@pytest.mark.parametrize("test", [tg.test_gemm_prompt_fp32_plans, tg.test_gemm_fp32_parts_tiles,
+                                  tg.test_gemm_fp32_outliers])
+def test_gpu_shapes_reach_both_fp32_tiles(plans, test):
+    got = {(tm, s > 1) for tm, _, s, *_ in plans([(m, k, ns, 4, cus) for m, k, ns, cus in _shapes(test)])}
+    assert got == {(tm, split) for tm in (64, 128) for split in (False, True)}

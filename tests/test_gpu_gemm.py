@@ -202,13 +202,14 @@ def test_gemm_prompt_split_k(dtype, M, K, Ns):
 
 
 @pytest.mark.parametrize("M,K,Ns", [(2048, 960, (960, 320, 320)), (2048, 960, (960,)), (2048, 960, (320,)),
-                                   (2000, 2560, (960,)), (1999, 964, (2560, 2560))])
-def test_gemm_prompt_fp32_64_row_plans(M, K, Ns):
-    """fp32 prompt products with few 128-row tiles per CU (SmolLM2-360M's
-    projections at a 2048-token prompt) run 64-row tiles, whole-K or with K
-    split in 2-4: the grouped q/k/v, o / down with their splits, ragged M and
-    a K tail inside a 16-k stage."""
-    print(f"[case] gemm fp32 64-row {M}x{K} -> {Ns}", flush=True)
+                                   (2000, 2560, (960,)), (1999, 964, (2560, 2560)), (1600, 960, (2560,)),
+                                   (1999, 964, (648,))])
+def test_gemm_prompt_fp32_plans(M, K, Ns):
+    """fp32 prompt products of SmolLM2-360M's projections at about 2048 tokens:
+    128- and 64-row tiles, whole-K and with K split (test_gemm_plans.py checks
+    that both are reached): the grouped q/k/v, o / down with their splits, ragged
+    M and a K tail inside a 32-k stage."""
+    print(f"[case] gemm fp32 prompt {M}x{K} -> {Ns}", flush=True)
     rng = np.random.default_rng(M + 5 * K + sum(Ns))
     a = rng.standard_normal((M, K), dtype=np.float32)
     bs = [rng.standard_normal((K, n), dtype=np.float32) / np.float32(np.sqrt(K)) for n in Ns]
@@ -219,7 +220,7 @@ def test_gemm_prompt_fp32_64_row_plans(M, K, Ns):
         outs = gemm_grouped(a_dev, [gpu.to_device(b) for b in bs])
     for b, o in zip(bs, outs):
         err = H.max_abs(H.download(o), gemm_ref(a, b))
-        H.report(f"fp32 64-row {M}x{K}@{K}x{b.shape[1]}", err, 2e-3)
+        H.report(f"fp32 prompt {M}x{K}@{K}x{b.shape[1]}", err, 2e-3)
         assert err <= 2e-3
 
 
@@ -410,8 +411,9 @@ def test_gemm_zero_k_strided_output_keeps_padding():
     assert not c2h[:, :8].any() and (c2h[:, 8:] == 7.0).all()
 
 
-# The 16-bit prompt kernel's tiles (64 x 128 to 256 x 256), each reached by
-# capping the CUs the plan counts rounds for: ragged last rows and columns, odd
+# The 16-bit prompt kernel's tiles (64 x 128 to 256 x 256), each reached, whole and
+# with K split, by capping the CUs the plan counts rounds for
+# (test_gemm_plans.py checks that they are): ragged last rows and columns, odd
 # and even counts of 32-k stages, k tails of 8, 16 and 24, one stage, groups; NaN
 # past k in A's padding, past n in B's. Tolerance as above: the output's rounding.
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
@@ -420,7 +422,10 @@ def test_gemm_zero_k_strided_output_keeps_padding():
     (300, 136, (584,), 16), (300, 136, (584, 200), 5), (193, 1000, (400,), 1), (193, 1000, (400,), 2),
     (130, 264, (328,), 4),
     (449, 72, (776,), 3), (449, 72, (776,), 256), (257, 24, (264,), 1), (65, 32, (8,), 256), (16, 8, (136,), 256),
-    (1025, 64, (256,), 2)])
+    (1025, 64, (256,), 2), (300, 136, (584,), 5), (300, 136, (584,), 9),
+    # with K split, every tile again
+    (193, 2000, (400,), 6), (130, 1000, (400,), 4), (193, 2000, (400,), 12), (130, 2000, (328,), 16),
+    (130, 2000, (328,), 12), (130, 1000, (328,), 24)])
 def test_gemm_wide_tiles(monkeypatch, dtype, M, K, Ns, cus):
     print(f"[case] gemm wide {dtype} {M}x{K} -> {Ns} cus {cus}", flush=True)
     H.set_override(monkeypatch, "TRITON_LLM_HIP_MAX_CUS", cus)
