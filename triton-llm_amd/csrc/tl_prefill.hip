@@ -991,26 +991,26 @@ __global__ __launch_bounds__(kThreads, D == 128 ? 1 : 2) void flash_fwd_f32(Flas
 // ---------------------------------------------------------------------------
 constexpr int KS_ROWS = 32;  // query rows per workgroup
 constexpr int KS_KEYS = 32;  // keys per chunk
-// 128-row blocks below which the keys are split: at half the CUs the tiled
-// kernel's blocks, a CU each, still take as long as their longest chain.  Causal,
-// key-split against tiled: 15 heads of d_k 64 at 700 / 1023 tokens (90 / 120
-// blocks) 40.7 / 41.5 against 59.2 / 83.6 us, 9 heads at 1500 (108) 67 / 123, 24
-// heads of d_k 128 at 400 (96) 47.6 / 69.2; at 192 blocks and d_k 128 it loses
-// (175 / 157), non-causal from 144 blocks on (135 / 109 us, 24 heads at 700).
-constexpr int KS_SMALL_GRID = 128;
+// Taken below a 128-row block for every second CU: the tiled kernel's blocks, a CU each,
+// then take as long as their longest chain whatever their number.  Measured against
+// it at 60 to 240 blocks (256 CUs), 9 to 96 heads of d_k 64, 24 of d_k 128: below 128
+// blocks 1.28 to 2.1 times its speed causal and 1.11 to 2.2 not (96 blocks of 64 tokens
+// 1.03), 15 heads at 960 tokens (120) 76.6 against 48.3 us; from 135 to 189 causal
+// 1.21 to 1.82, not causal 0.81 to 1.37, where the line would need both; at 192 and
+// more down to 0.86 and 0.63 (24 heads of d_k 128 at 960 143.7 against 147.4 us).
 template <int D, bool CAUSAL>
-__global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p) {
+__global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p, int cus) {
   constexpr int NDB = D / 32;
   constexpr int NC = D / 8;  // 16-byte chunks per lane half
   __shared__ float s_ml[4][2][KS_ROWS];
   __shared__ float s_o[3][NDB][16][64];  // waves 1..3's O^T accumulators, lane-minor (no bank conflicts)
 
   const int n_rb = (p.seq_q + KS_ROWS - 1) / KS_ROWS;
-  // Longest blocks first in the heads of the first 256 workgroups, shortest first
+  // Longest blocks first in the heads of the first workgroup of every CU, shortest first
   // in those of the next, and so on: the second workgroup a CU gets then evens
   // out the first (15 heads, 1023 tokens: 60.8 -> 41.5 us).
   const int head = (int)(blockIdx.x / n_rb), at = (int)(blockIdx.x % n_rb);
-  const int rb = (head * n_rb / 256) & 1 ? at : n_rb - 1 - at;
+  const int rb = (head * n_rb / cus) & 1 ? at : n_rb - 1 - at;
   const int hq = head % p.n_head;
   const int b = head / p.n_head;
   const int hkv = hq / p.group;
@@ -1655,13 +1655,14 @@ template <int D>
 int launch_flash_f32(FlashParams& p, bool causal, hipStream_t st) {
   p.n_qt = (p.seq_q + BM - 1) / BM;
   const int64_t blocks = (int64_t)p.n_qt * p.n_head * p.batch;
-  if (blocks < KS_SMALL_GRID) {
+  const int cus = tl_device_cus();
+  if (blocks < cus / 2) {
     // few 128-row blocks: split each 32-row block's keys over 4 waves
     dim3 g((unsigned)((int64_t)((p.seq_q + KS_ROWS - 1) / KS_ROWS) * p.n_head * p.batch));
     if (causal)
-      hipLaunchKernelGGL((flash_fwd_f32_ks<D, true>), g, dim3(kThreads), 0, st, p);
+      hipLaunchKernelGGL((flash_fwd_f32_ks<D, true>), g, dim3(kThreads), 0, st, p, cus);
     else
-      hipLaunchKernelGGL((flash_fwd_f32_ks<D, false>), g, dim3(kThreads), 0, st, p);
+      hipLaunchKernelGGL((flash_fwd_f32_ks<D, false>), g, dim3(kThreads), 0, st, p, cus);
     return tl_launch_status();
   }
   dim3 grid((unsigned)blocks);
