@@ -490,13 +490,13 @@ def cpu_decode_baseline(cfg, data, oa, on, budget_s=10.0):
 # ---------------------------------------------------------------------------
 
 def prefill_kernel_name(cfg):
-    """The kernels tl_attention_fwd runs for a prefill config: fp32 takes the
-    key-split kernel when fewer than 64 blocks of 128 query rows would run;
-    16-bit d_k 128 reads V through the vt_pack copy."""
+    """The kernel tl_attention_fwd runs for a prefill config: fp32 takes the
+    key-split kernel when fewer blocks of 128 query rows than half the 256 CUs
+    would run; the 16-bit kernel reads V in place."""
     if cfg.dtype == "float32":
         blocks = -(-cfg.seq // 128) * cfg.n_head * cfg.batch
-        return "flash_fwd_f32_ks" if blocks < 64 else "flash_fwd_f32"
-    return "flash_fwd_16 + vt_pack_kernel" if cfg.d_k == 128 else "flash_fwd_16"
+        return "flash_fwd_f32_ks" if blocks < 128 else "flash_fwd_f32"
+    return "flash_fwd_16"
 
 
 def bench_prefill(cfg, steps, warmup, replicas=1, cpu=True, cpu_budget_s=10.0, ramp_ms=0.0):
@@ -531,7 +531,7 @@ def bench_prefill(cfg, steps, warmup, replicas=1, cpu=True, cpu_budget_s=10.0, r
         q, k, v, out = sets[i % replicas]
         flash_attention(q, k, v, causal=True, sm_scale=cfg.scale, out=out, workspace=ws)
 
-    # one recorded launcher (V^T staging + flash kernel) per input replica
+    # one recorded launcher per input replica
     from triton_llm.kernels._common import record
 
     for i in range(replicas):
