@@ -370,3 +370,24 @@ def test_prefill_output_over_v(dtype, causal):
         flash_attention(qd, kd, vd, causal=causal, out=vd)
         got = on.from_storage(H.download(vd), dtype)
         compare(f"over v {dtype}", got, on.from_storage(apart, dtype), TOL[dtype])
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("d_k", [64, 128])
+@pytest.mark.parametrize("s", [1, 31, 33, 100, 128, 161])
+def test_prefill_fp32_key_split_ends(d_k, s, causal):
+    """The fp32 key-split kernel on rows that end inside a chunk of 32 keys, NaN
+    behind them in the same allocation: nothing of it may reach an output."""
+    print(f"[case] fp32 key split ends d_k={d_k} s={s} causal={causal}", flush=True)
+    h, rng = 3, np.random.default_rng(s + d_k)
+    parents = [np.full((h, s + 40, d_k), np.nan, np.float32) for _ in range(3)]
+    for x in parents:
+        x[:, :s] = rng.standard_normal((h, s, d_k), dtype=np.float32)
+    dev = [gpu.to_device(x) for x in parents]
+    out = gpu.to_device(np.full((h, s, d_k), 7.0, np.float32))
+    st = (0, (s + 40) * d_k, d_k)
+    flash_attention_strided(*dev, out, batch=1, n_head=h, n_kv_head=h, seq_q=s, seq_k=s, d_k=d_k, q_strides=st,
+                            k_strides=st, v_strides=st, o_strides=(0, s * d_k, d_k), causal=causal)
+    q, k, v = (x[None, :, :s] for x in parents)
+    exp = oa.attention_bhsd(q, k, v, causal=causal, dtype="float32")
+    compare(f"fp32 key split s {s}", H.download(out)[None], exp, TOL["float32"])

@@ -993,11 +993,17 @@ constexpr int KS_ROWS = 32;  // query rows per workgroup
 constexpr int KS_KEYS = 32;  // keys per chunk
 // Taken below a 128-row block for every second CU: the tiled kernel's blocks, a CU each,
 // then take as long as their longest chain whatever their number.  Measured against
-// it at 60 to 240 blocks (256 CUs), 9 to 96 heads of d_k 64, 24 of d_k 128: below 128
-// blocks 1.28 to 2.1 times its speed causal and 1.11 to 2.2 not (96 blocks of 64 tokens
-// 1.03), 15 heads at 960 tokens (120) 76.6 against 48.3 us; from 135 to 189 causal
-// 1.21 to 1.82, not causal 0.81 to 1.37, where the line would need both; at 192 and
-// more down to 0.86 and 0.63 (24 heads of d_k 128 at 960 143.7 against 147.4 us).
+// it at 60 to 240 blocks (256 CUs), 9 to 96 heads of d_k 64, 24 and 192 of d_k 128:
+// below 128 blocks 1.48 to 2.6 times its speed causal and 1.31 to 2.6 not (96 blocks of
+// 64 tokens 1.06); from 135 to 198 still 1.09 to 2.1 causal, but 0.73 to 1.5 not and
+// 0.86 at 64 tokens; at 240 1.14 and 0.78.  15 heads at 960 tokens (120) 76.6 against
+// 42.0 us.
+//
+// One workgroup a CU and little to overlap: bound by the first loads' latency and the
+// MFMA chain.  12 heads at 128 tokens 8.6 -> 7.7 us and 15 at 1023 37.2 -> 30.6 when
+// the branches around the loads went; the next chunk's loads ahead of this one's MFMAs
+// gained nothing (12 heads at 256 tokens 10.8 -> 11.2, 15 at 1023 35.5 -> 37.2): this
+// one's V then has to arrive before its first MFMA.
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p, int cus) {
   constexpr int NDB = D / 32;
@@ -1006,11 +1012,11 @@ __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p, int 
   __shared__ float s_o[3][NDB][16][64];  // waves 1..3's O^T accumulators, lane-minor (no bank conflicts)
 
   const int n_rb = (p.seq_q + KS_ROWS - 1) / KS_ROWS;
-  // Longest blocks first in the heads of the first workgroup of every CU, shortest first
-  // in those of the next, and so on: the second workgroup a CU gets then evens
-  // out the first (15 heads, 1023 tokens: 60.8 -> 41.5 us).
+  // Longest blocks first in the heads of each CU's first workgroup, shortest first in
+  // those of its second (there is no third: KS_ROWS x 4 rows to a block): they even
+  // out (15 heads, 1023 tokens: 60.8 -> 41.5 us).
   const int head = (int)(blockIdx.x / n_rb), at = (int)(blockIdx.x % n_rb);
-  const int rb = (head * n_rb / cus) & 1 ? at : n_rb - 1 - at;
+  const int rb = head * n_rb >= cus ? at : n_rb - 1 - at;
   const int hq = head % p.n_head;
   const int b = head / p.n_head;
   const int hkv = hq / p.group;
@@ -1030,10 +1036,7 @@ __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p, int 
   {
     const float* qrow = (const float*)p.q + b * p.q_sb + hq * p.q_sh + (int64_t)min(qi, p.seq_q - 1) * p.q_ss;
 #pragma unroll
-    for (int cc = 0; cc < NC; ++cc) {
-      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      qf[cc] = qi < p.seq_q ? *(const f32x4*)(qrow + h * (D / 2) + 4 * cc) : z;
-    }
+    for (int cc = 0; cc < NC; ++cc) qf[cc] = *(const f32x4*)(qrow + h * (D / 2) + 4 * cc);
   }
   f32x16 o_acc[NDB];
 #pragma unroll
@@ -1045,45 +1048,26 @@ __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p, int 
   const float* kbase = (const float*)p.k + b * p.k_sb + hkv * p.k_sh;
   const float* vbase = (const float*)p.v + b * p.v_sb + hkv * p.v_sh;
   const float c = p.scale_log2;
-  // K^T operand: lane (lq, h) holds key kb + lq, d = h D/2 + 4 cc + i;
-  // V^T operand of step r: key kb + 8 (r / 4) + 4 h + r % 4, d = 32 db + lq.
-  auto load_chunk = [&](int kb, f32x4 (&kf)[NC], float (&vf)[16][NDB]) __attribute__((always_inline)) {
-    const int key = kb + lq;
-    const float* krow = kbase + (int64_t)min(key, p.seq_k - 1) * p.k_ss + h * (D / 2);
-#pragma unroll
-    for (int cc = 0; cc < NC; ++cc) {
-      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      kf[cc] = key < p.seq_k ? *(const f32x4*)(krow + 4 * cc) : z;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kv = kb + 8 * (r >> 2) + 4 * h + (r & 3);
-      const float* vrow = vbase + (int64_t)min(kv, p.seq_k - 1) * p.v_ss + lq;
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) vf[r][db] = kv < p.seq_k ? vrow[32 * db] : 0.f;
-    }
-  };
-  // d_k 64: the wave's next chunk is loaded while this one's MFMAs run (the
-  // registers of two chunks fit beside the accumulators; at d_k 128 they do not):
-  // 3% to 10% off, and 25% where a CU holds two workgroups.
-  constexpr bool AHEAD = D == 64;
-  f32x4 kn[NC];
-  float vn[16][NDB];
-  if (AHEAD && wave < n_ch) load_chunk(wave * KS_KEYS, kn, vn);
   for (int ch = wave; ch < n_ch; ch += 4) {
     const int kb = ch * KS_KEYS;
+    // K^T operand: lane (lq, h) holds key kb + lq, d = h D/2 + 4 cc + i;
+    // V^T operand of step r: key kb + 8 (r / 4) + 4 h + r % 4, d = 32 db + lq.
+    // Every load is made, from the last row past the end (a branch around each kept the
+    // first MFMA behind V's): those keys' scores are masked and their V made zeros
+    // below, and rows of Q past the end are not stored.
     f32x4 kf[NC];
     float vf[16][NDB];
-    if constexpr (AHEAD) {
+    {
+      const float* krow = kbase + (int64_t)min(kb + lq, p.seq_k - 1) * p.k_ss + h * (D / 2);
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) kf[cc] = kn[cc];
+      for (int cc = 0; cc < NC; ++cc) kf[cc] = *(const f32x4*)(krow + 4 * cc);
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
+      for (int r = 0; r < 16; ++r) {
+        const int kv = kb + 8 * (r >> 2) + 4 * h + (r & 3);
+        const float* vrow = vbase + (int64_t)min(kv, p.seq_k - 1) * p.v_ss + lq;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) vf[r][db] = vn[r][db];
-      if (ch + 4 < n_ch) load_chunk(kb + 4 * KS_KEYS, kn, vn);
-    } else {
-      load_chunk(kb, kf, vf);
+        for (int db = 0; db < NDB; ++db) vf[r][db] = vrow[32 * db];
+      }
     }
     f32x16 s;
 #pragma unroll
@@ -1116,6 +1100,13 @@ __global__ __launch_bounds__(kThreads) void flash_fwd_f32_ks(FlashParams p, int 
       const float e = fast_exp2(s[r] - base);
       s[r] = e;
       l_run += e;
+    }
+    if (kb + KS_KEYS > p.seq_k) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+          if (kb + 8 * (r >> 2) + 4 * h + (r & 3) >= p.seq_k) vf[r][db] = 0.f;
     }
     // O^T += V^T . P^T: step r uses key 8 (r / 4) + 4 h + r % 4 of the chunk
     // in lane half h (MFMA k = h), so P^T is the lane's own S value.
