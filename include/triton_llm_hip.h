@@ -267,13 +267,11 @@ int tl_rope_kv_append(void* q, const void* k_new, const void* v_new,
  * :360-363, :375).  k = 0 writes zeros; m = 0 or n = 0 does nothing.
  * m <= 8 (a decoded token) runs a hand-written HBM-streaming kernel whose
  * K-slice partial sums need tl_gemm_workspace_bytes(m, n, k, dtype) bytes of
- * workspace; larger m runs a hand-written MFMA kernel (128 x 128 tiles of
- * C, or 256 x 256 for large 16-bit products; rows of A and B must be
+ * workspace; larger m runs a hand-written MFMA kernel (rows of A and B must be
  * 16-byte aligned, otherwise a simple FMA kernel takes the product), which
- * for fp32 products that leave CUs unevenly loaded, and for products of
- * any dtype with fewer than two tiles per CU (a batch of decoded tokens:
- * at most 64 rows take 64 x 128 tiles), splits K and keeps fp32 partials in
- * the workspace.  The query gives 0 when no workspace is used.
+ * splits K where its tiles of C would leave CUs idle (a batch of decoded
+ * tokens, fp32 prompts of few tiles) and keeps fp32 partials in the
+ * workspace.  The query gives 0 when no workspace is used.
  * Given less than the query asks for, the MFMA kernel runs whole-K instead
  * of failing; the skinny kernel needs its workspace.
  * C may overlap A or B only where K is split (rows 16-byte aligned, the query's

@@ -66,15 +66,17 @@ __device__ __forceinline__ void mma_drain() { asm volatile("s_nop 15\n\ts_nop 15
 //   * C through LDS, whole row pieces: epilogue 16600 -> 9000 cycles of a tile's
 //     150000, against 8-byte stores from the accumulators.
 // Against 64- to 256-row tiles of 32x32x16 MFMAs, weights rotated through 1 GB:
-// gate/up 205 -> 163 us (1250 TFLOP/s), down 122 -> 103, q/k/v 84 -> 55; of 74 products
-// of 9 to 4096 rows at these models' widths 66 ran at 0.98 to 1.76 times their speed.
-// The others: gate/up at 384 rows 51.9 -> 56.2 us (448 rows 60.0 -> 49.4: 192 tiles of
+// gate/up 205 -> 162 us (1270 TFLOP/s), down 141 -> 118, q/k/v 102 -> 65; 64 rows
+// gate/up 28.2 -> 26.5, down 24.2 -> 20.3; of 74 products of 9 to 4096 rows at these
+// models' widths 66 ran at 0.98 to 1.76 times their speed.  The others: gate/up at 384
+// rows 51.9 -> 56.2 us, 55.7 -> 56.3 when repeated (448 rows 60.0 -> 49.4: 192 tiles of
 // 128 x 256 take longer than 256 do), q/k/v at 256 24.5 -> 26.3, and six of 9 to 64 rows
-// of K 960 and 1536, up to 0.8 us each (64 x 960 x (2560, 2560) 11.8 -> 12.6).  What
+// of K 960 and 1536, up to 1 us each (64 x 960 x (2560, 2560) 12.1 -> 13.1).  What
 // bounds it now: at 4 and more rounds the power limit (1.67 GHz), at one or two
 // the HBM latency of the weights and each tile's first loads and stores.
 //
-// LDS layouts (16-byte chunks, XOR-swizzled; no bank conflict in the counters):
+// LDS layouts (16-byte chunks, XOR-swizzled; the counters show conflicts in 25% to 35% of
+// the LDS cycles, behind reads made a stage ahead):
 //   A: rows (m) of 64 bytes (k), chunk c of row r at slot c ^ ((r >> 2) & 3); lane
 //      (l % 16, g = l / 16) reads 8 consecutive k of row l % 16: chunk g.
 //   B: rows (k) of 64 NB bytes (n), chunk c of row r at slot c ^ b_swz(r): the
