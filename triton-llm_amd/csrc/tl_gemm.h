@@ -65,16 +65,26 @@ __device__ __forceinline__ bool gemm_tile(const GemmParams& p, int& grp, int& tm
   const int it = (L % 8) * p.per_xcd + L / 8;
   const int tiles = p.G.tile0[p.G.count];
   if (it >= tiles * p.ksplit) return false;
-  ks = it / tiles;
+  ks = p.ksplit > 1 ? it / tiles : 0;
   const int t = it - ks * tiles;
   grp = find_group(p.G.tile0, p.G.count, t);
   const int local = t - p.G.tile0[grp];
-  const int tiles_n = (p.G.tile0[grp + 1] - p.G.tile0[grp]) / p.tiles_m;
-  const int panel = local / (kPanelRows * tiles_n);
-  const int in = local - panel * kPanelRows * tiles_n;
-  const int h = min(kPanelRows, p.tiles_m - panel * kPanelRows);
-  tm = panel * kPanelRows + in % h;
-  tn = in / h;
+  // no more divisions than the height needs: each is a chain of some 30 instructions
+  // ahead of the first load
+  if (p.tiles_m == 1) {
+    tm = 0;
+    tn = local;
+  } else if (p.tiles_m <= kPanelRows) {
+    tn = local / p.tiles_m;
+    tm = local - tn * p.tiles_m;
+  } else {
+    const int tiles_n = (p.G.tile0[grp + 1] - p.G.tile0[grp]) / p.tiles_m;
+    const int panel = local / (kPanelRows * tiles_n);
+    const int in = local - panel * kPanelRows * tiles_n;
+    const int h = min(kPanelRows, p.tiles_m - panel * kPanelRows);
+    tm = panel * kPanelRows + in % h;
+    tn = in / h;
+  }
   return true;
 }
 
