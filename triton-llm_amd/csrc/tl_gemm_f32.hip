@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   constexpr int TM = 32 * MB, TN = 128, NB = 4;
   constexpr int SA = TM * 64, SB = kBk * 256;  // bytes of one plane of a stage
   __shared__ __attribute__((aligned(1024))) char smem[3 * (SA + SB)];
-  __shared__ float s_row[TM], s_col[8][TN], s_max[4], s_least[4];
+  __shared__ float s_row[TM], s_col[8][TN], s_max[4], s_amax[4], s_bmax[4], s_least[4];
 
   int grp, tm, tn, ks;
   if (!gemm_tile(p, grp, tm, tn, ks)) return;
@@ -248,20 +248,22 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
   // the tile through the fp32 MFMA: a row of A or a column of B whose largest
   // magnitude is not between 2^-40 and 2^60 (NaN and infinity included; all zeros are
   // fine), and a sum below 2^-44 of its row's largest times its column's, which may
-  // be made of entries below 2^-102 alone (above it they weigh k 2^-42 at most).  The
-  // look at the sums costs 0.5 us a product, 1.4% of a SmolLM2-360M layer.
+  // be made of entries below 2^-102 alone (above it they weigh k 2^-42 at most).
+  // First by what needs no exchange but the tile's largest magnitudes: every
+  // thread's own largest in range, the tile's smallest sum against them.  The rows and
+  // columns one by one only where that falls short, which took 0.5 us a product.
+  float a_most = 0.f, b_most = 0.f, least = INFINITY;
+  bool fine = true;
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
-    float v = a_max[i];
-#pragma unroll
-    for (int o = 4; o >= 1; o >>= 1) v = __builtin_elementwise_maximum(v, __shfl_xor(v, o));
-    if ((tid_e & 7) == 0) s_row[a_row_e + 32 * i] = v;
+    a_most = fmaxf(a_most, a_max[i]);
+    fine &= a_max[i] == 0.f || (a_max[i] >= 0x1p-40f && a_max[i] <= 0x1p60f);
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) s_col[b_row_e][b_n_e + e] = b_max[e];
-  // The tile's smallest sum against its largest row's and column's magnitudes; the
-  // sums one by one only where that falls short.
-  float least = INFINITY;
+  for (int e = 0; e < 4; ++e) {
+    b_most = fmaxf(b_most, b_max[e]);
+    fine &= b_max[e] == 0.f || (b_max[e] >= 0x1p-40f && b_max[e] <= 0x1p60f);
+  }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -270,39 +272,60 @@ __global__ __launch_bounds__(256, MB == 2 ? 3 : 2) void gemm_f32_kernel(GemmPara
       const bool inside = m_tile + m_e + 16 * mb + lc_e < p.m && n_tile + n_e + 16 * nb + 4 * g_e < pn;
       least = fminf(least, inside ? fminf(fminf(fabsf(c[0]), fabsf(c[1])), fminf(fabsf(c[2]), fabsf(c[3]))) : INFINITY);
     }
-  __syncthreads();
-  float v = 0.f;  // waves 0 and 1: a row's largest magnitude, 2 and 3: a column's
-  if (tid_e < TM) {
-    v = s_row[tid_e];
-  } else if (tid_e >= 128) {
-    v = s_col[0][tid_e - 128];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) v = __builtin_elementwise_maximum(v, s_col[i][tid_e - 128]);
-    if (n_tile + tid_e - 128 >= pn) v = 0.f;  // columns past n hold the next row's values
-    s_col[0][tid_e - 128] = v;
-  }
-  const bool in_range = __all(v == 0.f || (v >= 0x1p-40f && v <= 0x1p60f));
-  v = wave_max(v);
+  fine = __all(fine);
+  a_most = wave_max(a_most);
+  b_most = wave_max(b_most);
   least = -wave_max(-least);
   if ((tid_e & 63) == 0) {
-    s_max[wave_e] = in_range ? v : INFINITY;
+    s_amax[wave_e] = fine ? a_most : INFINITY;
+    s_bmax[wave_e] = b_most;
     s_least[wave_e] = least;
   }
   __syncthreads();
-  const float most = fmaxf(s_max[0], s_max[1]) * 0x1p-44f * fmaxf(s_max[2], s_max[3]);
-  bool plain = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3])) == INFINITY;
-  if (!plain && fminf(fminf(s_least[0], s_least[1]), fminf(s_least[2], s_least[3])) < most) {
-    float short_of = 0.f;  // by how much a sum falls short of its bound, at most
+  const float a_all = fmaxf(fmaxf(s_amax[0], s_amax[1]), fmaxf(s_amax[2], s_amax[3]));
+  const float b_all = fmaxf(fmaxf(s_bmax[0], s_bmax[1]), fmaxf(s_bmax[2], s_bmax[3]));
+  const float least_all = fminf(fminf(s_least[0], s_least[1]), fminf(s_least[2], s_least[3]));
+  bool plain = a_all == INFINITY || least_all < a_all * 0x1p-44f * b_all;
+  if (plain) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const float row = s_row[m_e + 16 * mb + lc_e] * 0x1p-44f;
+    for (int i = 0; i < AI; ++i) {
+      float v = a_max[i];
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)  // 0 past n, and past m
-          short_of = fmaxf(short_of, fmaf(row, s_col[0][n_e + 16 * nb + 4 * g_e + e], -fabsf(acc[mb][nb][e])));
+      for (int o = 4; o >= 1; o >>= 1) v = __builtin_elementwise_maximum(v, __shfl_xor(v, o));
+      if ((tid_e & 7) == 0) s_row[a_row_e + 32 * i] = v;
     }
-    plain = __syncthreads_or(short_of > 0.f);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s_col[b_row_e][b_n_e + e] = b_max[e];
+    __syncthreads();
+    float v = 0.f;  // waves 0 and 1: a row's largest magnitude, 2 and 3: a column's
+    if (tid_e < TM) {
+      v = s_row[tid_e];
+    } else if (tid_e >= 128) {
+      v = s_col[0][tid_e - 128];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) v = __builtin_elementwise_maximum(v, s_col[i][tid_e - 128]);
+      if (n_tile + tid_e - 128 >= pn) v = 0.f;  // columns past n hold the next row's values
+      s_col[0][tid_e - 128] = v;
+    }
+    const bool in_range = __all(v == 0.f || (v >= 0x1p-40f && v <= 0x1p60f));
+    v = wave_max(v);
+    if ((tid_e & 63) == 0) s_max[wave_e] = in_range ? v : INFINITY;
+    __syncthreads();
+    const float most = fmaxf(s_max[0], s_max[1]) * 0x1p-44f * fmaxf(s_max[2], s_max[3]);
+    plain = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3])) == INFINITY;
+    if (!plain && least_all < most) {
+      float short_of = 0.f;  // by how much a sum falls short of its bound, at most
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const float row = s_row[m_e + 16 * mb + lc_e] * 0x1p-44f;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)  // 0 past n, and past m
+            short_of = fmaxf(short_of, fmaf(row, s_col[0][n_e + 16 * nb + 4 * g_e + e], -fabsf(acc[mb][nb][e])));
+      }
+      plain = __syncthreads_or(short_of > 0.f);
+    }
   }
 
   const int mw = m_tile + m_e, nw = n_tile + n_e;
