@@ -15,16 +15,18 @@ constexpr int kBk = 32;  // k per LDS stage
 
 struct F32Tile {
   int tm, at_once;     // rows; workgroups a CU holds
+  double tile_us;      // launch, first loads, stores
   double stage_us[3];  // a 32-k stage of one, two, three of them on a CU
 };
-// Both heights, as measured at 30 to 256 stages; a split's partials are written,
-// read and summed at about 5 TB/s, with one more launch and a part per slice.  Of 74
-// products of 9 to 4096 rows at the Llama-3.2-3B and SmolLM2 widths, weights rotated
-// through 1 GB, 61 run at 1.0 to 2.3 times the speed of the best fp32 MFMA plan; 13, of
-// 9 to 500 rows at K 576 to 2560, at 0.88 to 0.97 (32 x 576 x (576, 192, 192) 10.1 ->
-// 11.5 us, the widest): two or three stages a slice, whose loads, splits and range
-// check follow one another.
-const F32Tile kF32Tiles[] = {{128, 2, {1.6, 2.75, 0}}, {64, 3, {1.3, 1.8, 2.55}}};
+// Both heights; a split's partials are written, read and summed at about 6.7 TB/s, with
+// one more launch and a part per slice.  Fitted to 139 products of 9 to 2048 rows
+// (SmolLM2 and Llama-3.2-3B widths, weights rotated through 0.8 GB) run on both heights
+// and every split: the choice is the fastest, or within 2% of it, but for three, within 4%.
+// Of 104 such products 78 run at 0.98 to 2.9 times the speed of the best fp32 MFMA plan;
+// 26, of 9 to 1000 rows at K 576 to 2560, at 0.89 to 0.98 (32 x 576 x 576 10.8 -> 12.1
+// us, the widest): a few stages a slice, whose loads, splits and range check follow one
+// another.
+const F32Tile kF32Tiles[] = {{128, 2, 5.7, {1.65, 2.75, 0}}, {64, 3, 5.1, {1.3, 1.8, 2.47}}};
 
 // x0, x1 as three pairs of bf16 whose sums are x0 and x1 exactly (8 significant
 // bits each, rounded to nearest, so every remainder is exact).
@@ -429,12 +431,12 @@ F32Plan gemm_f32_plan(int m, int k, const GemmGroups& G, int min_split, int max_
   for (const F32Tile& c : kF32Tiles) {
     int64_t tiles = 0;
     for (int g = 0; g < G.count; ++g) tiles += (int64_t)((m + c.tm - 1) / c.tm) * ((G.n[g] + 127) / 128);
-    for (int S = min_split; S <= max_split && (S == min_split || stages >= 2 * S); ++S) {
+    for (int S = min_split; S <= max_split && (S == min_split || stages >= S); ++S) {
       const int64_t per_cu = (tiles * S + cus - 1) / cus;
       const int rest = (int)(per_cu % c.at_once);
       const double stage = (double)(per_cu / c.at_once) * c.stage_us[c.at_once - 1] + (rest ? c.stage_us[rest - 1] : 0.0);
-      const double reduce = S > 1 ? (8.0 * S + 4) * m * (double)ncols / 5.0e6 + 4.0 + 0.3 * S : 0.0;
-      const double t = stage * ((stages + S - 1) / S) + 5.0 + reduce;
+      const double reduce = S > 1 ? (8.0 * S + 4) * m * (double)ncols / 6.7e6 + 3.7 + 0.26 * S : 0.0;
+      const double t = stage * ((stages + S - 1) / S) + c.tile_us + reduce;
       if (best.tm == 0 || t < best.us) best = F32Plan{c.tm, S, (stages + S - 1) / S, t};
     }
   }
