@@ -260,9 +260,9 @@ def test_gemm_few_rows_split_k(dtype, M, K, Ns):
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 @pytest.mark.parametrize("M", [9, 63, 64, 65])
 def test_gemm_row_tile_boundaries(dtype, M):
-    """Around the switch from 64-row to 128-row tiles (64 / 65 rows), with a K
-    tail in every dtype (1000 = 15 stages of 64 k + 40, or 62 of 16 + 8) and
-    column counts that are not whole tiles, grouped and single."""
+    """Around the end of a 64-row tile (64 / 65 rows: one and two of them), with a K
+    tail (1000 = 31 stages of 32 k + 8) and column counts that are not whole tiles,
+    grouped and single."""
     print(f"[case] gemm row-tile boundary {dtype} M={M}", flush=True)
     K, Ns = 1000, (1000, 200)
     rng = np.random.default_rng(M)
